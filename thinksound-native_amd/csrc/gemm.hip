@@ -420,6 +420,11 @@ __device__ __forceinline__ void add8(float (&v)[8], const float *p) {
     v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w; v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
 }
 
+// Paired rows (the VAE's operands): channel c's hi part at column pair_col(c), its lo part PAIR further,
+// so a 64-half K tile holds the hi and lo parts of 32 channels
+constexpr int PAIR = 32;
+__device__ __forceinline__ int pair_col(int n) { return n + (n & ~(PAIR - 1)); }
+
 // snake activation (shaders/ops_conv.metal:204-213) with exp(alpha) and exp(-beta) precomputed per column
 __device__ __forceinline__ void snake8(float (&v)[8], const float (&a)[8], const float (&b)[8]) {
 #pragma unroll
@@ -532,10 +537,9 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
                 hi[e] = (half_t)v[e];
                 lo[e] = (half_t)(v[e] - (float)hi[e]);
             }
-            half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + n;
+            half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
             *(half8 *)y = hi;
-            *(half8 *)(y + P.y_lo) = lo;
-            *(half8 *)(y + P.y_hi2) = hi;
+            *(half8 *)(y + PAIR) = lo;
         }
     } else if constexpr (EPI == EPI_RSNAKE) {
         // bias and snake table as in EPI_SNAKE; the stream rows of all four passes are read before
@@ -544,8 +548,10 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
         float bv[8], ea[8], eb[8], xr[4][8];
         if (n < N) {
             if (P.bias) load8(P.bias + n, bv);
-            load8(P.snake + n, ea);
-            load8(P.snake + N + n, eb);
+            if (P.Y) {
+                load8(P.snake + n, ea);
+                load8(P.snake + N + n, eb);
+            }
         }
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
@@ -568,6 +574,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
             float *x = P.R + rowmap_phys(P.rmap, m) * (long long)P.ldr + n;
             *(float4 *)x = make_float4(v[0], v[1], v[2], v[3]);
             *(float4 *)(x + 4) = make_float4(v[4], v[5], v[6], v[7]);
+            if (!P.Y) continue;
             snake8(v, ea, eb);
             half8 hi, lo;
 #pragma unroll
@@ -575,11 +582,9 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
                 hi[e] = (half_t)v[e];
                 lo[e] = (half_t)(v[e] - (float)hi[e]);
             }
-            const int C = P.y_lo;
-            half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + n + 2 * C * (n / C);
+            half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
             *(half8 *)y = hi;
-            *(half8 *)(y + C) = lo;
-            *(half8 *)(y + 2 * C) = hi;
+            *(half8 *)(y + PAIR) = lo;
         }
     } else if constexpr (EPI == EPI_RESID) {
 #pragma unroll
@@ -765,7 +770,12 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
     // kt / taps of tap kt % taps, so the 7 taps of a chunk re-read the same A rows (shifted by
     // dil) in consecutive K tiles while they are still in L2 (4% of a VAE decode; the DiT's k3
     // convs measured 0.4% slower that way).
-    constexpr bool chunk_major = EPI == EPI_SNAKE || EPI == EPI_RSNAKE;
+    // The same kernels read paired rows (PAIR): one K tile is 32 channels with both parts of A and W,
+    // and feeds three products per fragment pair. As a GEMM over [hi | lo | hi] x [W_hi | W_hi | W_lo]
+    // every part that enters two products was staged and read from LDS twice (18 fragments and 48 KB
+    // per 24 MFMAs of a wave against 12 and 32 KB now), and the loop is bound by those: 8 s decode
+    // 4.40 -> 3.41 ms, 1 s 1.07 -> 0.89 ms (same box; operand rows also shrink from 6 to 4 bytes a value).
+    constexpr bool chunk_major = EPI == EPI_SNAKE || EPI == EPI_RSNAKE, pairs = chunk_major;
     const int dil = EPI == EPI_SNAKE ? P.dil : 1;   // dilated taps only in the snake-conv kernels
     const int taps = P.taps;
     int nt_tap, nt_trow, nt_kin, nt_kw;
@@ -853,6 +863,24 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
     }
     auto compute = [&](int stage) {
         const half_t *sa = smem + stage * STAGE, *sb = smem + (NSX + stage) * STAGE;
+        if constexpr (pairs) {   // half 0 holds the hi parts of 32 channels, half 1 their lo parts
+            half8 af[2][2], bf[2][4];
+#pragma unroll
+            for (int kh = 0; kh < 2; ++kh) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) af[kh][i] = *(const half8 *)(sa + a_rd[kh][i]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) bf[kh][j] = *(const half8 *)(sb + b_rd[kh][j]);
+            }
+#pragma unroll
+            for (int q = 0; q < 3; ++q)   // hi * hi, lo * hi, hi * lo
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[q == 1][i], bf[q == 2][j], acc[i][j], 0, 0, 0);
+            return;
+        }
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh) {
             half8 af[2], bf[4];
@@ -1627,10 +1655,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmBatch bt) 
             hi[j] = (half_t)e[j];
             lo[j] = (half_t)(e[j] - (float)hi[j]);
         }
-        half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + n;
+        half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
         *(half4 *)y = hi;
-        *(half4 *)(y + P.y_lo) = lo;
-        *(half4 *)(y + P.y_hi2) = hi;
+        *(half4 *)(y + PAIR) = lo;
     } else if constexpr (EPI == EPI_RSNAKE) {
         float4 *xr = (float4 *)(P.R + rowmap_phys(P.rmap, m) * (long long)P.ldr + n);
         if (P.r_add) {
@@ -1638,6 +1665,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmBatch bt) 
             v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
         }
         *xr = v;
+        if (!P.Y) return;
         float e[4] = {v.x, v.y, v.z, v.w};
         half4 hi, lo;
 #pragma unroll
@@ -1646,11 +1674,9 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmBatch bt) 
             hi[j] = (half_t)e[j];
             lo[j] = (half_t)(e[j] - (float)hi[j]);
         }
-        const int C = P.y_lo;
-        half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + n + 2 * C * (n / C);
+        half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
         *(half4 *)y = hi;
-        *(half4 *)(y + C) = lo;
-        *(half4 *)(y + 2 * C) = hi;
+        *(half4 *)(y + PAIR) = lo;
     } else if constexpr (EPI == EPI_RESID) {
         const float4 g = *(const float4 *)(P.gate + (long long)(m / P.gate_L) * P.gate_ld + n);
         float4 *xr = (float4 *)(P.R + rowmap_phys(P.rmap, m) * (long long)P.ldr + n);
@@ -1752,24 +1778,22 @@ int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
         if (p.w_half)
             TSN_REQUIRE(p.Kc % (2 * BK) == 0 && p.ldw >= p.taps * (p.Kc / 2),
                         "gemm: half-width W needs Kc a multiple of 128 and ldw >= taps*Kc/2");
-        if (p.y_lo && epi != EPI_SNAKE && epi != EPI_RSNAKE) {
+        if (p.y_lo) {
             const int wout = epi == EPI_SWIGLU ? p.N / 2 : p.N;
             TSN_REQUIRE((epi == EPI_STORE || epi == EPI_SWIGLU) && p.y_f16 && p.y_lo % 8 == 0 && p.y_lo >= wout &&
                             p.ldy >= p.y_lo + wout,
                         "gemm: hi|lo output needs f16 Y, lo offset a multiple of 8 past the hi columns, ldy >= y_lo + width");
         }
-        if (epi == EPI_SNAKE)
-            TSN_REQUIRE(p.Y && p.ymap.L > 0 && p.snake && (((uintptr_t)p.snake) & 15) == 0 && p.N % 8 == 0 &&
-                            p.y_lo % 8 == 0 && p.y_hi2 % 8 == 0 && p.y_lo >= p.N && p.y_hi2 >= p.y_lo + p.N &&
-                            p.ldy >= p.y_hi2 + p.N && p.ldy % 8 == 0 && !p.w_half,
-                        "gemm snake: table, three 8-aligned N-wide parts (hi, lo at y_lo, hi at y_hi2) inside ldy");
-        else if (epi == EPI_RSNAKE)
-            TSN_REQUIRE(p.R && p.rmap.L > 0 && p.Y && p.ymap.L > 0 && p.snake && (((uintptr_t)p.snake) & 15) == 0 &&
-                            p.y_lo > 0 && p.y_lo % 8 == 0 && p.N % p.y_lo == 0 && p.ldr % 4 == 0 && p.ldy % 8 == 0 &&
-                            !p.w_half,
-                        "gemm residual snake: stream R, table, phases of y_lo (a multiple of 8) columns");
-        else
-            TSN_REQUIRE(!p.snake && !p.y_hi2, "gemm: snake table and second hi part only with the snake epilogues");
+        if (epi == EPI_SNAKE || epi == EPI_RSNAKE) {
+            TSN_REQUIRE(p.Kc % (2 * PAIR) == 0 && p.N % PAIR == 0 && !p.w_half && !p.y_lo,
+                        "gemm snake: paired operands (whole 32-channel hi|lo groups), N a multiple of 32");
+            TSN_REQUIRE(epi == EPI_RSNAKE ? p.R && p.rmap.L > 0 && p.ldr % 4 == 0 : p.Y != nullptr,
+                        "gemm snake: output rows (residual: the stream R)");
+            TSN_REQUIRE(!p.Y || (p.ymap.L > 0 && p.snake && (((uintptr_t)p.snake) & 15) == 0 && p.ldy >= 2 * p.N &&
+                                 p.ldy % 8 == 0),
+                        "gemm snake: table and paired rows of 2N halves inside ldy");
+        } else
+            TSN_REQUIRE(!p.snake, "gemm: snake table only with the snake epilogues");
         if (epi == EPI_SWIGLU)
             TSN_REQUIRE(p.Y && p.ymap.L > 0 && p.y_f16 && p.N % BN == 0 && p.ldy % 8 == 0 &&
                             (((uintptr_t)p.Y) & 15) == 0,
@@ -1880,7 +1904,7 @@ int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
         return TSN_OK;
     }
     const bool snake_epi = epi == EPI_SNAKE || epi == EPI_RSNAKE;
-    if (pipe && (epi == EPI_RESID || epi == EPI_STORE || snake_epi) && b.ws && (!any_lo || snake_epi)) {
+    if (pipe && (epi == EPI_RESID || epi == EPI_STORE || snake_epi) && b.ws && !any_lo) {
         int nkmin = 1 << 30;
         for (int i = 0; i < b.nprob; ++i) nkmin = std::min(nkmin, b.p[i].K / BK);
         int best = 0;

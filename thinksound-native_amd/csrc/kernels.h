@@ -31,15 +31,15 @@ struct GemmProblem {
     // f16 Y (EPI_STORE, EPI_SWIGLU): nonzero also writes lo = f16(y - f16(y)) at column offset y_lo
     // of the same row (hi|lo operand of a following GEMM against [W | W]); K is then never split
     int y_lo;
+    // EPI_SNAKE, EPI_RSNAKE: A and W rows are paired: every 32 channels as 32 hi halves, then their 32
+    // lo halves (Kc = 2*IC), and the product sums hi*W_hi + lo*W_hi + hi*W_lo (the dropped lo*W_lo term
+    // is below 2^-22 relative), f32-accurate.
     // EPI_SNAKE: y = snake(acc + bias) = v + sin(v*ea[n])^2 * eb[n] with snake = [ea (N) | eb (N)],
-    // stored f16 as a three-part row: hi at column n, lo = f16(y - hi) at n + y_lo, hi again at
-    // n + y_hi2 ([hi | lo | hi], the operand of a following GEMM against [W_hi | W_hi | W_lo]);
-    // K is never split
-    int y_hi2;
+    // stored f16 as such a paired row (2N halves), the operand of the following conv
     const float *snake;
     // EPI_RSNAKE: x = (r_add ? R[rmap(m)*ldr + n] : 0) + acc + bias[n] is stored to R, and snake(x) (table
-    // as EPI_SNAKE) as a three-part f16 row: columns come in phases of C = y_lo, and column n of phase
-    // n / C lands at n + 2C*(n / C) (hi), + C (lo), + 2C (hi) of Y row ymap(m)*ldy
+    // as EPI_SNAKE) as a paired row of Y (Y null: x only). Columns may stack the phases of a transposed
+    // conv: phase p's C columns (C a multiple of 32) are halves 2Cp .. 2Cp + 2C - 1 of the row
     int r_add;
     // EPI_RESID: R[rmap(m)*ldr + n] += gate[(m / gate_L)*gate_ld + n] * (acc + bias)
     float *R; int ldr; RowMap rmap; const float *gate; int gate_ld; int gate_L;
@@ -310,10 +310,12 @@ int launch_bcast_add_silu_f16(const float *x, const float *v, half_t *y, int L, 
 
 // out [M][2K] f16 hi|lo of x[m][k] + pe[m % P][k] (pe null: x alone)
 int launch_add_period_hilo(const float *x, const float *pe, int P, half_t *out, int M, int K, hipStream_t st);
-// VAE decoder (vae.hip). split3: f32 rows [rows][C] (C % 8 == 0) -> f16 [rows][3C], v = x or, with a
-// table ab = [exp(alpha) (C) | exp(-beta) (C)], snake(x) = x + sin(x*ea)^2*eb; parts [hi | lo | hi]
-// (lo_part 1, activation operand) or [hi | hi | lo] (lo_part 2, weight operand)
-int launch_split3(const float *x, long long rows, int C, const float *ab, int lo_part, half_t *out, hipStream_t st);
+// VAE decoder (vae.hip). split_pairs: f32 rows [rows][C] (C % 32 == 0) -> paired f16 rows [rows][2C]
+// (EPI_SNAKE's operands: each 32 channels as 32 hi halves, then 32 lo halves, lo = f16(x - hi))
+int launch_split_pairs(const float *x, long long rows, int C, half_t *out, hipStream_t st);
+// split3: f32 rows [rows][C] (C % 8 == 0) -> f16 [rows][hi (C) | lo (C) | hi (C)], the operand of a GEMM
+// against [W_hi | W_hi | W_lo]
+int launch_split3(const float *x, long long rows, int C, half_t *out, hipStream_t st);
 // y [T][OC] = conv(snake(x), W [OC][C][KK], pad), no bias; x [T][C] f32, OC in {1, 2, 4}, KK == 7, C % 8 == 0
 int launch_conv_out(const float *x, const float *ab, const float *W, float *y, int T, int C, int OC, int KK, int pad,
                     hipStream_t st);

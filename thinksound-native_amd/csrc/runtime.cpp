@@ -315,7 +315,7 @@ int Runtime::conv(int wdt, const void *Wp, const float *bias, const float *x, fl
         void *buf = nullptr;
         TSN_TRY(scratch((size_t)T * ich * sizeof(half_t), &buf));
         if (parts == 1) TSN_TRY(launch_split_hilo(x, (int)IC, rowmap_dense((int)T), (half_t *)buf, (int)T, (int)IC, st));
-        else TSN_TRY(launch_split3(x, (long long)T, (int)IC, nullptr, 1, (half_t *)buf, st));
+        else TSN_TRY(launch_split3(x, (long long)T, (int)IC, (half_t *)buf, st));
         q.A = buf; q.lda = ich; q.amap = rowmap_dense((int)OL);
         q.taps = (int)K; q.Kc = ich; q.pad = (int)pad; q.a_T = (int)T;
         q.M = (int)OL; q.K = (int)K * ich;

@@ -142,18 +142,13 @@ int VaeModel::create(Runtime *r, const VaeSpec &sp) {
     // input conv's output)
     size_t tc = (size_t)s.T * std::max(s.width[0], s.latent);
     long long T = s.T;
-    int wmax = s.width[0];
     for (int n = 0; n < 5; ++n) {
         T *= s.stride[n];
         tc = std::max(tc, (size_t)T * s.width[n + 1]);
-        wmax = std::max(wmax, s.width[n + 1]);
     }
     TSN_TRY(alloc(tc * sizeof(float), (void **)&X_));
-    TSN_TRY(alloc(tc * 3 * sizeof(half_t), (void **)&A1_));
-    TSN_TRY(alloc(tc * 3 * sizeof(half_t), (void **)&A2_));
-    std::vector<float> ones((size_t)wmax, 1.0f);
-    TSN_TRY(alloc(ones.size() * sizeof(float), (void **)&ones_));
-    TSN_TRY(rt->dev.upload(ones_, ones.data(), ones.size() * sizeof(float)));
+    TSN_TRY(alloc(tc * 2 * sizeof(half_t), (void **)&A1_));
+    TSN_TRY(alloc(tc * 2 * sizeof(half_t), (void **)&A2_));
     ws_bytes_ = (size_t)64 << 20;
     TSN_TRY(alloc(ws_bytes_, (void **)&ws_));
     TSN_TRY(alloc_skcnt());
@@ -173,7 +168,7 @@ int VaeModel::upload_weights(const float *host, size_t numel) { return upload(ho
 // Host side: conv weights reordered to [rows][taps][IC] f32 (transposed convs split into phase
 // groups), snake parameters turned into [exp(alpha) | exp(-beta)] tables (double precision, then
 // rounded), biases repeated per phase. One f32 upload of each set; the device splits the conv
-// weights into f16 [rows][taps][W_hi | W_hi | W_lo].
+// weights into paired f16 [rows][taps][hi|lo groups] (EPI_SNAKE).
 int VaeModel::upload(const float *host, size_t numel) {
     TSN_REQUIRE(rt && host, "vae: not created / null weights");
     TSN_REQUIRE(!ready_, "vae: weights already uploaded");
@@ -284,9 +279,9 @@ int VaeModel::upload(const float *host, size_t numel) {
     TSN_TRY(alloc(wf32.size() * sizeof(float), (void **)&pf));
     TSN_TRY(rt->dev.upload(pf, wf32.data(), wf32.size() * sizeof(float)));
     for (auto &e : f32s) *e.second = pf + e.first;
-    // conv weights: f32 staging, split into the f16 three-part rows
+    // conv weights: f32 staging, split into the paired f16 rows
     size_t parts = 0;
-    for (const auto &c : convs) parts += (size_t)c.rows * 3 * c.IC;
+    for (const auto &c : convs) parts += (size_t)c.rows * 2 * c.IC;
     half_t *ph;
     float *stage;
     TSN_TRY(alloc(parts * sizeof(half_t), (void **)&ph));
@@ -294,9 +289,9 @@ int VaeModel::upload(const float *host, size_t numel) {
     TSN_TRY(rt->dev.upload(stage, wconv.data(), wconv.size() * sizeof(float)));
     size_t o = 0;
     for (const auto &c : convs) {
-        TSN_TRY(launch_split3(stage + c.off, c.rows, c.IC, nullptr, 2, ph + o, rt->dev.stream()));
+        TSN_TRY(launch_split_pairs(stage + c.off, c.rows, c.IC, ph + o, rt->dev.stream()));
         *c.dst = ph + o;
-        o += (size_t)c.rows * 3 * c.IC;
+        o += (size_t)c.rows * 2 * c.IC;
     }
     TSN_TRY(rt->dev.sync());
     TSN_TRY(release(stage));
@@ -309,18 +304,18 @@ int VaeModel::enqueue_decode(const float *latent, float *audio) {
     TSN_REQUIRE(latent && audio, "vae: null latent or audio");
     TSN_REQUIRE((((uintptr_t)latent) & 15) == 0, "vae: latent must be 16-byte aligned");
     const hipStream_t stq = rt->dev.stream();
-    const double third = 1.0 / 3.0;   // profiled flops: the f32 GEMM's 2*M*N*K, not the three f16 products
-    // three-part operands ping-pong between A1 and A2: each GEMM reads `in` and writes `out`
+    const double half = 0.5;   // profiled flops: the f32 GEMM's 2*M*N*taps*IC (K counts hi and lo columns)
+    // paired operands ping-pong between A1 and A2: each GEMM reads `in` and writes `out`
     half_t *in = A1_, *out = A2_;
     auto flip = [&]() { std::swap(in, out); };
-    // conv GEMM over the three-part operand A (lda = 3 IC); taps of width 3 IC
+    // conv GEMM over the paired operand A (lda = 2 IC); taps of width 2 IC
     auto conv = [&](GemmProblem &p, const half_t *A, int M, int IC, int taps, int pad, int dil, const half_t *W,
                     const float *bias, int N) {
         gemm_problem_init(p);
-        p.A = A; p.lda = 3 * IC; p.amap = rowmap_dense(M);
-        p.taps = taps; p.Kc = 3 * IC; p.pad = pad; p.a_T = M; p.dil = dil;
-        p.W = W; p.ldw = taps * 3 * IC; p.bias = bias;
-        p.M = M; p.N = N; p.K = taps * 3 * IC;
+        p.A = A; p.lda = 2 * IC; p.amap = rowmap_dense(M);
+        p.taps = taps; p.Kc = 2 * IC; p.pad = pad; p.a_T = M; p.dil = dil;
+        p.W = W; p.ldw = taps * 2 * IC; p.bias = bias;
+        p.M = M; p.N = N; p.K = taps * 2 * IC;
     };
     auto batch = [&](GemmBatch &b, int n) {
         b.nprob = n;
@@ -330,24 +325,24 @@ int VaeModel::enqueue_decode(const float *latent, float *audio) {
     };
 
     int T = s.T, C = s.width[0];
-    // input conv k7 pad 3 + b, then the first stage's snake: latent -> snake(x0) three-part
-    TSN_TRY(run("split3_kernel", 0, (double)T * s.latent * 10.0,
-                [&] { return launch_split3(latent, T, s.latent, nullptr, 1, in, stq); }));
+    // input conv k7 pad 3 + b, then the first stage's snake: latent -> snake(x0) paired
+    TSN_TRY(run("split_kernel<false>", 0, (double)T * s.latent * 8.0,
+                [&] { return launch_split_pairs(latent, T, s.latent, in, stq); }));
     {
         GemmBatch b;
         batch(b, 1);
         GemmProblem &p = b.p[0];
         conv(p, in, T, s.latent, KRES, 3, 1, W0_, b0_, C);
-        p.Y = out; p.ldy = 3 * C; p.ymap = rowmap_dense(T);
-        p.y_f16 = 1; p.y_lo = C; p.y_hi2 = 2 * C; p.snake = st_[0].ab_in;
-        TSN_TRY(gemm_run(b, EPI_SNAKE, third));
+        p.Y = out; p.ldy = 2 * C; p.ymap = rowmap_dense(T);
+        p.y_f16 = 1; p.snake = st_[0].ab_in;
+        TSN_TRY(gemm_run(b, EPI_SNAKE, half));
         flip();
     }
     for (int n = 0; n < 5; ++n) {
         const Stage &g = st_[n];
         const int stv = s.stride[n], co = s.width[n + 1];
         // transposed conv as phase-group convs: x rows interleave straight into X, and the first
-        // residual unit's snake(x) into the three-part rows of `out`
+        // residual unit's snake(x) into the paired rows of `out`
         {
             GemmBatch b;
             batch(b, g.ngroups);
@@ -355,10 +350,10 @@ int VaeModel::enqueue_decode(const float *latent, float *audio) {
                 GemmProblem &p = b.p[q];
                 conv(p, in, T, C, g.taps, g.pad[q], 1, g.Wt[q], g.bt[q], g.nph[q] * co);
                 p.R = X_ + (size_t)g.r0[q] * co; p.ldr = stv * co; p.rmap = rowmap_dense(T); p.r_add = 0;
-                p.Y = out + (size_t)g.r0[q] * 3 * co; p.ldy = stv * 3 * co; p.ymap = rowmap_dense(T);
-                p.y_lo = co; p.snake = g.abt[q];
+                p.Y = out + (size_t)g.r0[q] * 2 * co; p.ldy = stv * 2 * co; p.ymap = rowmap_dense(T);
+                p.snake = g.abt[q];
             }
-            TSN_TRY(gemm_run(b, EPI_RSNAKE, third));
+            TSN_TRY(gemm_run(b, EPI_RSNAKE, half));
             flip();
         }
         T *= stv;
@@ -366,14 +361,14 @@ int VaeModel::enqueue_decode(const float *latent, float *audio) {
         for (int r = 0; r < 3; ++r) {
             const Unit &u = g.u[r];
             const int d = DILS[r];
-            {   // conv k7, dilation d, + bias -> snake -> three-part f16
+            {   // conv k7, dilation d, + bias -> snake -> paired f16
                 GemmBatch b;
                 batch(b, 1);
                 GemmProblem &p = b.p[0];
                 conv(p, in, T, C, KRES, 3 * d, d, u.W7, u.b7, C);
-                p.Y = out; p.ldy = 3 * C; p.ymap = rowmap_dense(T);
-                p.y_f16 = 1; p.y_lo = C; p.y_hi2 = 2 * C; p.snake = u.ab2;
-                TSN_TRY(gemm_run(b, EPI_SNAKE, third));
+                p.Y = out; p.ldy = 2 * C; p.ymap = rowmap_dense(T);
+                p.y_f16 = 1; p.snake = u.ab2;
+                TSN_TRY(gemm_run(b, EPI_SNAKE, half));
                 flip();
             }
             {   // conv k1 + bias added to x; the next snake (next unit, or next stage's input) from the new x
@@ -383,16 +378,13 @@ int VaeModel::enqueue_decode(const float *latent, float *audio) {
                 GemmProblem &p = b.p[0];
                 conv(p, in, T, C, 1, 0, 1, u.W1, u.b1, C);
                 p.R = X_; p.ldr = C; p.rmap = rowmap_dense(T);
-                if (next) {
-                    p.r_add = 1;
-                    p.Y = out; p.ldy = 3 * C; p.ymap = rowmap_dense(T);
-                    p.y_lo = C; p.snake = next;
-                    TSN_TRY(gemm_run(b, EPI_RSNAKE, third));
-                    flip();
-                } else {   // the final snake belongs to the output conv
-                    p.gate = ones_; p.gate_ld = 0; p.gate_L = T;
-                    TSN_TRY(gemm_run(b, EPI_RESID, third));
+                p.r_add = 1;
+                if (next) {   // else x only: the final snake belongs to the output conv
+                    p.Y = out; p.ldy = 2 * C; p.ymap = rowmap_dense(T);
+                    p.snake = next;
                 }
+                TSN_TRY(gemm_run(b, EPI_RSNAKE, half));
+                if (next) flip();
             }
         }
     }

@@ -5,9 +5,10 @@
 //   -> snake -> conv k7 pad 3 (no bias) -> audio [T*prod(s)][2]
 //
 // The reference keeps this network in f32 (src/vae.cpp:12). Every GEMM here runs f32-accurate
-// on f16 MFMA with three products per term: the activation row is stored [hi | lo | hi] and the
-// weight row [W_hi | W_hi | W_lo], so one f16 GEMM over K = 3*IC sums hi*W_hi + lo*W_hi + hi*W_lo
-// (the dropped lo*W_lo term is below 2^-22 relative). The residual stream x stays f32.
+// on f16 MFMA with three products per term: activation and weight rows hold every 32 channels as
+// 32 hi halves, then their 32 lo halves, so each staged K tile has both parts of both operands and
+// the kernel sums hi*W_hi + lo*W_hi + hi*W_lo from them (the dropped lo*W_lo term is below 2^-22
+// relative). The residual stream x stays f32.
 //
 // Every snake runs in the epilogue of the GEMM that produces its input (the residual units' closing
 // k1 conv writes x and snake(x) for the next unit or stage), so x is read once per GEMM.
@@ -53,14 +54,14 @@ public:
 private:
     struct Unit {   // one residual unit
         const float *ab1 = nullptr, *ab2 = nullptr;   // snake tables [exp(alpha) | exp(-beta)]
-        const half_t *W7 = nullptr, *W1 = nullptr;    // [C][7][3C], [C][3C]
+        const half_t *W7 = nullptr, *W1 = nullptr;    // [C][7][2C], [C][2C]
         const float *b7 = nullptr, *b1 = nullptr;
     };
     struct Stage {
         const float *ab_in = nullptr;   // snake before the transposed conv, [2][C_in]
         int ngroups = 0, taps = 0;
         int r0[2] = {0, 0}, nph[2] = {0, 0}, pad[2] = {0, 0};   // phase group: first phase, phases, row pad
-        const half_t *Wt[2] = {nullptr, nullptr};               // [nph*C_out][taps][3 C_in]
+        const half_t *Wt[2] = {nullptr, nullptr};               // [nph*C_out][taps][2 C_in]
         const float *bt[2] = {nullptr, nullptr};                // bias repeated per phase
         const float *abt[2] = {nullptr, nullptr};               // first unit's snake table, per phase
         Unit u[3];
@@ -68,7 +69,7 @@ private:
     Stage st_[5];
     const half_t *W0_ = nullptr;
     const float *b0_ = nullptr, *ab_out_ = nullptr, *Wout_ = nullptr;
-    float *X_ = nullptr, *ones_ = nullptr, *ws_ = nullptr;
+    float *X_ = nullptr, *ws_ = nullptr;
     half_t *A1_ = nullptr, *A2_ = nullptr;
     size_t ws_bytes_ = 0;
     bool ready_ = false;

@@ -1,6 +1,6 @@
 // vae.hip — the element-wise and output kernels of the VAE decoder (src/vae.cpp:17-86): the
-// three-part f16 split of f32 rows (optionally after the snake activation), and the final
-// snake + narrow conv to the audio channels.
+// f16 splits of f32 rows (paired for the decoder's convs, three-part for the launcher convs), and
+// the final snake + narrow conv to the audio channels.
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
@@ -11,11 +11,10 @@ namespace tsn {
 
 namespace {
 
-// One thread per 8 channels of a row: v = x (or snake(x) with ea = exp(alpha), eb = exp(-beta)),
-// hi = f16(v), lo = f16(v - hi); the row of out holds three C-wide parts: [hi | lo | hi] when
-// lo_part == 1 (an activation operand), [hi | hi | lo] when lo_part == 2 (a weight operand).
-__global__ void split3_kernel(const float *__restrict__ x, long long rows, int C, const float *__restrict__ ab,
-                              int lo_part, half_t *__restrict__ out) {
+// One thread per 8 channels of a row: hi = f16(x), lo = f16(x - hi). THREE: the row of out holds three
+// C-wide parts [hi | lo | hi]; otherwise paired groups of 32 hi halves, then their 32 lo halves.
+template <bool THREE>
+__global__ void split_kernel(const float *__restrict__ x, long long rows, int C, half_t *__restrict__ out) {
     const int cg = C >> 3;
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= rows * cg) return;
@@ -23,23 +22,23 @@ __global__ void split3_kernel(const float *__restrict__ x, long long rows, int C
     const int c = (int)(i - r * cg) * 8;
     const float *xp = x + r * C + c;
     const float4 x0 = *(const float4 *)xp, x1 = *(const float4 *)(xp + 4);
-    float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-    if (ab) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            v[e] = v[e] + snake_sin2(v[e] * ab[c + e]) * ab[C + c + e];
-        }
-    }
+    const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
     half8 hi, lo;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         hi[e] = (half_t)v[e];
         lo[e] = (half_t)(v[e] - (float)hi[e]);
     }
-    half_t *o = out + r * 3 * C + c;
-    *(half8 *)o = hi;
-    *(half8 *)(o + C) = lo_part == 1 ? lo : hi;
-    *(half8 *)(o + 2 * C) = lo_part == 1 ? hi : lo;
+    if constexpr (THREE) {
+        half_t *o = out + r * 3 * C + c;
+        *(half8 *)o = hi;
+        *(half8 *)(o + C) = lo;
+        *(half8 *)(o + 2 * C) = hi;
+    } else {
+        half_t *o = out + r * 2 * C + c + (c & ~31);
+        *(half8 *)o = hi;
+        *(half8 *)(o + 32) = lo;
+    }
 }
 
 constexpr int CO_TB = 64;    // output rows per workgroup (16 per wave)
@@ -130,12 +129,20 @@ __global__ void __launch_bounds__(256) conv_out_kernel(const float *__restrict__
 
 } // namespace
 
-int launch_split3(const float *x, long long rows, int C, const float *ab, int lo_part, half_t *out, hipStream_t st) {
-    TSN_REQUIRE(x && out && rows > 0 && C > 0 && C % 8 == 0 && (lo_part == 1 || lo_part == 2),
-                "split3: arguments (C a multiple of 8, lo part 1 or 2)");
+int launch_split3(const float *x, long long rows, int C, half_t *out, hipStream_t st) {
+    TSN_REQUIRE(x && out && rows > 0 && C > 0 && C % 8 == 0, "split3: arguments (C a multiple of 8)");
     TSN_REQUIRE((((uintptr_t)x) & 15) == 0 && (((uintptr_t)out) & 15) == 0, "split3: 16-byte aligned rows");
     const long long n = rows * (C / 8);
-    TSN_LAUNCH(split3_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, rows, C, ab, lo_part, out);
+    TSN_LAUNCH(split_kernel<true>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, rows, C, out);
+    TSN_HIP_CHECK(hipGetLastError());
+    return TSN_OK;
+}
+
+int launch_split_pairs(const float *x, long long rows, int C, half_t *out, hipStream_t st) {
+    TSN_REQUIRE(x && out && rows > 0 && C > 0 && C % 32 == 0, "split pairs: arguments (C a multiple of 32)");
+    TSN_REQUIRE((((uintptr_t)x) & 15) == 0 && (((uintptr_t)out) & 15) == 0, "split pairs: 16-byte aligned rows");
+    const long long n = rows * (C / 8);
+    TSN_LAUNCH(split_kernel<false>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, rows, C, out);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
