@@ -457,12 +457,13 @@ __global__ __launch_bounds__(512, NSTG == 2 ? 2 : 1) void flash_attn_kernel(cons
                 float *op = (float *)a.O + orow + d0;
                 *(float4 *)op = make_float4(od[0] * inv, od[1] * inv, od[2] * inv, od[3] * inv);
             } else {
-                half_t *op = (half_t *)a.O + orow + d0;
+                const bool pair = q < a.o_pair;   // paired row: head h's 64 columns are 128 halves
+                half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
                 const float y0 = od[0] * inv, y1 = od[1] * inv, y2 = od[2] * inv, y3 = od[3] * inv;
                 const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
                 *(half4 *)op = hi;
-                if (a.o_lo)   // f16 remainder at column offset o_lo: hi + lo carries the f32 value
-                    *(half4 *)(op + a.o_lo) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
+                if (pair)   // the f16 remainder: hi + lo carries the f32 value
+                    *(half4 *)(op + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
                                                     (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
             }
         }
@@ -609,12 +610,13 @@ __global__ __launch_bounds__(256, 3) void flash_attn4_kernel(const AttnArgs a) {
                 float *op = (float *)a.O + orow + d0;
                 *(float4 *)op = make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
             } else {
-                half_t *op = (half_t *)a.O + orow + d0;
+                const bool pair = q < a.o_pair;
+                half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
                 const float y0 = o[dt][0] * inv, y1 = o[dt][1] * inv, y2 = o[dt][2] * inv, y3 = o[dt][3] * inv;
                 const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
                 *(half4 *)op = hi;
-                if (a.o_lo)
-                    *(half4 *)(op + a.o_lo) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
+                if (pair)
+                    *(half4 *)(op + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
                                                     (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
             }
         }
@@ -770,12 +772,13 @@ __global__ __launch_bounds__(256, 3) void flash_attn4q2_kernel(const AttnArgs a)
                 float *op = (float *)a.O + orow + d0;
                 *(float4 *)op = make_float4(o[u][dt][0] * inv, o[u][dt][1] * inv, o[u][dt][2] * inv, o[u][dt][3] * inv);
             } else {
-                half_t *op = (half_t *)a.O + orow + d0;
+                const bool pair = q[u] < a.o_pair;
+                half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
                 const float y0 = o[u][dt][0] * inv, y1 = o[u][dt][1] * inv, y2 = o[u][dt][2] * inv, y3 = o[u][dt][3] * inv;
                 const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
                 *(half4 *)op = hi;
-                if (a.o_lo)
-                    *(half4 *)(op + a.o_lo) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
+                if (pair)
+                    *(half4 *)(op + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
                                                     (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
             }
         }
@@ -810,8 +813,8 @@ int launch_attention(const AttnArgs &a, hipStream_t st) {
     TSN_REQUIRE(a.BH > 0 && a.nh > 0 && a.BH % a.nh == 0, "attention: BH must be a multiple of nh");
     TSN_REQUIRE(a.omap.L > 0, "attention: output row map");
     TSN_REQUIRE(a.ldo % 4 == 0, "attention: ldo must be a multiple of 4");
-    TSN_REQUIRE(a.o_lo == 0 || (!a.o_f32 && a.o_lo % 4 == 0 && a.o_lo >= a.nh * 64 && a.ldo >= a.o_lo + a.nh * 64),
-                "attention: hi|lo output needs f16 O, o_lo >= nh*64 (multiple of 4) and ldo >= o_lo + nh*64");
+    TSN_REQUIRE(a.o_pair == 0 || (!a.o_f32 && a.o_pair > 0 && a.ldo >= 2 * a.nh * 64),
+                "attention: paired output rows need f16 O and ldo >= 2*nh*64");
     TSN_REQUIRE((((uintptr_t)a.Q) & 15) == 0 && (((uintptr_t)a.K) & 15) == 0 && (((uintptr_t)a.Vt) & 15) == 0,
                 "attention: 16-byte aligned Q/K/Vt");
     TSN_REQUIRE((long long)a.S * 64 * 2 < (1LL << 31) && (long long)a.Sp * 64 * 2 < (1LL << 31),

@@ -196,10 +196,10 @@ int DitModel::upload_weights(const uint16_t *host, size_t numel) {
     {
         half_t *w;
         TSN_TRY(alloc((size_t)H * 2 * s.latent * 2, (void **)&w));
-        TSN_TRY(launch_dup_cols_bf16_to_f16(raw("audio_input_proj.weight"), w, (int)H, s.latent, st));
+        TSN_TRY(launch_dup_cols_bf16_to_f16(raw("audio_input_proj.weight"), w, (int)H, s.latent, s.latent, st));
         Win2_ = w;
         TSN_TRY(alloc((size_t)s.latent * 2 * H * 2, (void **)&w));
-        TSN_TRY(launch_dup_cols_bf16_to_f16(raw("final_layer.linear.weight"), w, s.latent, (int)H, st));
+        TSN_TRY(launch_dup_cols_bf16_to_f16(raw("final_layer.linear.weight"), w, s.latent, (int)H, final_fused() ? (int)H : PAIR, st));
         Wfin2_ = w;
     }
     TSN_TRY(f32("t_embed.mlp.0.bias", &bt0_));

@@ -378,6 +378,16 @@ __device__ __forceinline__ unsigned lds_addr(const half_t *base) {
     return (unsigned)(unsigned long)(const lds_char *)base;
 }
 
+// s_waitcnt vmcnt(L*n) for n tiles of L DMAs, n <= NMAX (L*NMAX < 16); the other counters at their maxima
+template <int L, int NMAX>
+__device__ __forceinline__ void wait_tiles(int n) {
+    static_assert(L * NMAX < 16, "vmcnt's low field");
+    if constexpr (NMAX > 0) {
+        if (n < NMAX) return wait_tiles<L, NMAX - 1>(n);
+    }
+    __builtin_amdgcn_s_waitcnt(L * NMAX | (7 << 4) | (0xF << 8));
+}
+
 // s_waitcnt vmcnt(n) (n in {0, 4, 8, 12}) with expcnt/lgkmcnt left at their maxima
 __device__ __forceinline__ void wait_vmcnt(int n) {
     if (n >= 12) __builtin_amdgcn_s_waitcnt(12 | (7 << 4) | (0xF << 8));
@@ -413,17 +423,25 @@ __device__ __forceinline__ void load8(const float *t, float (&v)[8]) {
     const floatx4 a = *(const floatx4 *)t, b = *(const floatx4 *)(t + 4);
     v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3]; v[4] = b[0]; v[5] = b[1]; v[6] = b[2]; v[7] = b[3];
 }
-__device__ __forceinline__ void ldsum8(const float *t, int off, float (&v)[8]) { load8(t + off, v); }
-__device__ __forceinline__ float ldsum1(const float *t, int off) { return t[off]; }
+template <int T2>
+__device__ __forceinline__ void ldsum8(const float *t, int off, float (&v)[8]) {
+    load8(t + off, v);
+    if constexpr (T2 != 0) {
+        float u[8];
+        load8(t + T2 + off, u);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] += u[e];
+    }
+}
+template <int T2>
+__device__ __forceinline__ float ldsum1(const float *t, int off) {
+    if constexpr (T2 != 0) return t[off] + t[off + T2];
+    return t[off];
+}
 __device__ __forceinline__ void add8(float (&v)[8], const float *p) {
     const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
     v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w; v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
 }
-
-// Paired rows (the VAE's operands): channel c's hi part at column pair_col(c), its lo part PAIR further,
-// so a 64-half K tile holds the hi and lo parts of 32 channels
-constexpr int PAIR = 32;
-__device__ __forceinline__ int pair_col(int n) { return n + (n & ~(PAIR - 1)); }
 
 // snake activation (shaders/ops_conv.metal:204-213) with exp(alpha) and exp(-beta) precomputed per column
 __device__ __forceinline__ void snake8(float (&v)[8], const float (&a)[8], const float (&b)[8]) {
@@ -433,20 +451,23 @@ __device__ __forceinline__ void snake8(float (&v)[8], const float (&a)[8], const
     }
 }
 
-template <int EPI, int PITCH = TP>
+// ROWS: rows of the tile (a multiple of 32). T2: nonzero adds a second tile, T2 floats further (the
+// other wave group's partial product).
+template <int EPI, int PITCH = TP, int ROWS = BM, int T2 = 0>
 __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float *tile, int m0, int n0, int ks, int tid) {
+    constexpr int NP = ROWS / 32;   // passes of 32 rows x 16 threads
     const int M = P.M, N = P.N;
     if (P.splits > 1) {
         // raw f32 partial of this split: ws[(ks*M + m)*N + n]
         float *w = P.ws + (long long)ks * M * N;
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int c = tid + 512 * p, row = c >> 4, col = (c & 15) * 8;
             const int m = m0 + row, n = n0 + col;
             if (m < M && n < N) {
                 float *o = w + (long long)m * N + n;
                 float v[8];
-                ldsum8(tile, row * PITCH + col, v);
+                ldsum8<T2>(tile, row * PITCH + col, v);
                 *(float4 *)o = make_float4(v[0], v[1], v[2], v[3]);
                 *(float4 *)(o + 4) = make_float4(v[4], v[5], v[6], v[7]);
             }
@@ -455,12 +476,12 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
     }
     if constexpr (EPI == EPI_STORE) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int c = tid + 512 * p, row = c >> 4, col = (c & 15) * 8;
             const int m = m0 + row, n = n0 + col;
             if (m >= M || n >= N) continue;
             float v[8];
-            ldsum8(tile, row * PITCH + col, v);
+            ldsum8<T2>(tile, row * PITCH + col, v);
             if (P.bias) add8(v, P.bias + n);
             if (P.silu)
 #pragma unroll
@@ -470,13 +491,15 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
                 half8 hi;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) hi[e] = (half_t)v[e];
-                *(half8 *)((half_t *)P.Y + o) = hi;
-                if (P.y_lo) {
+                half_t *y = (half_t *)P.Y + o;
+                if (P.y_pair) {
                     half8 lo;
 #pragma unroll
                     for (int e = 0; e < 8; ++e) lo[e] = (half_t)(v[e] - (float)hi[e]);
-                    *(half8 *)((half_t *)P.Y + o + P.y_lo) = lo;
+                    y += pair_col(n) - n;
+                    *(half8 *)(y + PAIR) = lo;
                 }
+                *(half8 *)y = hi;
             } else {
                 float *y = (float *)P.Y + o;
                 *(float4 *)y = make_float4(v[0], v[1], v[2], v[3]);
@@ -486,13 +509,13 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
     } else if constexpr (EPI == EPI_SWIGLU) {
         // tile columns 0..63: w1 rows 64j.., columns 64..127: the matching w3 rows (j = n0 / 128)
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
+        for (int p = 0; p < (ROWS + 63) / 64; ++p) {
             const int c = tid + 512 * p, row = c >> 3, col = (c & 7) * 8;
             const int m = m0 + row;
-            if (m >= M) continue;
+            if (m >= M || (ROWS % 64 && row >= ROWS)) continue;
             float a[8], b[8];
-            ldsum8(tile, row * PITCH + col, a);
-            ldsum8(tile, row * PITCH + 64 + col, b);
+            ldsum8<T2>(tile, row * PITCH + col, a);
+            ldsum8<T2>(tile, row * PITCH + 64 + col, b);
             float y[8];
             half8 o;
 #pragma unroll
@@ -500,13 +523,14 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
                 y[e] = silu_f(a[e]) * b[e];
                 o[e] = (half_t)y[e];
             }
-            half_t *dst = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + n0 / 2 + col;
+            const int n = n0 / 2 + col;
+            half_t *dst = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + (P.y_pair ? pair_col(n) : n);
             *(half8 *)dst = o;
-            if (P.y_lo) {
+            if (P.y_pair) {
                 half8 lo;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) lo[e] = (half_t)(y[e] - (float)o[e]);
-                *(half8 *)(dst + P.y_lo) = lo;
+                *(half8 *)(dst + PAIR) = lo;
             }
         }
     } else if constexpr (EPI == EPI_SNAKE) {
@@ -521,12 +545,12 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
             load8(P.snake + N + n, eb);
         }
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int row = (tid >> 4) + 32 * p;
             const int m = m0 + row;
             if (m >= M || n >= N) continue;
             float v[8];
-            ldsum8(tile, row * PITCH + col, v);
+            ldsum8<T2>(tile, row * PITCH + col, v);
             if (P.bias)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] += bv[e];
@@ -545,7 +569,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
         // bias and snake table as in EPI_SNAKE; the stream rows of all four passes are read before
         // the first store
         const int col = (tid & 15) * 8, n = n0 + col;
-        float bv[8], ea[8], eb[8], xr[4][8];
+        float bv[8], ea[8], eb[8], xr[NP][8];
         if (n < N) {
             if (P.bias) load8(P.bias + n, bv);
             if (P.Y) {
@@ -554,17 +578,17 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
             }
         }
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int m = m0 + (tid >> 4) + 32 * p;
             if (P.r_add && m < M && n < N) load8(P.R + rowmap_phys(P.rmap, m) * (long long)P.ldr + n, xr[p]);
         }
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int row = (tid >> 4) + 32 * p;
             const int m = m0 + row;
             if (m >= M || n >= N) continue;
             float v[8];
-            ldsum8(tile, row * PITCH + col, v);
+            ldsum8<T2>(tile, row * PITCH + col, v);
             if (P.bias)
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] += bv[e];
@@ -588,12 +612,12 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
         }
     } else if constexpr (EPI == EPI_RESID) {
 #pragma unroll
-        for (int p = 0; p < 4; ++p) {
+        for (int p = 0; p < NP; ++p) {
             const int c = tid + 512 * p, row = c >> 4, col = (c & 15) * 8;
             const int m = m0 + row, n = n0 + col;
             if (m >= M || n >= N) continue;
             float v[8];
-            ldsum8(tile, row * PITCH + col, v);
+            ldsum8<T2>(tile, row * PITCH + col, v);
             if (P.bias) add8(v, P.bias + n);
             const float *g = P.gate + (long long)(m / P.gate_L) * P.gate_ld + n;
             float *x = P.R + rowmap_phys(P.rmap, m) * (long long)P.ldr + n;
@@ -621,18 +645,18 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
             load8(nw + d0, nwv);
             // the RoPE rows of all four passes, loaded before any store: a store to Q/K may alias
             // the table, so a load left inside the loop would wait for the previous pass's store
-            float cs4[4][8];
+            float cs4[NP][8];
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            for (int p = 0; p < NP; ++p) {
                 const int m = m0 + (tid >> 4) + 32 * p;
                 const int t = m < M ? m % P.q_L : P.rope_len;
                 if (t < P.rope_len) load8(P.rope + (t * 32 + (d0 >> 1)) * 2, cs4[p]);
             }
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
+            for (int p = 0; p < NP; ++p) {
                 const int row = (tid >> 4) + 32 * p, m = m0 + row;
                 float v[8];
-                ldsum8(tile, row * PITCH + col, v);
+                ldsum8<T2>(tile, row * PITCH + col, v);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] += bw[e];
                 // per-head RMS over the 64 columns held by 8 neighbouring lanes (same row, same head)
@@ -669,7 +693,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
             const int col = tid & 127, n = n0 + col;
             const int h = (n - 2 * P.Hq) >> 6, d = n & 63;
             const float bn = P.bias ? P.bias[n] : 0.0f;
-            const int m1 = min(m0 + BM, M);
+            const int m1 = min(m0 + ROWS, M);
             const int b0 = m0 / P.q_L, b1 = (m1 - 1) / P.q_L;
             int total = 0;
             for (int b = b0; b <= b1; ++b) {
@@ -691,13 +715,13 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
                 if (s8 >= P.q_soff + ta && s8 + 8 <= P.q_soff + tb) {
                     half8 hv;
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) hv[e] = (half_t)(ldsum1(tile, (r8 + e) * PITCH + col) + bn);
+                    for (int e = 0; e < 8; ++e) hv[e] = (half_t)(ldsum1<T2>(tile, (r8 + e) * PITCH + col) + bn);
                     *(half8 *)o = hv;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) {
                         const int ss = s8 + e;
-                        if (ss >= P.q_soff + ta && ss < P.q_soff + tb) o[e] = (half_t)(ldsum1(tile, (r8 + e) * PITCH + col) + bn);
+                        if (ss >= P.q_soff + ta && ss < P.q_soff + tb) o[e] = (half_t)(ldsum1<T2>(tile, (r8 + e) * PITCH + col) + bn);
                     }
                 }
             }
@@ -720,36 +744,39 @@ struct SkFix {
     }
 };
 
-// One C tile (rows m0.., columns n0..) over the K tiles [kbeg, kbeg + nk): the pipelined K loop,
-// then either the epilogue (part == null; ks = split index for a classic split-K partial) or a raw
-// f32 [BM][BN] store of the accumulators to part (a stream-K segment, finished by the fixup kernel).
-// HL: problems may read half-width W (hi|lo A operand); SEG: more tiles follow in this workgroup
-// (stream-K), so the LDS C tile is released with a barrier at the end.
-// NSX: LDS stages (4: 128 KB, one workgroup per CU; 2: 68 KB, two workgroups per CU, for grids
-// of several rounds where the second workgroup covers the first's barrier and load waits).
-template <int EPI, bool HL, bool SEG, int NSX = NS, bool BF = false>
-__device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, int kbeg, int nk, float *part, int ks,
-                                          int tid, const SkFix *fx = nullptr) {
-    // stage s: A tile at smem + s*STAGE, W tile at smem + (NSX + s)*STAGE; reused for the C tile
-    constexpr int SMEM = 2 * NSX * STAGE > BM * TP * 2 ? 2 * NSX * STAGE : BM * TP * 2;
-    __shared__ __attribute__((aligned(1024))) half_t smem[SMEM];
+// LDS stages of the hi|lo ring (a stage is one 16 KB A tile and one 8 KB W half tile): the 128 KB ring
+// of four plain stages becomes six (144 KB), the two-workgroups-per-CU ring three (72 KB)
+constexpr int hl_stages(int nsx) { return nsx == 2 ? 3 : 6; }
 
+// The K loop of one C tile (rows m0.., columns n0..) over the K tiles [kbeg, kbeg + nk): wave w
+// leaves rows 32*(w>>1)..+31 and columns 64*(w&1)..+63 of the product in acc, as 2 x 4 MFMA blocks.
+// HLP: A rows are paired (PAIR: every 32 channels as 32 hi, then 32 lo halves; Kc = 2 x channels) and W
+// has the channels once (GemmProblem::w_half). A K tile is 32 channels: 128 A rows of 128 bytes
+// (hi chunks 0..3, lo chunks 4..7) and 128 W rows of 64 bytes, and each W fragment read from LDS
+// feeds the hi and the lo product. Against staging W a second time for the lo half (64-wide hi and lo
+// K tiles in turn) that is 24 instead of 32 KB through the L2 -> LDS path and 8 instead of 12
+// fragment reads per 16 MFMAs of a wave.
+template <int EPI, bool HLP, int NSX, bool BF>
+__device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, int m0, int n0, int kbeg, int nk, int tid,
+                                           floatx4 (&acc)[2][4]) {
+    constexpr int NST = HLP ? hl_stages(NSX) : NSX;          // stages
+    constexpr int WST = HLP ? STAGE / 2 : STAGE;             // halves of a W stage
+    constexpr int LPT = HLP ? 3 : 4;                         // DMAs per wave per K tile
+    // stage s: A tile at smem + s*STAGE, W tile at smem + NST*STAGE + s*WST
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int M = P.M, N = P.N, lda = P.lda, Kc = P.Kc, pad = P.pad, aT = P.a_T;
-    // w_half: W holds hc = Kc/2 channels per tap and the A row of a tap is [hi (hc) | lo (hc)]; the
-    // tap's K tiles run interleaved (hi chunk c, lo chunk c, hi chunk c+1, ...) so the second read
-    // of a W tile follows the first at once (L2 hit)
-    const int hl = HL && P.w_half ? 1 : 0, hc = Kc / 2;
     const RowMap am = P.amap;
     const int ldw = P.ldw;
 
     const i32x4 rsa = make_rsrc(P.A);
     const i32x4 rsb = make_rsrc(P.W);
 
-    // loader rows of this lane: wave*16 + i*8 + (lane >> 3), chunk (lane & 7) ^ (lane >> 3).
+    // loader rows of this lane: wave*16 + i*8 + (lane >> 3), chunk (lane & 7) ^ (lane >> 3); of a W
+    // half tile: row wave*16 + (lane >> 2), chunk (lane & 3) ^ (row >> 1 & 3).
     // A row offsets are kept for tap 0 (byte offset of source row t - pad); tap j adds j*lda.
     const int lr = lane >> 3, lc = (lane & 7) ^ lr;
-    int a_base[2], a_ts0[2], b_off[2];
+    int a_base[2], a_ts0[2];
+    unsigned vb[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int r = wave * 16 + i * 8 + lr;
@@ -759,31 +786,32 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
         const int t = mm - b * am.L;
         a_ts0[i] = m < M ? t - pad : -(1 << 29);   // source position at tap 0; invalid rows never pass
         a_base[i] = ((b * am.seg + am.off + t - pad) * lda + lc * 8) * 2;
-        const int n = n0 + r;
-        b_off[i] = n < N ? (n * ldw + lc * 8) * 2 : -1;
+        const int n = n0 + (HLP ? wave * 16 + (lane >> 2) : r);
+        const int ch = HLP ? (lane & 3) ^ ((lane >> 3) & 3) : lc;
+        vb[i] = n < N ? (unsigned)((n * ldw + ch * 8) * 2) : 0x80000000u;   // W row offsets are fixed
     }
     const int lda2 = lda * 2;
     // K tiles are issued in order kbeg, kbeg + 1, ...: the source-row offset of the tap (tap*dil),
     // the channel offset and the W column of the next one are carried from call to call (no
-    // division in the loop). The taps run in order (each tap's hi and lo chunks interleaved for
-    // hi|lo problems), except in the snake-conv kernels: there K tile kt is channel chunk
-    // kt / taps of tap kt % taps, so the 7 taps of a chunk re-read the same A rows (shifted by
-    // dil) in consecutive K tiles while they are still in L2 (4% of a VAE decode; the DiT's k3
-    // convs measured 0.4% slower that way).
-    // The same kernels read paired rows (PAIR): one K tile is 32 channels with both parts of A and W,
-    // and feeds three products per fragment pair. As a GEMM over [hi | lo | hi] x [W_hi | W_hi | W_lo]
-    // every part that enters two products was staged and read from LDS twice (18 fragments and 48 KB
-    // per 24 MFMAs of a wave against 12 and 32 KB now), and the loop is bound by those: 8 s decode
-    // 4.40 -> 3.41 ms, 1 s 1.07 -> 0.89 ms (same box; operand rows also shrink from 6 to 4 bytes a value).
+    // division in the loop). The taps run in order, except in the snake-conv kernels: there K tile
+    // kt is channel chunk kt / taps of tap kt % taps, so the 7 taps of a chunk re-read the same A
+    // rows (shifted by dil) in consecutive K tiles while they are still in L2 (4% of a VAE decode;
+    // the DiT's k3 convs measured 0.4% slower that way).
+    // The same kernels read paired rows (PAIR) of both operands: one K tile is 32 channels with both
+    // parts of A and W, and feeds three products per fragment pair. As a GEMM over [hi | lo | hi] x
+    // [W_hi | W_hi | W_lo] every part that enters two products was staged and read from LDS twice
+    // (18 fragments and 48 KB per 24 MFMAs of a wave against 12 and 32 KB now), and the loop is bound
+    // by those: 8 s decode 4.40 -> 3.41 ms, 1 s 1.07 -> 0.89 ms (same box; operand rows also shrink
+    // from 6 to 4 bytes a value).
     constexpr bool chunk_major = EPI == EPI_SNAKE || EPI == EPI_RSNAKE, pairs = chunk_major;
     const int dil = EPI == EPI_SNAKE ? P.dil : 1;   // dilated taps only in the snake-conv kernels
     const int taps = P.taps;
     int nt_tap, nt_trow, nt_kin, nt_kw;
-    if (!chunk_major || hl) {
+    if (!chunk_major) {
         nt_tap = kbeg * BK / Kc;
         nt_trow = nt_tap * dil;
         nt_kin = kbeg * BK - nt_tap * Kc;
-        nt_kw = hl ? nt_tap * hc + ((nt_kin >> 7) << 6) : kbeg * BK;
+        nt_kw = kbeg * (HLP ? BK / 2 : BK);
     } else {
         const int c0 = kbeg / taps;
         nt_tap = kbeg - c0 * taps;
@@ -795,8 +823,7 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
     // out of range where it falls outside its sample), rebuilt after an issue whose successor
     // shifts the rows (every K tile of the snake convs, once per tap otherwise): the rebuild's
     // branch then follows the DMAs instead of splitting them from the MFMAs around the barrier.
-    // W row offsets are fixed.
-    unsigned va[2], vb[2];
+    unsigned va[2];
     int va_trow = nt_trow;
     auto set_va = [&]() {
 #pragma unroll
@@ -806,17 +833,13 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
         }
     };
     set_va();
-#pragma unroll
-    for (int i = 0; i < 2; ++i) vb[i] = b_off[i] >= 0 ? (unsigned)b_off[i] : 0x80000000u;
-    const unsigned ldsw = lds_addr(smem) + wave * 2048;   // this wave's 2 KB of each operand tile
+    const unsigned ldsa = lds_addr(smem) + wave * 2048;                                   // this wave's 2 KB of an A tile
+    const unsigned ldsb = lds_addr(smem) + NST * STAGE * 2 + wave * (HLP ? 1024 : 2048);   // and its part of a W tile
     auto issue = [&](int kt, int stage) {
         (void)kt;   // = the previous call's kt + 1
         const int kin = nt_kin, kw = nt_kw;
-        // hi|lo: K tile j of the tap is chunk j >> 1 of the hi (j even) or lo (j odd) half
-        const int odd = (kin >> 6) & 1;
-        const int acol = hl ? odd * hc + ((kin >> 7) << 6) : kin;
-        if (!chunk_major || hl) {
-            nt_kw += (hl && !odd) ? 0 : BK;
+        if (!chunk_major) {
+            nt_kw += HLP ? BK / 2 : BK;
             nt_kin += BK;
             if (nt_kin == Kc) {
                 nt_kin = 0;
@@ -831,27 +854,26 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
             nt_trow += dil;
             nt_kw += Kc;
         }
-        const unsigned sa = ldsw + stage * STAGE * 2, sb = ldsw + (NSX + stage) * STAGE * 2;
+        const unsigned sa = ldsa + stage * STAGE * 2, sb = ldsb + stage * WST * 2;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) dma16s(rsa, va[i], (unsigned)acol * 2, sa + i * 1024);
+        for (int i = 0; i < 2; ++i) dma16s(rsa, va[i], (unsigned)kin * 2, sa + i * 1024);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) dma16s(rsb, vb[i], (unsigned)kw * 2, sb + i * 1024);
+        for (int i = 0; i < LPT - 2; ++i) dma16s(rsb, vb[i], (unsigned)kw * 2, sb + i * 1024);
         if (nt_trow != va_trow) {
             va_trow = nt_trow;
             set_va();
         }
     };
 
-    // wave w owns rows 32*(w>>1)..+31 and columns 64*(w&1)..+63 of the tile over the full K:
-    // 2 x 4 MFMA blocks of 16x16, two 32-wide K halves per 64-wide stage
-    floatx4 acc[2][4];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     const int wm = wave >> 1, wn = wave & 1;
-    // operand read offsets (halves) inside a stage, per K half kh: slot (4kh + lane>>4) ^ (row & 7)
+    // operand read offsets (halves) inside a stage, per half kh of the 64 staged columns: slot
+    // (4kh + lane>>4) ^ (row & 7); in a W half tile (rows of 4 chunks) slot (lane>>4) ^ (row>>1 & 3),
+    // which puts 8 rows' chunks into 8 distinct 16-byte slots mod 128 bytes as well
     int a_rd[2][2], b_rd[2][4];
 #pragma unroll
     for (int kh = 0; kh < 2; ++kh) {
@@ -859,26 +881,31 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
 #pragma unroll
         for (int i = 0; i < 2; ++i) a_rd[kh][i] = (wm * 32 + i * 16 + (lane & 15)) * BK + slot * 8;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b_rd[kh][j] = (wn * 64 + j * 16 + (lane & 15)) * BK + slot * 8;
+        for (int j = 0; j < 4; ++j) {
+            const int row = wn * 64 + j * 16 + (lane & 15);
+            b_rd[kh][j] = HLP ? row * (BK / 2) + ((lane >> 4) ^ ((lane >> 1) & 3)) * 8 : row * BK + slot * 8;
+        }
     }
     auto compute = [&](int stage) {
-        const half_t *sa = smem + stage * STAGE, *sb = smem + (NSX + stage) * STAGE;
-        if constexpr (pairs) {   // half 0 holds the hi parts of 32 channels, half 1 their lo parts
-            half8 af[2][2], bf[2][4];
+        const half_t *sa = smem + stage * STAGE, *sb = smem + NST * STAGE + stage * WST;
+        if constexpr (pairs || HLP) {   // half 0 of the A tile holds 32 channels' hi parts, half 1 their lo parts
+            constexpr int WP = pairs ? 2 : 1;   // W parts
+            half8 af[2][2], bf[WP][4];
 #pragma unroll
             for (int kh = 0; kh < 2; ++kh) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) af[kh][i] = *(const half8 *)(sa + a_rd[kh][i]);
+                if (kh < WP)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) bf[kh][j] = *(const half8 *)(sb + b_rd[kh][j]);
+                    for (int j = 0; j < 4; ++j) bf[kh][j] = *(const half8 *)(sb + b_rd[kh][j]);
             }
 #pragma unroll
-            for (int q = 0; q < 3; ++q)   // hi * hi, lo * hi, hi * lo
+            for (int q = 0; q < WP + 1; ++q)   // hi * hi, lo * hi, hi * lo
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[q == 1][i], bf[q == 2][j], acc[i][j], 0, 0, 0);
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[q == 1][i], bf[q / 2][j], acc[i][j], 0, 0, 0);
             return;
         }
 #pragma unroll
@@ -901,40 +928,64 @@ __device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, 
         }
     };
 
-    // Loop invariant at the top of an iteration: tile kt has landed in stage kt%NS for every wave,
-    // tiles kt+1..kt+NS-1 are in flight. Each step multiplies one stage, waits for its own DMAs of
-    // the next tile (4 per wave per tile), meets the other waves at the barrier (the stage just used
-    // is now free) and refills that stage NS tiles ahead.
+    // Loop invariant at the top of an iteration: tile kt has landed in stage kt%NST for every wave,
+    // tiles kt+1..kt+NST-1 are in flight. Each step multiplies one stage, waits for its own DMAs of
+    // the next tile (LPT per wave per tile), meets the other waves at the barrier (the stage just used
+    // is now free) and refills that stage NST tiles ahead.
     issue(0, 0);
 #pragma unroll
-    for (int j = 1; j < NSX - 1; ++j)
+    for (int j = 1; j < NST - 1; ++j)
         if (nk > j) issue(j, j);
-    wait_vmcnt(4 * min(nk - 1, NSX - 2));
+    auto wait_left = [&](int n) {   // until only n later tiles' DMAs are in flight
+        if constexpr (HLP) wait_tiles<LPT, NST - 2>(n);
+        else wait_vmcnt(4 * n);
+    };
+    wait_left(min(nk - 1, NST - 2));
     block_barrier();
-    if (nk > NSX - 1) issue(NSX - 1, NSX - 1);
+    if (nk > NST - 1) issue(NST - 1, NST - 1);
 #define TSN_GEMM_STEP(NEXT, S)                                                                  \
     {                                                                                           \
         compute(S);                                                                             \
-        wait_vmcnt(4 * (NSX - 2));                                                              \
+        wait_left(NST - 2);                                                                     \
         block_barrier();                                                                        \
         issue(NEXT, S);                                                                         \
     }
     int kt = 0;
-    for (; kt + 2 * NSX <= nk; kt += NSX) {
+    for (; kt + 2 * NST <= nk; kt += NST) {
 #pragma unroll
-        for (int s2 = 0; s2 < NSX; ++s2) TSN_GEMM_STEP(kt + NSX + s2, s2)
+        for (int s2 = 0; s2 < NST; ++s2) TSN_GEMM_STEP(kt + NST + s2, s2)
     }
 #undef TSN_GEMM_STEP
-    // tail: the last < 2*NSX tiles; tile kt is visible, kt+1..min(kt+NSX-1, nk-1) in flight
+    // tail: the last < 2*NST tiles; tile kt is visible, kt+1..min(kt+NST-1, nk-1) in flight
     for (; kt < nk; ++kt) {
-        const int st = kt % NSX;
+        const int st = kt % NST;
         compute(st);
         if (kt + 1 < nk) {
-            wait_vmcnt(4 * min(nk - 2 - kt, NSX - 2));
+            wait_left(min(nk - 2 - kt, NST - 2));
             block_barrier();
-            if (kt + NSX < nk) issue(kt + NSX, st);
+            if (kt + NST < nk) issue(kt + NST, st);
         }
     }
+}
+
+// One C tile over the K tiles [kbeg, kbeg + nk): the K loop,
+// then either the epilogue (part == null; ks = split index for a classic split-K partial) or a raw
+// f32 [BM][BN] store of the accumulators to part (a stream-K segment, finished by the fixup kernel).
+// HL: problems may read half-width W (hi|lo A operand); SEG: more tiles follow in this workgroup
+// (stream-K), so the LDS C tile is released with a barrier at the end.
+// NSX: LDS stages (4: 128 KB, one workgroup per CU; 2: 68 KB, two workgroups per CU, for grids
+// of several rounds where the second workgroup covers the first's barrier and load waits); hi|lo
+// problems take hl_stages(NSX).
+template <int EPI, bool HL, bool SEG, int NSX = NS, bool BF = false>
+__device__ __forceinline__ void pipe_tile(const GemmProblem &P, int m0, int n0, int kbeg, int nk, float *part, int ks,
+                                          int tid, const SkFix *fx = nullptr) {
+    constexpr int RING = HL ? hl_stages(NSX) * (STAGE + STAGE / 2) : 2 * NSX * STAGE;   // >= the plain ring
+    constexpr int SMEM = RING > BM * TP * 2 ? RING : BM * TP * 2;
+    __shared__ __attribute__((aligned(1024))) half_t smem[SMEM];   // the ring, then the C tile
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+    floatx4 acc[2][4];
+    if (HL && P.w_half) pipe_kloop<EPI, HL, NSX, BF>(P, smem, m0, n0, kbeg, nk, tid, acc);
+    else pipe_kloop<EPI, false, NSX, BF>(P, smem, m0, n0, kbeg, nk, tid, acc);
     // Every DMA has landed (the last tile was waited for). The waves store their accumulators as a
     // row-major f32 C tile in LDS, then all 8 waves run the epilogue on 8-column chunks (16-byte
     // accesses).
@@ -1533,6 +1584,178 @@ __global__ __launch_bounds__(512, 1) void gemm_small2_kernel(const GemmBatch bt)
     small_tile<EPI, 2, SNS2>(bt);
 }
 
+// ---------------------------------------------------------------------------------------------
+// gemm_hl2_kernel: hi|lo operands (every problem w_half) on grids that fit one round of the chip.
+// Tiles of 16*MB rows x 128 columns over K steps of 64 channels: a stage holds the rows' two paired
+// lines (2 x 128 bytes) and 128 W rows of 128 bytes. Two groups of four waves share the tile: group g
+// multiplies channels 32g .. 32g + 31 of every step, each wave 8*MB rows x 64 columns (MB + 4 fragment
+// reads per 4*MB MFMAs), and the epilogue adds the two partial products (group 0's first).
+//
+// Why this kernel: at the checkpoint graph's 344 latent rows the 128x128 grids leave CUs idle (QKV 72
+// tiles) or are cut into K ranges whose partial tiles cost more than they save (SwiGLU, stream-K: 43
+// us a launch, of which about 26 do not depend on M). Choosing the rows of a tile by the grid instead
+// (96: 4 x 44 tiles for the SwiGLU; 64: 6 x 24 for QKV) keeps each K loop whole on one CU. Why steps of
+// 64 channels: the loop runs at the L2 -> LDS rate, and W rows of 64 bytes (steps of 32) take whole
+// requests for half lines: SwiGLU 39.4 us a launch with them.
+// ---------------------------------------------------------------------------------------------
+constexpr int hl2_stages(int mb) { return mb == 8 ? 3 : mb == 2 ? 6 : 4; }   // 144, 160, 128, 144 KB (MB 8, 6, 4, 2)
+
+template <int EPI, int MB>
+__global__ __launch_bounds__(512, 1) void gemm_hl2_kernel(const GemmBatch bt) {
+    constexpr int ROWS = 16 * MB, NST = hl2_stages(MB);
+    constexpr int AHALF = ROWS * BK, AST = 2 * AHALF, WST = STAGE;   // halves: a group's A tile, both, the W tile
+    constexpr int NA = MB / 2, LPT = NA + 2;    // A and W DMAs per wave per step
+    constexpr int T2 = ROWS * TP;               // the second group's C tile (floats)
+    constexpr int RING = NST * (AST + WST);     // A stages, then W stages
+    constexpr int SMEM = RING > 4 * T2 ? RING : 4 * T2;
+    __shared__ __attribute__((aligned(1024))) half_t smem[SMEM];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int grp = wave >> 2, w4 = wave & 3;
+    const int wg = xcd_remap(blockIdx.x, bt.total_tiles);
+    const int pi = (bt.nprob > 2 && wg >= bt.p[2].tile_start) ? 2 : (bt.nprob > 1 && wg >= bt.p[1].tile_start) ? 1 : 0;
+    const GemmProblem &P = bt.p[pi];
+    const int local = wg - P.tile_start, per_split = P.tiles_m * P.tiles_n, ks = local / per_split;
+    int tm, tn;
+    tile_mn(local - ks * per_split, P.tiles_m, P.tiles_n, tm, tn);
+    const int m0 = tm * ROWS, n0 = tn * BN;
+    const int nkt = P.K / (2 * BK);   // K steps, shared out over the splits
+    const int kbeg = (int)((long long)ks * nkt / P.splits), nk = (int)((long long)(ks + 1) * nkt / P.splits) - kbeg;
+    const int M = P.M, N = P.N, lda = P.lda, Kc = P.Kc, pad = P.pad, aT = P.a_T, ldw = P.ldw;
+    const RowMap am = P.amap;
+    const i32x4 rsa = make_rsrc(P.A);
+    const i32x4 rsb = make_rsrc(P.W);
+
+    // loader: the group's own A tile (line grp of each row), 8-row blocks w4*NA + i; W 8-row blocks
+    // 2*wave + i; chunk (lane & 7) ^ (lane >> 3) of row lane >> 3
+    const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+    int a_base[NA], a_ts0[NA];
+    unsigned va[NA], vb[2];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int m = m0 + (w4 * NA + i) * 8 + lr;
+        const int mm = m < M ? m : 0;
+        const int b = mm / am.L, t = mm - b * am.L;
+        a_ts0[i] = m < M ? t - pad : -(1 << 29);
+        a_base[i] = ((b * am.seg + am.off + t - pad) * lda + grp * BK + lc * 8) * 2;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int n = n0 + (wave * 2 + i) * 8 + lr;
+        vb[i] = n < N ? (unsigned)((n * ldw + lc * 8) * 2) : 0x80000000u;
+    }
+    // tap row and column inside the tap of the next step, carried (Kc is a multiple of 2*BK)
+    int nt_trow = kbeg * 2 * BK / Kc, nt_kin = kbeg * 2 * BK - nt_trow * Kc, nt_kw = kbeg * BK;
+    int va_trow = nt_trow;
+    auto set_va = [&]() {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int ts = a_ts0[i] + va_trow;
+            va[i] = (ts >= 0 && ts < aT) ? (unsigned)(a_base[i] + va_trow * lda * 2) : 0x80000000u;
+        }
+    };
+    set_va();
+    const unsigned ldsa = lds_addr(smem) + (grp * AHALF + w4 * NA * 512) * 2;
+    const unsigned ldsb = lds_addr(smem) + (NST * AST + wave * 1024) * 2;
+    auto issue = [&](int stage) {
+        const int kin = nt_kin, kw = nt_kw;
+        nt_kw += BK;
+        nt_kin += 2 * BK;
+        if (nt_kin == Kc) {
+            nt_kin = 0;
+            ++nt_trow;
+        }
+        const unsigned sa = ldsa + stage * AST * 2, sb = ldsb + stage * WST * 2;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) dma16s(rsa, va[i], (unsigned)kin * 2, sa + i * 1024);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) dma16s(rsb, vb[i], (unsigned)kw * 2, sb + i * 1024);
+        if (nt_trow != va_trow) {
+            va_trow = nt_trow;
+            set_va();
+        }
+    };
+
+    floatx4 acc[NA][4];
+#pragma unroll
+    for (int i = 0; i < NA; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int wm = w4 >> 1, wn = w4 & 1;
+    // operand read offsets inside a stage: A row r of the group's tile, hi chunk lane>>4 (lo: + 4), and W
+    // row r, chunk 4*grp + lane>>4, at slot chunk ^ (r & 7)
+    int a_rd[2];
+#pragma unroll
+    for (int kh = 0; kh < 2; ++kh)
+        a_rd[kh] = grp * AHALF + (wm * NA * 16 + (lane & 15)) * BK + ((kh * 4 + (lane >> 4)) ^ (lane & 7)) * 8;
+    const int b_rd = NST * AST + (wn * 64 + (lane & 15)) * BK + ((grp * 4 + (lane >> 4)) ^ (lane & 7)) * 8;
+    // The two groups alternate: while one reads its fragments from LDS and refills a stage, the other
+    // issues MFMAs, so on every SIMD one wave keeps the LDS port and one the matrix core busy. Each step
+    // has a read phase and a multiply phase, closed by one workgroup barrier each; group 1 runs one
+    // barrier behind. When a wave refills the stage of step kt - 1 (in its read phase of step kt), both
+    // groups' reads of that stage have ended a barrier earlier or more; its own DMAs of step kt + 1 are
+    // waited for before the read phase's barrier, two barriers before any wave reads that step.
+    auto wait_left = [&](int n) { wait_tiles<LPT, NST - 2>(n); };   // until only n later steps' DMAs are in flight
+    auto phase_end = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto step = [&](int kt, int stage, int refill, bool steady) {
+        const half_t *sa = smem + stage * AST, *sb = smem + stage * WST;
+        half8 af[2][NA], bf[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) bf[j] = *(const half8 *)(sb + b_rd + j * 16 * BK);
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+            for (int i = 0; i < NA; ++i) af[kh][i] = *(const half8 *)(sa + a_rd[kh] + i * 16 * BK);
+        asm volatile("" ::: "memory");
+        if (steady || (kt > 0 && kt - 1 + NST < nk)) issue(refill);   // the stage of step kt - 1
+        wait_left(steady ? NST - 2 : max(min(nk - 2 - kt, NST - 2), 0));
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // this wave's LDS reads are done (lgkmcnt 0)
+        phase_end();
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh)
+#pragma unroll
+            for (int i = 0; i < NA; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[kh][i], bf[j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_s_setprio(0);
+        phase_end();
+    };
+#pragma unroll
+    for (int j = 0; j < NST; ++j)
+        if (nk > j) issue(j);
+    wait_tiles<LPT, NST - 1>(min(nk, NST) - 1);
+    block_barrier();
+    if (grp == 1) phase_end();
+    // step kt refills stage (kt - 1) % NST with step kt - 1 + NST
+    int kt = 1;
+    step(0, 0, 0, false);
+    for (; kt + 2 * NST - 1 <= nk; kt += NST) {
+#pragma unroll
+        for (int u = 0; u < NST; ++u) step(kt + u, (1 + u) % NST, u, true);
+    }
+    for (; kt < nk; ++kt) step(kt, kt % NST, (kt - 1) % NST, false);
+    if (grp == 0) phase_end();
+    block_barrier();
+    float *tile = (float *)smem;
+    {
+        float *t = tile + grp * T2;
+        const int rb = wm * NA * 16 + (lane >> 4) * 4, cb = wn * 64 + (lane & 15);
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) t[(rb + i * 16 + r) * TP + cb + j * 16] = acc[i][j][r];
+    }
+    block_barrier();
+    tile_epilogue<EPI, TP, ROWS, T2>(P, tile, m0, n0, ks, tid);
+}
+
 // the workgroup w of G holding unit u: w*U/G <= u < (w + 1)*U/G
 __device__ __forceinline__ long long sk_owner(long long u, long long U, long long G) {
     long long w = u * G / U;
@@ -1751,16 +1974,91 @@ void gemm_problem_init(GemmProblem &p) {
     p.splits = 1;
 }
 
+// The one-round hi|lo kernel (gemm_hl2_kernel) for a batch whose every problem is w_half: the rows of a
+// tile (32, 64, 96 or 128) and, where the epilogue takes partial sums, one K split with the least
+// estimated time among those whose grid fits one round of the chip; false if none does. A K tile's
+// time per tile height is the LDS port's (fragment reads plus DMA writes, 128 bytes a clock); a split
+// adds its partial sums written and read (about 2.15 MB per 128-row K tile) and split_overhead K tiles.
+static bool hl2_plan(GemmBatch &b, int epi) {
+    static const int cost[5] = {0, 281, 375, 470, 562};   // clocks per K tile, by MB / 2
+    bool lo = false;
+    int nkmin = 1 << 30;
+    for (int i = 0; i < b.nprob; ++i) {
+        if (!b.p[i].w_half) return false;
+        lo = lo || b.p[i].y_pair;
+        nkmin = std::min(nkmin, b.p[i].K / BK);
+    }
+    const bool can_split = b.ws && !lo && (epi == EPI_RESID || epi == EPI_STORE);
+    double best = 1e30;
+    int best_mb = 0, best_s = 1;
+    for (int mb = 2; mb <= 8; mb += 2)
+        for (int s = 1; s <= (can_split ? nkmin / 8 : 1); ++s) {
+            long long wg = 0;
+            int nk = 0;
+            double part = 0;
+            for (int i = 0; i < b.nprob; ++i) {
+                const GemmProblem &p = b.p[i];
+                wg += (long long)((p.M + 16 * mb - 1) / (16 * mb)) * ((p.N + BN - 1) / BN) * s;
+                nk = std::max(nk, 2 * ((p.K / (2 * BK) + s - 1) / s));
+                part += 8.0 * s * p.M * (double)p.N;
+            }
+            if (wg > NCU || (s > 1 && part / 2 > (double)b.ws_bytes)) continue;
+            const double c = (double)nk * cost[mb / 2] + (s > 1 ? cost[4] * (b.split_overhead + part / 2.15e6) : 0.0);
+            if (c < best) {
+                best = c;
+                best_mb = mb;
+                best_s = s;
+            }
+        }
+    if (best_mb == 0) return false;
+    int tiles = 0;
+    size_t off = 0;
+    for (int i = 0; i < b.nprob; ++i) {
+        GemmProblem &p = b.p[i];
+        p.splits = best_s;
+        p.ws = nullptr;
+        if (best_s > 1) {
+            p.ws = b.ws + off;
+            off += (size_t)best_s * p.M * p.N;
+        }
+        p.tiles_m = (p.M + 16 * best_mb - 1) / (16 * best_mb);
+        p.tiles_n = (p.N + BN - 1) / BN;
+        p.tile_start = tiles;
+        tiles += p.tiles_m * p.tiles_n * best_s;
+    }
+    static const char *const names[4] = {"gemm_hl2_kernel<0>", "gemm_hl2_kernel<1>", "gemm_hl2_kernel<2>", "gemm_hl2_kernel<3>"};
+    b.total_tiles = tiles;
+    b.hl2 = best_mb;
+    b.hl = 1;
+    b.pipe = 1;
+    b.sk = 0;
+    b.sk_cnt = nullptr;
+    b.ns2 = b.wide = 0;
+    b.pf_nwg = b.gv_nwg = 0;
+    b.kname = names[epi];
+    return true;
+}
+
+template <int EPI>
+static void hl2_launch(const GemmBatch &b, hipStream_t st) {
+    const dim3 grid(b.total_tiles), block(512);
+    if (b.hl2 == 2) TSN_LAUNCH((gemm_hl2_kernel<EPI, 2>), grid, block, 0, st, b);
+    else if (b.hl2 == 4) TSN_LAUNCH((gemm_hl2_kernel<EPI, 4>), grid, block, 0, st, b);
+    else if (b.hl2 == 6) TSN_LAUNCH((gemm_hl2_kernel<EPI, 6>), grid, block, 0, st, b);
+    else TSN_LAUNCH((gemm_hl2_kernel<EPI, 8>), grid, block, 0, st, b);
+}
+
 int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
     TSN_REQUIRE(b.nprob >= 1 && b.nprob <= 3, "gemm: 1 to 3 problems");
     b.pf_nwg = 0;
     b.gv_nwg = 0;
+    b.hl2 = 0;
     if (b.bf16) {   // one data-parallel schedule: no workspace, so no split and no stream-K
         TSN_REQUIRE(epi == EPI_STORE && !a_f32 && !b.small, "gemm bf16: plain store epilogue, bf16 A");
         b.ws = nullptr;
         b.ws_bytes = 0;
         for (int i = 0; i < b.nprob; ++i)
-            TSN_REQUIRE(!b.p[i].y_f16 && !b.p[i].w_half && !b.p[i].y_lo && b.p[i].taps == 1,
+            TSN_REQUIRE(!b.p[i].y_f16 && !b.p[i].w_half && !b.p[i].y_pair && b.p[i].taps == 1,
                         "gemm bf16: one tap, f32 Y, no hi|lo operands");
     }
     int tiles = 0;
@@ -1778,14 +2076,13 @@ int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
         if (p.w_half)
             TSN_REQUIRE(p.Kc % (2 * BK) == 0 && p.ldw >= p.taps * (p.Kc / 2),
                         "gemm: half-width W needs Kc a multiple of 128 and ldw >= taps*Kc/2");
-        if (p.y_lo) {
+        if (p.y_pair) {
             const int wout = epi == EPI_SWIGLU ? p.N / 2 : p.N;
-            TSN_REQUIRE((epi == EPI_STORE || epi == EPI_SWIGLU) && p.y_f16 && p.y_lo % 8 == 0 && p.y_lo >= wout &&
-                            p.ldy >= p.y_lo + wout,
-                        "gemm: hi|lo output needs f16 Y, lo offset a multiple of 8 past the hi columns, ldy >= y_lo + width");
+            TSN_REQUIRE((epi == EPI_STORE || epi == EPI_SWIGLU) && p.y_f16 && wout % PAIR == 0 && p.ldy >= 2 * wout,
+                        "gemm: hi|lo output needs f16 Y, a multiple of 32 columns, ldy >= twice the width");
         }
         if (epi == EPI_SNAKE || epi == EPI_RSNAKE) {
-            TSN_REQUIRE(p.Kc % (2 * PAIR) == 0 && p.N % PAIR == 0 && !p.w_half && !p.y_lo,
+            TSN_REQUIRE(p.Kc % (2 * PAIR) == 0 && p.N % PAIR == 0 && !p.w_half && !p.y_pair,
                         "gemm snake: paired operands (whole 32-channel hi|lo groups), N a multiple of 32");
             TSN_REQUIRE(epi == EPI_RSNAKE ? p.R && p.rmap.L > 0 && p.ldr % 4 == 0 : p.Y != nullptr,
                         "gemm snake: output rows (residual: the stream R)");
@@ -1841,7 +2138,7 @@ int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
     for (int i = 0; i < b.nprob; ++i) {
         b.p[i].splits = 1;
         b.p[i].ws = nullptr;
-        any_lo = any_lo || b.p[i].y_lo;
+        any_lo = any_lo || b.p[i].y_pair;
     }
     bool any_half = false;
     for (int i = 0; i < b.nprob; ++i) any_half = any_half || b.p[i].w_half;
@@ -1903,6 +2200,7 @@ int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
         }
         return TSN_OK;
     }
+    if (pipe && any_half && hl2_plan(b, epi)) return TSN_OK;
     const bool snake_epi = epi == EPI_SNAKE || epi == EPI_RSNAKE;
     if (pipe && (epi == EPI_RESID || epi == EPI_STORE || snake_epi) && b.ws && !any_lo) {
         int nkmin = 1 << 30;
@@ -2099,6 +2397,14 @@ int gemm_launch_planned(const GemmBatch &b, int epi, bool a_f32, hipStream_t st)
             set_error("gemm small tiles: residual or plain store epilogue only");
             return TSN_ERR_ARG;
         }
+        TSN_HIP_CHECK(hipGetLastError());
+        return TSN_OK;
+    }
+    if (b.hl2) {
+        if (epi == EPI_STORE) hl2_launch<EPI_STORE>(b, st);
+        else if (epi == EPI_RESID) hl2_launch<EPI_RESID>(b, st);
+        else if (epi == EPI_QKV) hl2_launch<EPI_QKV>(b, st);
+        else hl2_launch<EPI_SWIGLU>(b, st);
         TSN_HIP_CHECK(hipGetLastError());
         return TSN_OK;
     }

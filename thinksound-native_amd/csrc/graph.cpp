@@ -194,7 +194,7 @@ double gemm_bytes(const GemmBatch &b, int epi) {
         const GemmProblem &p = b.p[i];
         double out = epi == EPI_RESID ? 8.0 : epi == EPI_SWIGLU ? 1.0 : epi == EPI_SNAKE ? 4.0
                    : epi == EPI_RSNAKE ? (p.r_add ? 8.0 : 4.0) + (p.Y ? 4.0 : 0.0) : (p.y_f16 || epi == EPI_QKV ? 2.0 : 4.0);
-        if (p.y_lo && (epi == EPI_STORE || epi == EPI_SWIGLU)) out *= 2.0;
+        if (p.y_pair && (epi == EPI_STORE || epi == EPI_SWIGLU)) out *= 2.0;
         x += 2.0 * p.M * (double)p.Kc + 2.0 * p.N * (double)p.K / (p.w_half ? 2 : 1) + out * p.M * (double)p.N;
     }
     return x;

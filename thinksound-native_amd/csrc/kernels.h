@@ -6,6 +6,12 @@
 
 namespace tsn {
 
+// Paired f16 rows: an f32 value as hi = f16(v) and lo = f16(v - hi), every PAIR columns stored as PAIR
+// hi halves, then their PAIR lo halves, so a 128-byte line holds both parts of 32 columns. Column c's
+// hi part is at pair_col(c), its lo part PAIR further.
+constexpr int PAIR = 32;
+__host__ __device__ inline int pair_col(int c) { return c + (c & ~(PAIR - 1)); }
+
 /* ------------------------------------------------------------------ GEMM (MFMA) */
 // C[M,N] = A[M,K] · W[N,K]ᵀ with f16 operands and f32 accumulation; 128x128x64 tiles,
 // v_mfma_f32_16x16x32_f16 (pipelined kernel: 8 waves, 5 direct-to-LDS stages).
@@ -19,8 +25,9 @@ struct GemmProblem {
     // dil > 1 (dilated taps) only with EPI_SNAKE.
     int taps, Kc, pad, a_T, dil;
     const half_t *W; int ldw;          // [N][K] row-major
-    // w_half: the A operand is an f16 hi|lo pair per tap (Kc = 2*IC: hi channels, then lo) and W
-    // holds IC channels per tap ([N][taps][IC], ldw >= taps*IC); both halves read the same W columns
+    // w_half: the A rows are paired: each tap's channels in groups of 32 as 32 hi halves, then their 32
+    // lo halves (Kc = 2*IC), and W holds IC channels per tap ([N][taps][IC], ldw >= taps*IC); both
+    // parts read the same W columns, so the product is f32-accurate in A
     int w_half;
     const float *bias;                 // [N] or null
     int M, N, K;
@@ -28,9 +35,9 @@ struct GemmProblem {
     // EPI_SWIGLU: W rows interleaved in 64-row blocks (w1 block j, then w3 block j), N = 2F;
     // Y[ymap(m)*ldy + 64j + c] = silu(w1 row 64j+c · a) * (w3 row 64j+c · a), f16, no bias
     void *Y; int ldy; RowMap ymap; int y_f16; int silu;
-    // f16 Y (EPI_STORE, EPI_SWIGLU): nonzero also writes lo = f16(y - f16(y)) at column offset y_lo
-    // of the same row (hi|lo operand of a following GEMM against [W | W]); K is then never split
-    int y_lo;
+    // f16 Y (EPI_STORE, EPI_SWIGLU): nonzero writes paired rows (hi = f16(y), lo = f16(y - hi)), the A
+    // operand of a following w_half GEMM; K is then never split
+    int y_pair;
     // EPI_SNAKE, EPI_RSNAKE: A and W rows are paired: every 32 channels as 32 hi halves, then their 32
     // lo halves (Kc = 2*IC), and the product sums hi*W_hi + lo*W_hi + hi*W_lo (the dropped lo*W_lo term
     // is below 2^-22 relative), f32-accurate.
@@ -110,6 +117,9 @@ struct GemmBatch {
     unsigned *sk_cnt = nullptr;
     int sk_cnt_n = 0;
     int hl = 0;   // some problem reads half-width W (selects the kernel variant)
+    // set by gemm_plan: 16-row blocks per tile (2, 4, 6 or 8) of the one-round hi|lo kernel
+    // (gemm_hl2_kernel; every problem w_half), 0 for the other kernels
+    int hl2 = 0;
     // nonzero: never stream-K, and choose the classic K split by the estimated time (waves x K tiles
     // per split, plus the partial-sum traffic). For long-K GEMMs with few tiles, whose A and W tiles
     // would not be shared in L2 under stream-K's staggered K ranges.
@@ -172,7 +182,8 @@ struct AttnArgs {
     const half_t *Q, *K, *Vt;
     int S, Sp, nh, BH;
     void *O; int o_f32; int ldo; RowMap omap;
-    int o_lo;           // f16 O: nonzero also writes lo = f16(o - f16(o)) at column offset o_lo
+    int o_pair;         // f16 O: rows s < o_pair of each sample are written paired (w_half operand rows of
+                        // 2 * nh*64 halves: 32 hi, then their 32 lo), the others as plain f16
 };
 int launch_attention(const AttnArgs &a, hipStream_t st);
 
@@ -198,8 +209,8 @@ struct LnArgs {
     PfRange pf[PF_RANGES];
     int pf_nwg;   // set by the launcher: prefetch workgroups, ahead of the row workgroups
 };
-// ymode: 0 f32 output, 1 f16 output, 2 f16 hi|lo pair (y_hi at column c, y_lo = f16(y - y_hi) at
-// column H + c; ldy >= 2H): an f16 GEMM over [hi|lo] against a [W|W] weight reproduces the f32 y.
+// ymode: 0 f32 output, 1 f16 output, 2 paired f16 rows (groups of 32 columns as 32 hi = f16(y), then
+// 32 lo = f16(y - hi); ldy >= 2H): the A operand of a w_half GEMM, which reproduces the f32 y.
 enum { LN_F32 = 0, LN_F16 = 1, LN_F16_HILO = 2 };
 int launch_ln_mod(const LnArgs &a, int ymode, hipStream_t st);
 
@@ -216,7 +227,7 @@ struct RedLnSeg {
     int ln, ln_len;
     const float *mod; int mod_ld, mod_L, shift_off, scale_off;
     void *Y; int ldy; RowMap ymap;
-    int hilo;   // this segment's LN output as an f16 hi|lo pair (lo at column H + c) whatever ymode
+    int hilo;   // this segment's LN output as paired f16 rows (LN_F16_HILO) whatever ymode
 };
 struct RedLnArgs {
     RedLnSeg seg[3];
@@ -275,18 +286,20 @@ int launch_copy_rows(const float *src, int lds, RowMap smap, float *dst, int ldd
                      int M, int H, hipStream_t st);
 // sampler step on x2 [2P][n]: v = vu + (vc - vu)*cfg; x += dt*v; both arms of prompt p get x.
 int launch_cfg_euler_pairs(const float *V, float *x2, int P, int n, float cfg, float dt, hipStream_t st);
-// x f32 rows -> out [M][2K] f16: out[m][k] = hi = f16(x), out[m][K + k] = f16(x - hi)
+// x f32 rows -> out [M][2K] f16, paired (w_half operand): groups of 32 columns as 32 hi = f16(x), then
+// 32 lo = f16(x - hi); K % 32 == 0
 int launch_split_hilo(const float *x, int ldx, RowMap xmap, half_t *out, int M, int K, hipStream_t st);
 // one launch at the start of an evaluation: temb = sinusoid(t) (skipped when t is null), z2 =
-// hi|lo split of z, and cM rows copied csrc -> cdst (each part as its standalone kernel)
+// [hi (sK) | lo (sK)] split of z, and cM rows copied csrc -> cdst (each part as its standalone kernel)
 struct EvalPrepArgs {
     const float *t; float *temb; int tnb, tD; float tmax;
     const float *z; int ldz; RowMap zmap; half_t *z2; int sM, sK;
     const float *csrc; int clds; RowMap csmap; float *cdst; int cldd; RowMap cdmap; int cM, cH;
 };
 int launch_eval_prep(const EvalPrepArgs &a, hipStream_t st);
-// bf16 [N][K] -> f16 [N][2K] = [W | W] (weight of a GEMM over a hi|lo operand)
-int launch_dup_cols_bf16_to_f16(const uint16_t *src, half_t *dst, int N, int K, hipStream_t st);
+// bf16 [N][K] -> f16 [N][2K], every group of g columns written twice (g = K: [W | W]; g = 32 against
+// paired A rows): the weight of a plain GEMM over a hi|lo operand; K % g == 0
+int launch_dup_cols_bf16_to_f16(const uint16_t *src, half_t *dst, int N, int K, int g, hipStream_t st);
 // format conversions
 int launch_bf16_to_f16(const uint16_t *src, half_t *dst, size_t n, hipStream_t st);
 int launch_bf16_to_f32(const uint16_t *src, float *dst, size_t n, hipStream_t st);
@@ -305,10 +318,10 @@ int launch_conv_weight_reorder(const void *src, int src_bf16, half_t *dst, int O
 enum { WP_SRC_BF16 = 0, WP_SRC_F32 = 1, WP_SRC_F16 = 2, WP_SRC_Q8_0 = 3 };
 int launch_weight_prep(const void *src, int src_type, void *dst, int out_f32, int OC, int IC, int KT, int dup, int ra,
                        int rb, int rc, int rd, long long dst_rows, hipStream_t st);
-// y = silu(x[m] + v[m / L]) (x [M][H], v [M/L][H] f32) as f16 hi|lo rows [M][2H] (LN_F16_HILO layout)
+// y = silu(x[m] + v[m / L]) (x [M][H], v [M/L][H] f32) as paired f16 rows [M][2H] (LN_F16_HILO)
 int launch_bcast_add_silu_f16(const float *x, const float *v, half_t *y, int L, int M, int H, hipStream_t st);
 
-// out [M][2K] f16 hi|lo of x[m][k] + pe[m % P][k] (pe null: x alone)
+// out [M][2K] paired f16 of x[m][k] + pe[m % P][k] (pe null: x alone)
 int launch_add_period_hilo(const float *x, const float *pe, int P, half_t *out, int M, int K, hipStream_t st);
 // VAE decoder (vae.hip). split_pairs: f32 rows [rows][C] (C % 32 == 0) -> paired f16 rows [rows][2C]
 // (EPI_SNAKE's operands: each 32 channels as 32 hi halves, then 32 lo halves, lo = f16(x - hi))
@@ -373,7 +386,7 @@ int conv_prep_cols(int sdt, int IC, int K);
 // sources [hi | hi | lo] of each tap's channels (the weight of a three-part product)
 int launch_conv_prepare(const void *W, int sdt, half_t *Wp, int OC, int IC, int K, hipStream_t st);
 // gathered operand rows [t0, t0 + rows) of the conv (the reference's im2col, src/net.mm:36-48):
-// parts 1 -> [rows][2*Kp] f16 hi|lo halves; parts 3 -> [rows][Kp] with [hi | lo | hi] per tap
+// parts 1 -> [rows][2*Kp] paired f16 (w_half operand); parts 3 -> [rows][Kp] with [hi | lo | hi] per tap
 int launch_conv_gather(const float *x, const ConvGeom &g, int t0, int rows, int parts, int Kp, half_t *out,
                        hipStream_t st);
 // direct f32 conv on a prepared weight (outputs too narrow for a GEMM tile)

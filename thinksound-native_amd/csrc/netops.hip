@@ -55,14 +55,14 @@ __global__ void conv_prep_kernel(const void *src, int sdt, half_t *dst, int OC, 
 }
 
 // Gathered conv operand rows t0 .. t0 + rows - 1 (the im2col of src/net.mm:36-48, in the layout of
-// the prepared weight). parts 1: row [2*Kp] = [hi (Kp) | lo (Kp)], column k*IC + ic of each half;
+// the prepared weight). parts 1: row [2*Kp] paired (groups of 32 columns as 32 hi, then 32 lo), column k*IC + ic;
 // parts 3: row [Kp], tap k = [hi | lo | hi] of its IC channels at k*3IC. Zero past the data.
 __global__ void conv_gather_kernel(const float *x, ConvGeom g, int t0, int rows, int parts, int Kp, half_t *out) {
     const int width = parts == 1 ? 2 * Kp : Kp;
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (long long)rows * width) return;
     const int r = (int)(i / width), c = (int)(i - (long long)r * width);
-    const int j = parts == 1 ? (c < Kp ? c : c - Kp) : c;
+    const int j = parts == 1 ? (c >> 6) * PAIR + (c & (PAIR - 1)) : c;
     half_t out_v = (half_t)0.0f;
     if (j < g.K * g.IC * parts) {
         const int w_ic = g.IC * parts;
@@ -70,7 +70,7 @@ __global__ void conv_gather_kernel(const float *x, ConvGeom g, int t0, int rows,
         const int ti = conv_src_row(t0 + r, k, g);
         const float v = ti >= 0 ? x[(long long)ti * g.ldx + ic] : 0.0f;
         const half_t hi = (half_t)v;
-        const bool lo = parts == 1 ? c >= Kp : part == 1;
+        const bool lo = parts == 1 ? (c & PAIR) != 0 : part == 1;
         out_v = lo ? (half_t)(v - (float)hi) : hi;
     }
     out[i] = out_v;

@@ -75,8 +75,9 @@ __global__ __launch_bounds__(256) void ln_mod_kernel(const LnArgs a) {
             const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
             const half4 lo = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
                                    (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
-            *(half4 *)((half_t *)S.Y + yrow + col) = hi;
-            *(half4 *)((half_t *)S.Y + yrow + NV * 256 + col) = lo;
+            half_t *y = (half_t *)S.Y + yrow + pair_col(col);
+            *(half4 *)y = hi;
+            *(half4 *)(y + PAIR) = lo;
         } else {
             *(float4 *)((float *)S.Y + yrow + col) = make_float4(y0, y1, y2, y3);
         }
@@ -144,12 +145,13 @@ __global__ __launch_bounds__(512) void reduce_ln_kernel(const RedLnArgs a) {
     const float y1 = d1 * inv * (1.0f + scl.y) + sh.y;
     const float y2 = d2 * inv * (1.0f + scl.z) + sh.z;
     const float y3 = d3 * inv * (1.0f + scl.w) + sh.w;
-    half_t *y = (half_t *)S.Y + rowmap_phys(S.ymap, v) * (long long)S.ldy + col;
+    const bool pair = YMODE == LN_F16_HILO || S.hilo;   // uniform over the workgroup
+    half_t *y = (half_t *)S.Y + rowmap_phys(S.ymap, v) * (long long)S.ldy + (pair ? pair_col(col) : col);
     const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
     *(half4 *)y = hi;
-    if (YMODE == LN_F16_HILO || S.hilo)   // uniform over the workgroup
-        *(half4 *)(y + H) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
-                                  (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
+    if (pair)
+        *(half4 *)(y + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
+                                     (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
 }
 
 /* ---------------- calibration probes (achievable MFMA and HBM rates) ---------------- */
@@ -363,16 +365,19 @@ __global__ void cfg_euler_pairs_kernel(const float *V, float *x2, int P, int n, 
     x2[(long long)(2 * p + 1) * n + i] = xn;
 }
 
-__device__ __forceinline__ void split_hilo_elem(const float *x, int ldx, RowMap xmap, half_t *out, int M, int K, long long i) {
+// hi|lo split of an element: groups of g columns as g hi, then their g lo halves (g = PAIR: paired rows)
+__device__ __forceinline__ void split_hilo_elem(const float *x, int ldx, RowMap xmap, half_t *out, int M, int K, int g,
+                                                long long i) {
     if (i >= (long long)M * K) return;
     const int m = (int)(i / K), k = (int)(i - (long long)m * K);
     const float v = x[rowmap_phys(xmap, m) * (long long)ldx + k];
     const half_t hi = (half_t)v;
-    out[(long long)m * 2 * K + k] = hi;
-    out[(long long)m * 2 * K + K + k] = (half_t)(v - (float)hi);
+    half_t *o = out + (long long)m * 2 * K + k + k / g * g;
+    o[0] = hi;
+    o[g] = (half_t)(v - (float)hi);
 }
 __global__ void split_hilo_kernel(const float *x, int ldx, RowMap xmap, half_t *out, int M, int K) {
-    split_hilo_elem(x, ldx, xmap, out, M, K, (long long)blockIdx.x * blockDim.x + threadIdx.x);
+    split_hilo_elem(x, ldx, xmap, out, M, K, PAIR, (long long)blockIdx.x * blockDim.x + threadIdx.x);
 }
 
 // The start of an evaluation in one launch: the timestep sinusoid (optional), the hi|lo split of
@@ -385,18 +390,19 @@ __global__ void eval_prep_kernel(const EvalPrepArgs a) {
     if (blk < nt) {
         temb_elem(a.t, a.temb, a.tnb, a.tD, a.tmax, blk * 256 + threadIdx.x);
     } else if (blk < nt + ns) {
-        split_hilo_elem(a.z, a.ldz, a.zmap, a.z2, a.sM, a.sK, (long long)(blk - nt) * 256 + threadIdx.x);
+        split_hilo_elem(a.z, a.ldz, a.zmap, a.z2, a.sM, a.sK, a.sK, (long long)(blk - nt) * 256 + threadIdx.x);
     } else if (blk - nt - ns < a.cM) {
         copy_row(a.csrc, a.clds, a.csmap, a.cdst, a.cldd, a.cdmap, a.cH, blk - nt - ns);
     }
 }
-__global__ void dup_cols_kernel(const uint16_t *src, half_t *dst, int N, int K) {
+__global__ void dup_cols_kernel(const uint16_t *src, half_t *dst, int N, int K, int g) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (long long)N * K) return;
     const int n = (int)(i / K), k = (int)(i - (long long)n * K);
     const half_t w = (half_t)bf16_to_f32(src[i]);
-    dst[(long long)n * 2 * K + k] = w;
-    dst[(long long)n * 2 * K + K + k] = w;
+    half_t *d = dst + (long long)n * 2 * K + k + k / g * g;
+    d[0] = w;
+    d[g] = w;
 }
 __global__ void bf16_to_f16_kernel(const uint16_t *s, half_t *d, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -472,9 +478,8 @@ __global__ void weight_prep_kernel(const void *src, int src_type, void *dst, int
     }
 }
 
-// y = silu(x[m][c] + v[m / L][c]) as an f16 hi|lo pair: y[m][c] = hi = f16(y), y[m][H + c] =
-// f16(y - hi). Rows of extended_c = sync_gather + global_c with SiLU applied, the operand of the
-// per-row modulation GEMM against [W | W] (src/dit_fwd.cpp:133-136).
+// y = silu(x[m][c] + v[m / L][c]) as paired f16 rows. Rows of extended_c = sync_gather + global_c with SiLU applied, the operand of the
+// per-row modulation GEMM (src/dit_fwd.cpp:133-136).
 __global__ void bcast_add_silu_kernel(const float *x, const float *v, half_t *y, int L, int M, int H) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (long long)M * H) return;
@@ -482,11 +487,12 @@ __global__ void bcast_add_silu_kernel(const float *x, const float *v, half_t *y,
     const float a = x[i] + v[(long long)(m / L) * H + c];
     const float s = a / (1.0f + __expf(-a));
     const half_t hi = (half_t)s;
-    y[(long long)m * 2 * H + c] = hi;
-    y[(long long)m * 2 * H + H + c] = (half_t)(s - (float)hi);
+    half_t *o = y + (long long)m * 2 * H + pair_col(c);
+    o[0] = hi;
+    o[PAIR] = (half_t)(s - (float)hi);
 }
 
-// out [M][2K] f16 hi|lo of x[m][k] + pe[m % P][k] (pe may be null): the sync features plus their
+// out [M][2K] paired f16 of x[m][k] + pe[m % P][k] (pe may be null): the sync features plus their
 // 8-periodic positional embedding (src/dit.cpp:93-99), as the operand of the following conv
 __global__ void add_period_hilo_kernel(const float *x, const float *pe, int P, half_t *out, int M, int K) {
     const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -494,8 +500,9 @@ __global__ void add_period_hilo_kernel(const float *x, const float *pe, int P, h
     const int m = (int)(i / K), k = (int)(i - (long long)m * K);
     const float v = x[i] + (pe ? pe[(long long)(m % P) * K + k] : 0.0f);
     const half_t hi = (half_t)v;
-    out[(long long)m * 2 * K + k] = hi;
-    out[(long long)m * 2 * K + K + k] = (half_t)(v - (float)hi);
+    half_t *o = out + (long long)m * 2 * K + pair_col(k);
+    o[0] = hi;
+    o[PAIR] = (half_t)(v - (float)hi);
 }
 
 // dst[i] = src[idx[i]], rows of H floats
@@ -885,14 +892,14 @@ int launch_eval_prep(const EvalPrepArgs &a, hipStream_t st) {
 }
 
 int launch_split_hilo(const float *x, int ldx, RowMap xmap, half_t *out, int M, int K, hipStream_t st) {
-    TSN_REQUIRE(x && out && M > 0 && K > 0 && xmap.L > 0, "split_hilo: arguments");
+    TSN_REQUIRE(x && out && M > 0 && K > 0 && K % PAIR == 0 && xmap.L > 0, "split_hilo: arguments (K a multiple of 32)");
     TSN_LAUNCH(split_hilo_kernel, dim3(blocks_for((size_t)M * K)), dim3(256), 0, st, x, ldx, xmap, out, M, K);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
-int launch_dup_cols_bf16_to_f16(const uint16_t *src, half_t *dst, int N, int K, hipStream_t st) {
-    TSN_REQUIRE(src && dst && N > 0 && K > 0, "dup_cols: arguments");
-    TSN_LAUNCH(dup_cols_kernel, dim3(blocks_for((size_t)N * K)), dim3(256), 0, st, src, dst, N, K);
+int launch_dup_cols_bf16_to_f16(const uint16_t *src, half_t *dst, int N, int K, int g, hipStream_t st) {
+    TSN_REQUIRE(src && dst && N > 0 && K > 0 && g > 0 && K % g == 0, "dup_cols: arguments");
+    TSN_LAUNCH(dup_cols_kernel, dim3(blocks_for((size_t)N * K)), dim3(256), 0, st, src, dst, N, K, g);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
@@ -946,7 +953,7 @@ int launch_bcast_add_silu_f16(const float *x, const float *v, half_t *y, int L, 
     return TSN_OK;
 }
 int launch_add_period_hilo(const float *x, const float *pe, int P, half_t *out, int M, int K, hipStream_t st) {
-    TSN_REQUIRE(x && out && M > 0 && K > 0 && (!pe || P > 0), "add_period_hilo: arguments");
+    TSN_REQUIRE(x && out && M > 0 && K > 0 && K % PAIR == 0 && (!pe || P > 0), "add_period_hilo: arguments (K a multiple of 32)");
     TSN_LAUNCH(add_period_hilo_kernel, dim3(blocks_for((size_t)M * K)), dim3(256), 0, st, x, pe, P, out, M, K);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;

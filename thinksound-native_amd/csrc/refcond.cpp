@@ -205,7 +205,7 @@ int RefCondModel::proj_silu(int rows, int K, int taps, const half_t *W, const fl
     g.nprob = 1;
     store_problem(g.p[0], IN_, 2 * K, RowMap{rows, rows, 0}, taps, 2 * K, rows, s.H, W, XA_, 2 * s.H, 1);
     g.p[0].bias = b;
-    g.p[0].y_lo = s.H;
+    g.p[0].y_pair = 1;
     half_w(g.p[0]);
     g.ws = ws_;
     g.ws_bytes = ws_bytes_;
@@ -218,7 +218,7 @@ int RefCondModel::swiglu_mlp(int rows, int taps, const half_t *W13, const half_t
     GemmBatch a;
     a.nprob = 1;
     store_problem(a.p[0], XA_, 2 * s.H, D, taps, 2 * s.H, rows, 2 * s.F, W13, HF_, 2 * s.F, 0);
-    a.p[0].y_lo = s.F;
+    a.p[0].y_pair = 1;
     half_w(a.p[0]);
     a.ws = ws_;
     a.ws_bytes = ws_bytes_;

@@ -438,7 +438,7 @@ int RefDitModel::block_joint(int i, bool ln1, Next next) {
     AttnArgs at;
     memset(&at, 0, sizeof at);
     at.Q = Q_; at.K = K_; at.Vt = Vt_; at.S = S; at.Sp = Sp; at.nh = s.NH; at.BH = B * s.NH;
-    at.O = AO_; at.o_f32 = 0; at.ldo = 2 * H; at.o_lo = H; at.omap = rowmap_dense(B * S);
+    at.O = AO_; at.o_f32 = 0; at.ldo = 2 * H; at.o_pair = s.T; at.omap = rowmap_dense(B * S);
     TSN_TRY(run(K_ATTN, 4.0 * B * s.NH * (double)S * S * 64, 8.0 * B * (double)S * H,
                 [&] { return launch_attention(at, st); }));
 
@@ -467,7 +467,7 @@ int RefDitModel::block_joint(int i, bool ln1, Next next) {
         const RowMap m = stream_map(kinds[k]);
         store_problem(f1.p[k], XN_, 2 * H, m, w[k]->taps, w[k]->hl ? 2 * H : H, B * m.L, 2 * s.F, w[k]->W13, HF_,
                       2 * s.F, 0);
-        f1.p[k].y_lo = w[k]->hl ? s.F : 0;
+        f1.p[k].y_pair = w[k]->hl;
         if (w[k]->hl) half_w(f1.p[k]);
     }
     f1.ws = ws_;
@@ -518,7 +518,7 @@ int RefDitModel::block_fused(int i, bool ln1, Next next) {
     AttnArgs at;
     memset(&at, 0, sizeof at);
     at.Q = Q_; at.K = K_; at.Vt = VtF_; at.S = T; at.Sp = SpF; at.nh = s.NH; at.BH = B * s.NH;
-    at.O = AO_; at.o_f32 = 0; at.ldo = 2 * H; at.o_lo = H; at.omap = Lm;
+    at.O = AO_; at.o_f32 = 0; at.ldo = 2 * H; at.o_pair = T; at.omap = Lm;
     TSN_TRY(run(K_ATTN, 4.0 * B * s.NH * (double)T * T * 64, 8.0 * B * (double)T * H,
                 [&] { return launch_attention(at, st); }));
 
@@ -537,7 +537,7 @@ int RefDitModel::block_fused(int i, bool ln1, Next next) {
     GemmBatch f1;
     f1.nprob = 1;
     store_problem(f1.p[0], XN_, 2 * H, Lm, w.taps, 2 * H, M, 2 * s.F, w.W13, HF_, 2 * s.F, 0);
-    f1.p[0].y_lo = s.F;
+    f1.p[0].y_pair = 1;
     half_w(f1.p[0]);
     f1.ws = ws_;
     f1.ws_bytes = ws_bytes_;
@@ -644,7 +644,7 @@ int RefDitModel::enqueue_eval(const float *x, const float *t, const float *clip_
         ib.nprob = 1;
         store_problem(ib.p[0], Z2_, 2 * L, D, 3, 2 * L, B * T, H, Win_, XN_, 2 * H, 1);
         ib.p[0].bias = bin_;
-        ib.p[0].y_lo = H;
+        ib.p[0].y_pair = 1;
         half_w(ib.p[0]);
         ib.ws = ws_;
         ib.ws_bytes = ws_bytes_;
@@ -652,7 +652,7 @@ int RefDitModel::enqueue_eval(const float *x, const float *t, const float *clip_
         GemmBatch sb;
         sb.nprob = 1;
         store_problem(sb.p[0], XN_, 2 * H, D, 3, 2 * H, B * T, 2 * s.F, W13in_, HF_, 2 * s.F, 0);
-        sb.p[0].y_lo = s.F;
+        sb.p[0].y_pair = 1;
         half_w(sb.p[0]);
         sb.ws = ws_;
         sb.ws_bytes = ws_bytes_;
