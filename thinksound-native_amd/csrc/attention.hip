@@ -460,11 +460,15 @@ __global__ __launch_bounds__(512, NSTG == 2 ? 2 : 1) void flash_attn_kernel(cons
                 const bool pair = q < a.o_pair;   // paired row: head h's 64 columns are 128 halves
                 half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
                 const float y0 = od[0] * inv, y1 = od[1] * inv, y2 = od[2] * inv, y3 = od[3] * inv;
-                const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-                *(half4 *)op = hi;
-                if (pair)   // the f16 remainder: hi + lo carries the f32 value
-                    *(half4 *)(op + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
-                                                    (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
+                if (pair) {   // the f16 remainder: hi + lo carries the f32 value
+                    const float y4[4] = {y0, y1, y2, y3};
+                    half4 hi, lo;
+                    split_parts4(y4, hi, lo);
+                    *(half4 *)op = hi;
+                    *(half4 *)(op + PAIR) = lo;
+                } else {
+                    *(half4 *)op = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
+                }
             }
         }
     }
@@ -613,11 +617,15 @@ __global__ __launch_bounds__(256, 3) void flash_attn4_kernel(const AttnArgs a) {
                 const bool pair = q < a.o_pair;
                 half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
                 const float y0 = o[dt][0] * inv, y1 = o[dt][1] * inv, y2 = o[dt][2] * inv, y3 = o[dt][3] * inv;
-                const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-                *(half4 *)op = hi;
-                if (pair)
-                    *(half4 *)(op + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
-                                                    (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
+                if (pair) {
+                    const float y4[4] = {y0, y1, y2, y3};
+                    half4 hi, lo;
+                    split_parts4(y4, hi, lo);
+                    *(half4 *)op = hi;
+                    *(half4 *)(op + PAIR) = lo;
+                } else {
+                    *(half4 *)op = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
+                }
             }
         }
     }
@@ -775,11 +783,15 @@ __global__ __launch_bounds__(256, 3) void flash_attn4q2_kernel(const AttnArgs a)
                 const bool pair = q[u] < a.o_pair;
                 half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
                 const float y0 = o[u][dt][0] * inv, y1 = o[u][dt][1] * inv, y2 = o[u][dt][2] * inv, y3 = o[u][dt][3] * inv;
-                const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-                *(half4 *)op = hi;
-                if (pair)
-                    *(half4 *)(op + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
-                                                    (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
+                if (pair) {
+                    const float y4[4] = {y0, y1, y2, y3};
+                    half4 hi, lo;
+                    split_parts4(y4, hi, lo);
+                    *(half4 *)op = hi;
+                    *(half4 *)(op + PAIR) = lo;
+                } else {
+                    *(half4 *)op = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
+                }
             }
         }
     }

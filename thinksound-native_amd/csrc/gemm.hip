@@ -488,16 +488,15 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
                 for (int e = 0; e < 8; ++e) v[e] = silu_f(v[e]);
             const long long o = rowmap_phys(P.ymap, m) * (long long)P.ldy + n;
             if (P.y_f16) {
-                half8 hi;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) hi[e] = (half_t)v[e];
                 half_t *y = (half_t *)P.Y + o;
+                half8 hi, lo;
                 if (P.y_pair) {
-                    half8 lo;
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) lo[e] = (half_t)(v[e] - (float)hi[e]);
+                    split_parts8(v, hi, lo);
                     y += pair_col(n) - n;
                     *(half8 *)(y + PAIR) = lo;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) hi[e] = (half_t)v[e];
                 }
                 *(half8 *)y = hi;
             } else {
@@ -517,21 +516,19 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
             ldsum8<T2>(tile, row * PITCH + col, a);
             ldsum8<T2>(tile, row * PITCH + 64 + col, b);
             float y[8];
-            half8 o;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                y[e] = silu_f(a[e]) * b[e];
-                o[e] = (half_t)y[e];
-            }
+            for (int e = 0; e < 8; ++e) y[e] = silu_f(a[e]) * b[e];
             const int n = n0 / 2 + col;
             half_t *dst = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + (P.y_pair ? pair_col(n) : n);
-            *(half8 *)dst = o;
+            half8 hi, lo;
             if (P.y_pair) {
-                half8 lo;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) lo[e] = (half_t)(y[e] - (float)o[e]);
+                split_parts8(y, hi, lo);
                 *(half8 *)(dst + PAIR) = lo;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) hi[e] = (half_t)y[e];
             }
+            *(half8 *)dst = hi;
         }
     } else if constexpr (EPI == EPI_SNAKE) {
         // the thread's 8 columns are the same in every pass: bias and snake table loaded once, before
@@ -556,11 +553,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
                 for (int e = 0; e < 8; ++e) v[e] += bv[e];
             snake8(v, ea, eb);
             half8 hi, lo;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                hi[e] = (half_t)v[e];
-                lo[e] = (half_t)(v[e] - (float)hi[e]);
-            }
+            split_parts8(v, hi, lo);
             half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
             *(half8 *)y = hi;
             *(half8 *)(y + PAIR) = lo;
@@ -601,11 +594,7 @@ __device__ __forceinline__ void tile_epilogue(const GemmProblem &P, const float 
             if (!P.Y) continue;
             snake8(v, ea, eb);
             half8 hi, lo;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                hi[e] = (half_t)v[e];
-                lo[e] = (half_t)(v[e] - (float)hi[e]);
-            }
+            split_parts8(v, hi, lo);
             half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
             *(half8 *)y = hi;
             *(half8 *)(y + PAIR) = lo;
@@ -1873,11 +1862,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmBatch bt) 
         float e[4] = {v.x, v.y, v.z, v.w};
         half4 hi, lo;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            e[j] = e[j] + snake_sin2(e[j] * P.snake[n + j]) * P.snake[P.N + n + j];
-            hi[j] = (half_t)e[j];
-            lo[j] = (half_t)(e[j] - (float)hi[j]);
-        }
+        for (int j = 0; j < 4; ++j) e[j] = e[j] + snake_sin2(e[j] * P.snake[n + j]) * P.snake[P.N + n + j];
+        split_parts4(e, hi, lo);
         half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
         *(half4 *)y = hi;
         *(half4 *)(y + PAIR) = lo;
@@ -1892,11 +1878,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmBatch bt) 
         float e[4] = {v.x, v.y, v.z, v.w};
         half4 hi, lo;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            e[j] = e[j] + snake_sin2(e[j] * P.snake[n + j]) * P.snake[P.N + n + j];
-            hi[j] = (half_t)e[j];
-            lo[j] = (half_t)(e[j] - (float)hi[j]);
-        }
+        for (int j = 0; j < 4; ++j) e[j] = e[j] + snake_sin2(e[j] * P.snake[n + j]) * P.snake[P.N + n + j];
+        split_parts4(e, hi, lo);
         half_t *y = (half_t *)P.Y + rowmap_phys(P.ymap, m) * (long long)P.ldy + pair_col(n);
         *(half4 *)y = hi;
         *(half4 *)(y + PAIR) = lo;

@@ -11,6 +11,34 @@ namespace tsn {
 // hi part is at pair_col(c), its lo part PAIR further.
 constexpr int PAIR = 32;
 __host__ __device__ inline int pair_col(int c) { return c + (c & ~(PAIR - 1)); }
+// The parts of v: hi = f16(v), lo = f16(v - hi). v passes through an empty asm statement, so hi is the
+// f16 rounding of the f32 value itself. Without it the compiler rounds hi straight from the
+// product or sum that makes v (v_fma_mixlo_f16) and subtracts another rounding; where the two straddle
+// an f16 tie, hi + lo is off by a whole f16 ulp of v (about one value in 10^4 of a SwiGLU output,
+// and most of the error of the f32-accurate GEMM chains).
+__device__ __forceinline__ void split_parts(float v, half_t &hi, half_t &lo) {
+    asm volatile("" : "+v"(v));
+    hi = (half_t)v;
+    lo = (half_t)(v - (float)hi);
+}
+__device__ __forceinline__ void split_parts8(const float (&v)[8], half8 &hi, half8 &lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        half_t h, l;
+        split_parts(v[e], h, l);
+        hi[e] = h;
+        lo[e] = l;
+    }
+}
+__device__ __forceinline__ void split_parts4(const float (&v)[4], half4 &hi, half4 &lo) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        half_t h, l;
+        split_parts(v[e], h, l);
+        hi[e] = h;
+        lo[e] = l;
+    }
+}
 
 /* ------------------------------------------------------------------ GEMM (MFMA) */
 // C[M,N] = A[M,K] · W[N,K]ᵀ with f16 operands and f32 accumulation; 128x128x64 tiles,

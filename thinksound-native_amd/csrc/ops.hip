@@ -72,9 +72,9 @@ __global__ __launch_bounds__(256) void ln_mod_kernel(const LnArgs a) {
         if constexpr (YMODE == LN_F16) {
             *(half4 *)((half_t *)S.Y + yrow + col) = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
         } else if constexpr (YMODE == LN_F16_HILO) {
-            const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-            const half4 lo = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
-                                   (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
+            const float y4[4] = {y0, y1, y2, y3};
+            half4 hi, lo;
+            split_parts4(y4, hi, lo);
             half_t *y = (half_t *)S.Y + yrow + pair_col(col);
             *(half4 *)y = hi;
             *(half4 *)(y + PAIR) = lo;
@@ -147,11 +147,15 @@ __global__ __launch_bounds__(512) void reduce_ln_kernel(const RedLnArgs a) {
     const float y3 = d3 * inv * (1.0f + scl.w) + sh.w;
     const bool pair = YMODE == LN_F16_HILO || S.hilo;   // uniform over the workgroup
     half_t *y = (half_t *)S.Y + rowmap_phys(S.ymap, v) * (long long)S.ldy + (pair ? pair_col(col) : col);
-    const half4 hi = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-    *(half4 *)y = hi;
-    if (pair)
-        *(half4 *)(y + PAIR) = half4{(half_t)(y0 - (float)hi[0]), (half_t)(y1 - (float)hi[1]),
-                                     (half_t)(y2 - (float)hi[2]), (half_t)(y3 - (float)hi[3])};
+    if (pair) {
+        const float y4[4] = {y0, y1, y2, y3};
+        half4 hi, lo;
+        split_parts4(y4, hi, lo);
+        *(half4 *)y = hi;
+        *(half4 *)(y + PAIR) = lo;
+    } else {
+        *(half4 *)y = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
+    }
 }
 
 /* ---------------- calibration probes (achievable MFMA and HBM rates) ---------------- */
@@ -371,10 +375,8 @@ __device__ __forceinline__ void split_hilo_elem(const float *x, int ldx, RowMap 
     if (i >= (long long)M * K) return;
     const int m = (int)(i / K), k = (int)(i - (long long)m * K);
     const float v = x[rowmap_phys(xmap, m) * (long long)ldx + k];
-    const half_t hi = (half_t)v;
     half_t *o = out + (long long)m * 2 * K + k + k / g * g;
-    o[0] = hi;
-    o[g] = (half_t)(v - (float)hi);
+    split_parts(v, o[0], o[g]);
 }
 __global__ void split_hilo_kernel(const float *x, int ldx, RowMap xmap, half_t *out, int M, int K) {
     split_hilo_elem(x, ldx, xmap, out, M, K, PAIR, (long long)blockIdx.x * blockDim.x + threadIdx.x);
@@ -486,10 +488,8 @@ __global__ void bcast_add_silu_kernel(const float *x, const float *v, half_t *y,
     const int m = (int)(i / H), c = (int)(i - (long long)m * H);
     const float a = x[i] + v[(long long)(m / L) * H + c];
     const float s = a / (1.0f + __expf(-a));
-    const half_t hi = (half_t)s;
     half_t *o = y + (long long)m * 2 * H + pair_col(c);
-    o[0] = hi;
-    o[PAIR] = (half_t)(s - (float)hi);
+    split_parts(s, o[0], o[PAIR]);
 }
 
 // out [M][2K] paired f16 of x[m][k] + pe[m % P][k] (pe may be null): the sync features plus their
@@ -499,10 +499,8 @@ __global__ void add_period_hilo_kernel(const float *x, const float *pe, int P, h
     if (i >= (long long)M * K) return;
     const int m = (int)(i / K), k = (int)(i - (long long)m * K);
     const float v = x[i] + (pe ? pe[(long long)(m % P) * K + k] : 0.0f);
-    const half_t hi = (half_t)v;
     half_t *o = out + (long long)m * 2 * K + pair_col(k);
-    o[0] = hi;
-    o[PAIR] = (half_t)(v - (float)hi);
+    split_parts(v, o[0], o[PAIR]);
 }
 
 // dst[i] = src[idx[i]], rows of H floats

@@ -24,11 +24,7 @@ __global__ void split_kernel(const float *__restrict__ x, long long rows, int C,
     const float4 x0 = *(const float4 *)xp, x1 = *(const float4 *)(xp + 4);
     const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
     half8 hi, lo;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        hi[e] = (half_t)v[e];
-        lo[e] = (half_t)(v[e] - (float)hi[e]);
-    }
+    split_parts8(v, hi, lo);
     if constexpr (THREE) {
         half_t *o = out + r * 3 * C + c;
         *(half8 *)o = hi;
