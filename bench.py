@@ -805,7 +805,7 @@ def bench_encoders(tsn, rt, args):
         flops = sum(k["flops"] for k in stats)
         wbytes = 4.0 * (int(lib_total(tsn, name, spec)))
         ms = statistics.median(ts)
-        gemm = [k for k in stats if k["name"] == "gemm_f32_kernel"][0]
+        gemm = [k for k in stats if k["name"] == "enc_gemm_kernel"][0]
         for k in sorted(stats, key=lambda k: -k["ms"]):
             log("  %s %-24s %4d launches %8.3f ms" % (name, k["name"], k["launches"], k["ms"]))
         log("bench %s: %.3f ms per prompt, %.1f GFLOP, gemm_f32 %.3f ms (%d launches, %.1f TFLOP/s)"

@@ -142,3 +142,40 @@ def test_encoders_gguf_load(tsn, rt, tmp_path):
     finally:
         for m in models:
             m.close()
+
+
+@pytest.mark.parametrize("ctx", [1, 16, 17, 32, 33, 80, 81, 128])
+@pytest.mark.parametrize("scale", [1.0, 3e4])
+def test_encoder_gemm_edges(tsn, rt, orc, ctx, scale):
+    """Row-block edges of the GEMMs (16-row MFMA blocks, the 32-, 80- and 128-row tiles), a K that ends half
+    way through a 64-column step (d_ff = 96, 352) and, with scale, T5 FFN activations of about scale^2
+    (past the f16 range) and rows of one weight 2^-20 of the others. f32 against f32: three layers
+    amplify a rounding-level difference (6e-8) by less than 50."""
+    ts = tsn.t5_spec_default().copy(d=192, d_ff=352 if ctx % 2 else 96, NL=3, NH=3, ctx=ctx, vocab=200)
+    cs = tsn.clip_spec_default().copy(H=192, NL=3, NH=3, ctx=ctx, vocab=300)
+    tw, cw = tsn.t5_synth_weights(ts, 31).copy(), tsn.clip_synth_weights(cs, 32).copy()
+    for name, n, off in tsn.t5_manifest(ts):
+        if name.endswith((".wi_0", ".wi_1")):
+            tw[off:off + n] *= scale
+        elif name.endswith(".wo"):
+            tw[off:off + n] /= scale * scale
+        elif name.endswith(".k") and scale != 1.0:
+            tw[off:off + 64 * ts.d] *= 2.0 ** -20
+    r = rng(ctx)
+    tids, cids = r.integers(2, 200, ctx).astype(np.int32), r.integers(0, 300, ctx).astype(np.int32)
+    tids[ctx // 2 + 1:] = 0
+    t, c = tsn.T5Model(rt, ts), tsn.ClipModel(rt, cs)
+    try:
+        t.upload_weights(tw)
+        c.upload_weights(cw)
+        out, pt, g = rt.empty((ctx, ts.d)), rt.empty((ctx, cs.H)), rt.empty((cs.H,))
+        t.encode(tids, out)
+        c.encode(cids, pt, g)
+        rt.sync()
+        rpt, rg = orc.clip_encode(cs.as_dict(), cw, cids)
+        e = (rel_l2(out.numpy(), orc.t5_encode(ts.as_dict(), tw, tids)), rel_l2(pt.numpy(), rpt), rel_l2(g.numpy(), rg))
+        print("ctx %d scale %g: t5 %.3g clip %.3g pooled %.3g" % ((ctx, scale) + e))
+        assert max(e) <= 3e-6
+    finally:
+        t.close()
+        c.close()

@@ -1,8 +1,17 @@
-// enc.hip — kernels of the text encoders (src/clip.cpp, src/t5.cpp): f32 GEMM on the f32 MFMA,
-// LayerNorm with weight and bias, RMSNorm with weight, attention over one short context with the
-// CLIP causal/EOT mask or the T5 bucketed relative bias and padding mask, GEGLU, and the token
-// (+ position) embedding gather. Everything stays f32: T5's activations leave the f16 range.
+// enc.hip — kernels of the text encoders (src/clip.cpp, src/t5.cpp): f32-accurate GEMM over streamed f32
+// weights, LayerNorm with weight and bias, RMSNorm with weight, attention over one short context with the
+// CLIP causal/EOT mask or the T5 bucketed relative bias and padding mask, quick GELU / GEGLU, and the
+// token (+ position) embedding gather. GEMM operands are pairs of f16 parts (hi + lo) of values scaled by
+// a power of two, per row of activations and per row of a weight, because T5's activations leave the
+// f16 range; everything else is f32.
+//
+// Per layer: norm -> QKV GEMM -> attention -> out GEMM -> norm -> FFN GEMM -> activation -> FFN GEMM.
+// A GEMM leaves the raw sums of its K splits in the workspace; the kernel that reads them adds the
+// splits in order with the bias (and the residual), so no GEMM has a reduce launch of its own, and
+// writes its result as the next GEMM's operand (pack_parts4).
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "kernels.h"
 #include "dpp.h"
@@ -12,136 +21,237 @@ namespace tsn {
 namespace {
 
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef unsigned uintx4_t __attribute__((ext_vector_type(4)));
 
-constexpr int FB_MT = 5;                 // 16-row MFMA blocks per tile: 80 rows hold a 77-token prompt
-constexpr int FB_M = 16 * FB_MT, FB_N = 64, FB_K = 64, FB_LD = FB_K + 1;
+// 2^(e - 14) for 2^e <= v < 2^(e + 1): a row of largest magnitude v divided by it lies below 2^15, and
+// parts of its values down to 2^-16 of the largest are exact to 22 bits (smaller ones to 2^-39 of the
+// largest). Zero and denormal rows take the smallest exponent that keeps the divisor's reciprocal finite.
+__device__ __forceinline__ float row_divisor(float v) {
+    return __uint_as_float((max(__float_as_uint(v) >> 23, 32u) - 14u) << 23);
+}
+__device__ __forceinline__ float pow2_recip(float v) { return __uint_as_float((254u << 23) - __float_as_uint(v)); }
 
-// The epilogue of one output element: v = sum + bias, then Y = act(v) or Y += v.
-__device__ __forceinline__ void enc_epi(const EncGemmArgs &g, int m, int n, float v) {
-    if (g.bias) v += g.bias[n];
-    float *y = g.Y + (long long)m * g.ldy + n;
-    if (g.resid) {
-        *y = *y + v;
-    } else {
-        if (g.act == 1) v = v / (1.0f + expf(-1.702f * v));   // quick GELU (shaders/ops_conv.metal:25-29)
-        *y = v;
+// A GEMM operand with M <= 16 mt rows, packed for enc_gemm_kernel: per 32-wide K step the hi and the lo
+// parts one after the other, each mt blocks of 16 rows x 32 columns (1 KB). A block is the 64 16-byte
+// operands of one MFMA: row r (0..15), columns 8 kq .. + 7 (kq 0..3) at slot 4 r + (kq ^ (r / 2 % 4)).
+// The slots of one row are 64 contiguous bytes (producers write one row), and the xor makes the reads of
+// 8 lanes cover 128 contiguous bytes.
+__device__ __forceinline__ int pack_slot(int r, int kq) { return 4 * r + (kq ^ ((r >> 1) & 3)); }
+// columns k .. k + 3 (k % 4 == 0) of row m
+__device__ __forceinline__ void pack_parts4(half_t *Ap, int mt, int m, int k, const float (&v)[4]) {
+    half4 hi, lo;
+    split_parts4(v, hi, lo);
+    half_t *d = Ap + (((long long)(k >> 5) * 2 * mt + (m >> 4)) * 64 + pack_slot(m & 15, (k & 31) >> 3)) * 8 + (k & 4);
+    *(half4 *)d = hi;
+    *(half4 *)(d + mt * 512) = lo;
+}
+
+__device__ __forceinline__ float4 add4(float4 a, float4 b) {
+    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+__device__ __forceinline__ float max4(float4 v) {   // largest magnitude
+    return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
+}
+// v[i] = the sum over the splits, in order, of the 4 columns at element off[i] of a GEMM's result. B splits
+// are loaded at a time (past the last one, that one again, not added), so a reader waits for memory
+// splits / B times, not once per split: these kernels are latency-bound.
+template <int NV, int B>
+__device__ __forceinline__ void parts_sum(const EncParts &p, const int (&off)[NV], float4 (&v)[NV]) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int z = 0; z < p.splits; z += B) {
+        float4 t[B][NV];
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const float *s = p.ws + min(z + b, p.splits - 1) * p.stride;
+#pragma unroll
+            for (int i = 0; i < NV; ++i) t[b][i] = *(const float4 *)(s + off[i]);
+        }
+#pragma unroll
+        for (int b = 0; b < B; ++b)
+            if (z + b < p.splits) {
+#pragma unroll
+                for (int i = 0; i < NV; ++i) v[i] = add4(v[i], t[b][i]);
+            }
     }
 }
 
-// 4 waves; wave w owns columns 16w..16w+15 of an 80x64 tile (five 16x16 blocks of
-// v_mfma_f32_16x16x4_f32 per 4-wide K slice). With 80 rows a whole prompt is one row tile, so each
-// weight is read from HBM once. A and W reach LDS in 64-wide K stages; the next stage is loaded into
-// registers while the current one is multiplied. blockIdx.z = split: K tiles [z*kps, (z+1)*kps);
-// with more than one split the raw sums go to ws[z][M][N] and enc_gemm_reduce_kernel adds them in
-// split order.
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const EncGemmArgs g) {
-    __shared__ float As[2][FB_M * FB_LD];
-    __shared__ float Ws[2][FB_N * FB_LD];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n0 = blockIdx.x * FB_N, m0 = blockIdx.y * FB_M, z = blockIdx.z;
-    const int M = g.M, N = g.N, K = g.K;
-    const int nkt = (K + FB_K - 1) / FB_K;
-    const int kt0 = z * g.kps, kt1 = min(nkt, kt0 + g.kps);
-    // loader: 16 lanes per 64-wide row (4 floats each); A rows lr + 16i (i < 5), W rows lr + 16i (i < 4).
-    // Two register sets: K tile kt + 2 is fetched while kt is multiplied and kt + 1 waits in the
-    // other set, so a tile has two K steps of MFMA work to arrive from HBM.
-    const int lr = tid >> 4, lc = (tid & 15) * 4;
-    float4 ra0[FB_MT], rw0[4], ra1[FB_MT], rw1[4];
-    auto fetch = [&](int kt, float4 (&ra)[FB_MT], float4 (&rw)[4]) {
-        const int k = kt * FB_K + lc;
-        const bool kin = k < K;
-        const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-        for (int i = 0; i < FB_MT; ++i) {
-            const int m = m0 + lr + 16 * i;
-            ra[i] = (kin && m < M) ? *(const float4 *)(g.A + (long long)m * g.lda + k) : z4;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int n = n0 + lr + 16 * i;
-            rw[i] = (kin && n < N) ? *(const float4 *)(g.W + (long long)n * g.ldw + k) : z4;
-        }
-    };
-    auto stash = [&](int b, const float4 (&ra)[FB_MT], const float4 (&rw)[4]) {
-#pragma unroll
-        for (int i = 0; i < FB_MT; ++i) {
-            float *a = &As[b][(lr + 16 * i) * FB_LD + lc];
-            a[0] = ra[i].x; a[1] = ra[i].y; a[2] = ra[i].z; a[3] = ra[i].w;
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float *w = &Ws[b][(lr + 16 * i) * FB_LD + lc];
-            w[0] = rw[i].x; w[1] = rw[i].y; w[2] = rw[i].z; w[3] = rw[i].w;
-        }
-    };
-    floatx4_t acc[FB_MT];
-#pragma unroll
-    for (int i = 0; i < FB_MT; ++i) acc[i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    const int r16 = lane & 15, kq = lane >> 4;   // operand lane: row / column r16, k offset kq
-    auto compute = [&](int b) {
-        const float *as = As[b], *ws = Ws[b];
-#pragma unroll
-        for (int kk = 0; kk < FB_K; kk += 4) {
-            const float bv = ws[(wave * 16 + r16) * FB_LD + kk + kq];
-#pragma unroll
-            for (int i = 0; i < FB_MT; ++i)
-                acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(as[(16 * i + r16) * FB_LD + kk + kq], bv, acc[i], 0, 0, 0);
-        }
-    };
-    // K tile kt0 + r lives in LDS buffer r & 1 and, before that, in register set r & 1
-    if (kt0 < kt1) {
-        fetch(kt0, ra0, rw0);
-        stash(0, ra0, rw0);
-        if (kt0 + 1 < kt1) fetch(kt0 + 1, ra1, rw1);
-        __syncthreads();
-        for (int kt = kt0; kt < kt1; kt += 2) {
-            // even step: tile kt in buffer 0; set 0 is free, set 1 holds kt + 1
-            if (kt + 2 < kt1) fetch(kt + 2, ra0, rw0);
-            compute(0);
-            if (kt + 1 >= kt1) break;
-            stash(1, ra1, rw1);
-            __syncthreads();
-            // odd step: tile kt + 1 in buffer 1; set 1 is free, set 0 holds kt + 2
-            if (kt + 3 < kt1) fetch(kt + 3, ra1, rw1);
-            compute(1);
-            if (kt + 2 >= kt1) break;
-            stash(0, ra0, rw0);
-            __syncthreads();
-        }
-    }
-    // lane holds rows 16i + 4*(lane/16) + r, column lane%16 of the wave's 16 columns
-    const int n = n0 + wave * 16 + r16;
-    if (n >= N) return;
-#pragma unroll
-    for (int i = 0; i < FB_MT; ++i)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int m = m0 + 16 * i + 4 * kq + r;
-            if (m >= M) continue;
-            if (g.splits > 1) g.ws[((long long)z * M + m) * N + n] = acc[i][r];
-            else enc_epi(g, m, n, acc[i][r]);
-        }
-}
-
-// split-K finish: sum the partials in split order, then the epilogue
-__global__ void enc_gemm_reduce_kernel(const EncGemmArgs g) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)g.M * g.N) return;
-    const int m = (int)(i / g.N), n = (int)(i - (long long)m * g.N);
-    float v = 0.0f;
-    for (int z = 0; z < g.splits; ++z) v += g.ws[(long long)z * g.M * g.N + i];
-    enc_epi(g, m, n, v);
-}
-
-// one 256-thread workgroup per row: LayerNorm (w, b; mean then variance of the centred row) or
-// RMSNorm (w); sums reduced per wave, then across the 4 waves in wave order through LDS
-template <bool LN>
-__global__ __launch_bounds__(256) void enc_norm_kernel(const float *__restrict__ x, float *__restrict__ y,
-                                                       const float *__restrict__ w, const float *__restrict__ b,
-                                                       int rows, int H, float eps) {
+// div[n] = row_divisor of the largest magnitude of row n
+__global__ __launch_bounds__(256) void enc_weight_scale_kernel(const float *__restrict__ src, float *__restrict__ div, int K) {
     __shared__ float part[4];
-    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const float *xr = x + (long long)row * H;
+    const int n = blockIdx.x, tid = threadIdx.x;
+    float mx = 0.0f;
+    for (int k = tid * 4; k < K; k += 1024) {
+        const float4 v = *(const float4 *)(src + (long long)n * K + k);
+        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    }
+    mx = wave_max(mx);
+    if ((tid & 63) == 0) part[tid >> 6] = mx;
+    __syncthreads();
+    if (tid == 0) div[n] = row_divisor(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
+}
+
+// Weights in the order the GEMM reads them, 4 bytes each: blocks of 64 rows (output columns) x 64 columns
+// of K, 16 KB each, K innermost. Inside a block, each of 4 waves has 4 KB (32 rows, 32 columns) as its
+// four 1 KB loads: rows 16 j .. + 15, part p (hi, lo), lane: row lane % 16, columns 8 (lane / 16) .. + 7.
+// Row-major weights took 8% more time: rows of 4 or 8 KB put the 64 rows that a workgroup touches at
+// once on a few memory channels.
+__global__ __launch_bounds__(256) void enc_weight_pack_kernel(const float *__restrict__ src, const float *__restrict__ div,
+                                                              half_t *__restrict__ dst, int K) {
+    const int s = blockIdx.x, t = blockIdx.y, nkt = gridDim.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    half_t *d = dst + (((long long)t * nkt + s) * 4 + wave) * 2048 + lane * 8;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int row = t * 64 + (wave & 1) * 32 + j * 16 + (lane & 15);
+        const int k = s * 64 + (wave >> 1) * 32 + (lane >> 4) * 8;
+        const float f = pow2_recip(div[row]);
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = k < K ? src[(long long)row * K + k + e] * f : 0.0f;
+        half8 hi, lo;
+        split_parts8(v, hi, lo);
+        *(half8 *)(d + j * 1024) = hi;
+        *(half8 *)(d + j * 1024 + 512) = lo;
+    }
+}
+
+// ws[z][M][N] = sums over K split z of A[M][K] W[N][K]^T, A and W packed, times adiv[m] wdiv[n].
+//
+// The bound is the weight stream: each weight is read once up to 80 rows (one tile holds them all; twice up to 128), so the
+// design keeps HBM loads in flight and everything else under them. Weights go straight from global
+// memory to the registers of the lane that multiplies them (no LDS), three steps ahead. Three
+// v_mfma_f32_16x16x32_f16 products (hi hi, hi lo, lo hi) replace eight f32 MFMAs of the same 32 columns
+// of K at 3/16 of their matrix-core time. The dropped lo lo is below 2^-22 of a product. The hi hi sums
+// and the others have accumulators of their own, added at the end, so the main sum rounds once
+// per 32 products instead of eight times. (Three bf16 parts a value, split from f32 weights in the
+// loop, need no scales, but six products and five vector instructions a weight, which this core does not
+// overlap with MFMAs of the same wave: 10240 x 2048 at 77 rows 27.6 us.)
+//
+// A step is 64 columns of K. 4 waves: wave w owns columns 32 (w & 1) .. + 31 of a 64-column tile and
+// K half w >> 1 of every step, and the two halves' sums are added through LDS at the end, so each
+// fragment of A read from LDS feeds two of W. A steps (4 KB per 16 rows) are shared by the waves through
+// two LDS buffers, loaded two steps ahead. Fetches past the split's end take its last step again, so
+// every wait in the loop has a fixed count of younger loads to leave in flight. (Eight waves with four
+// K ranges and half the K splits measured the same at 77 rows x 6144 x 2048 and 1.5 to 2 us a launch more
+// at a width of 1024; fragments read one step ahead of their products measured slower on both.)
+//
+// MTP: the operand's row blocks; with MTP > MT, blockIdx.z picks the MT of them that the workgroup takes.
+template <int MT, int MTP>
+__global__ __launch_bounds__(256, 2) void enc_gemm_kernel(const EncGemmArgs g) {
+    constexpr int CH = 2 * 2 * MT * 64, NA = CH / 256;   // 16-byte chunks of an A step, per thread
+    __shared__ __attribute__((aligned(16))) uintx4_t As[2][CH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, kq = lane >> 4, wn = wave & 1, kh = wave >> 1;
+    const int n0 = blockIdx.x * 64 + wn * 32, z = blockIdx.y, mb = MTP > MT ? blockIdx.z * MT : 0;
+    const int nkt = (g.K + 63) >> 6;
+    const int kt0 = z * g.kps, kt1 = min(nkt, kt0 + g.kps);
+    const half_t *wb = g.W + ((long long)blockIdx.x * nkt * 4 + wave) * 2048;   // wave-uniform
+    uintx4_t w[4][4], a[2][NA];
+    auto fetch_w = [&](int kt, uintx4_t (&d)[4]) {
+        const uintx4_t *p = (const uintx4_t *)(wb + (long long)min(kt, kt1 - 1) * 8192);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[q] = p[(unsigned)(q * 64 + lane)];
+    };
+    auto fetch_a = [&](int kt, uintx4_t (&d)[NA]) {
+        const uintx4_t *p = (const uintx4_t *)g.Ap + ((long long)min(kt, kt1 - 1) * 4 * MTP + mb) * 64;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int c = tid + 256 * i;
+            d[i] = p[(unsigned)(MTP > MT ? c / (64 * MT) * (64 * MTP) + c % (64 * MT) : c)];
+        }
+    };
+    auto stash_a = [&](int b, const uintx4_t (&d)[NA]) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) As[b][tid + 256 * i] = d[i];
+    };
+    floatx4_t acc[2][MT], low[2][MT];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < MT; ++i) acc[j][i] = low[j][i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int slot = kh * 2 * MT * 64 + pack_slot(r16, kq);
+    auto multiply = [&](int b, const uintx4_t (&o)[4]) {
+        half8 f[2][MT];
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) f[c][i] = __builtin_bit_cast(half8, As[b][(c * MT + i) * 64 + slot]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)   // A's hi with W's hi, hi with lo, lo with hi
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    floatx4_t &d = c == 0 ? acc[j][i] : low[j][i];
+                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, o[2 * j + (c == 1)]), f[c == 2][i], d, 0, 0, 0);
+                }
+    };
+    // Issue order A(kt + 2), W(kt + 3): when A(kt + 1) has to be in LDS, two weight steps and one A step
+    // issued after it are still in flight. LDS buffer (kt - kt0) & 1 holds A(kt); the other one was last
+    // read in step kt - 1, before the barrier that ended it.
+    fetch_a(kt0, a[0]);
+    fetch_w(kt0, w[0]);
+    fetch_w(kt0 + 1, w[1]);
+    fetch_a(kt0 + 1, a[1]);
+    fetch_w(kt0 + 2, w[2]);
+    stash_a(0, a[0]);
+    __syncthreads();
+    int kt = kt0;
+    for (; kt + 4 < kt1; kt += 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            fetch_a(kt + j + 2, a[j & 1]);
+            fetch_w(kt + j + 3, w[(j + 3) & 3]);
+            multiply(j & 1, w[j]);
+            stash_a((j + 1) & 1, a[(j + 1) & 1]);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {   // the last one to four steps
+        if (j < 2) fetch_a(kt + j + 2, a[j & 1]);
+        if (j < 1) fetch_w(kt + j + 3, w[3]);
+        multiply(j & 1, w[j]);
+        if (kt + j + 1 >= kt1) break;
+        stash_a((j + 1) & 1, a[(j + 1) & 1]);
+        __syncthreads();
+    }
+    // the weights are the first operand: a lane holds columns n0 + 16 j + 4 kq .. + 3 of row 16 i + r16
+    __syncthreads();
+    // 4 MT KB of the buffers' 8 MT
+    floatx4_t *sum = (floatx4_t *)&As[0][0] + wn * 2 * MT * 64 + lane;
+    if (kh > 0) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) sum[(j * MT + i) * 64] = acc[j][i] + low[j][i];
+    }
+    __syncthreads();
+    if (kh > 0) return;
+    floatx4_t wd[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wd[j] = *(const floatx4_t *)(g.wdiv + n0 + 16 * j + 4 * kq);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int m = 16 * (mb + i) + r16;
+        if (m >= g.M) continue;
+        const float ad = g.adiv[m];
+        float *y = g.ws + ((long long)z * g.M + m) * g.N + n0 + 4 * kq;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            *(floatx4_t *)(y + 16 * j) = ((acc[j][i] + low[j][i]) + sum[(j * MT + i) * 64]) * wd[j] * ad;
+    }
+}
+
+// One 256-thread workgroup per row: x += the previous GEMM's result (parts, if given; written back),
+// then LayerNorm (w, b; mean, then variance of the centred row) or RMSNorm (w) of x as f32 rows (y)
+// or as the next GEMM's operand (Ap). Sums are reduced per wave, then across the 4 waves in wave order.
+// NJ: 1024-column groups of a row (H <= 1024 NJ, H % 4 == 0).
+template <bool LN, int NJ>
+__global__ __launch_bounds__(256) void enc_norm_kernel(const EncNormArgs a) {
+    __shared__ float part[4];
+    const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, H = a.H;
     auto block_sum = [&](float v) {
         v = wave_sum(v);
         __syncthreads();   // part[] free from the previous reduction
@@ -149,232 +259,367 @@ __global__ __launch_bounds__(256) void enc_norm_kernel(const float *__restrict__
         __syncthreads();
         return ((part[0] + part[1]) + part[2]) + part[3];
     };
-    // the row in registers: columns 4*tid + 1024*j .. + 3 (H % 4 == 0, H <= 2048)
-    float4 v[2];
+    auto block_max = [&](float v) {
+        v = wave_max(v);
+        __syncthreads();
+        if (lane == 0) part[wave] = v;
+        __syncthreads();
+        return fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
+    };
+    // the row in registers: columns 4*tid + 1024*j .. + 3; all loads ahead of the first barrier
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 v[NJ], wv[NJ], bv[NJ];
+    int off[NJ];
+    bool in[NJ];
     float s = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int j = 0; j < NJ; ++j) {
         const int c = 4 * tid + 1024 * j;
-        v[j] = c < H ? *(const float4 *)(xr + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+        in[j] = c < H;
+        off[j] = row * H + (in[j] ? c : 0);
+        v[j] = in[j] ? *(const float4 *)(a.x + (long long)row * H + c) : zero;
+        wv[j] = in[j] ? *(const float4 *)(a.w + c) : zero;
+        bv[j] = LN && in[j] ? *(const float4 *)(a.b + c) : zero;
+    }
+    if (a.parts.ws) {
+        float4 t[NJ], pb[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            pb[j] = a.parts.bias && in[j] ? *(const float4 *)(a.parts.bias + 4 * tid + 1024 * j) : zero;
+        parts_sum<NJ, 8>(a.parts, off, t);
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            if (in[j]) {
+                v[j] = add4(v[j], add4(t[j], pb[j]));
+                *(float4 *)(a.xout + off[j]) = v[j];
+            }
+    }
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
         s += LN ? (v[j].x + v[j].y) + (v[j].z + v[j].w)
                 : (v[j].x * v[j].x + v[j].y * v[j].y) + (v[j].z * v[j].z + v[j].w * v[j].w);
-    }
     s = block_sum(s);
     float mean = 0.0f, inv;
     if (LN) {
         mean = s / (float)H;
         float q = 0.0f;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-            if (4 * tid + 1024 * j < H) {
+        for (int j = 0; j < NJ; ++j)
+            if (in[j]) {
                 const float d0 = v[j].x - mean, d1 = v[j].y - mean, d2 = v[j].z - mean, d3 = v[j].w - mean;
                 q += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
             }
         q = block_sum(q);
-        inv = 1.0f / sqrtf(q / (float)H + eps);
+        inv = 1.0f / sqrtf(q / (float)H + a.eps);
     } else {
-        inv = 1.0f / sqrtf(s / (float)H + eps);
+        inv = 1.0f / sqrtf(s / (float)H + a.eps);
     }
-    float *yr = y + (long long)row * H;
+    float4 o[NJ];
+    float mx = 0.0f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int c = 4 * tid + 1024 * j;
-        if (c >= H) continue;
-        const float4 wv = *(const float4 *)(w + c);
-        float4 o;
+    for (int j = 0; j < NJ; ++j) {   // columns past H: zero
         if (LN) {
-            const float4 bv = *(const float4 *)(b + c);
-            o = make_float4((v[j].x - mean) * inv * wv.x + bv.x, (v[j].y - mean) * inv * wv.y + bv.y,
-                            (v[j].z - mean) * inv * wv.z + bv.z, (v[j].w - mean) * inv * wv.w + bv.w);
+            o[j] = make_float4((v[j].x - mean) * inv * wv[j].x + bv[j].x, (v[j].y - mean) * inv * wv[j].y + bv[j].y,
+                               (v[j].z - mean) * inv * wv[j].z + bv[j].z, (v[j].w - mean) * inv * wv[j].w + bv[j].w);
         } else {
-            o = make_float4(v[j].x * inv * wv.x, v[j].y * inv * wv.y, v[j].z * inv * wv.z, v[j].w * inv * wv.w);
+            o[j] = make_float4(v[j].x * inv * wv[j].x, v[j].y * inv * wv[j].y, v[j].z * inv * wv[j].z, v[j].w * inv * wv[j].w);
         }
-        *(float4 *)(yr + c) = o;
+        mx = fmaxf(mx, max4(o[j]));
+    }
+    if (a.Ap) {
+        const float d = row_divisor(block_max(mx)), f = pow2_recip(d);
+        if (tid == 0) a.adiv[row] = d;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) {
+            const float o4[4] = {o[j].x * f, o[j].y * f, o[j].z * f, o[j].w * f};
+            if (in[j]) pack_parts4(a.Ap, a.mt, row, 4 * tid + 1024 * j, o4);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+            if (in[j]) *(float4 *)(a.y + off[j]) = o[j];
     }
 }
 
 constexpr int EA_Q = 16;      // queries per workgroup
 constexpr int EA_SMAX = 128;  // longest context
 constexpr int EA_HD = 64;
-constexpr int EA_KP = EA_HD + 4;   // K row pitch (floats): 16-byte rows, 16 consecutive keys in distinct banks
-constexpr int EA_PP = EA_SMAX + 1;
+constexpr int EA_PP = EA_SMAX + 4;   // pitches (floats): the four k groups and sixteen rows or columns that
+constexpr int EA_VP = EA_HD + 16;    // one MFMA operand read touches lie in distinct banks
 
-// one workgroup per (16 queries, head): scores, mask / bias, softmax and P·V in f32. Thread t
-// serves query t / 16: its scores are keys t % 16 + 16j (query row in registers, K rows read as
-// float4), its outputs columns 4 (t % 16) .. + 3 (V rows read as float4).
-__global__ __launch_bounds__(256) void enc_attn_kernel(const EncAttnArgs a) {
-    __shared__ __attribute__((aligned(16))) float Ks[EA_SMAX * EA_KP];
-    __shared__ __attribute__((aligned(16))) float Vs[EA_SMAX * EA_HD];
-    __shared__ __attribute__((aligned(16))) float Qs[EA_Q * EA_HD];
-    __shared__ float P[EA_Q * EA_PP];
-    const int tid = threadIdx.x, h = blockIdx.y, q0 = blockIdx.x * EA_Q, S = a.S;
-    for (int e = tid; e < S * (EA_HD / 4); e += 256) {
-        const int k = e >> 4, d = (e & 15) * 4;
-        const float *row = a.qkv + (long long)k * a.ld + h * EA_HD + d;
-        *(float4 *)&Ks[k * EA_KP + d] = *(const float4 *)(row + a.k_off);
-        *(float4 *)&Vs[k * EA_HD + d] = *(const float4 *)(row + a.v_off);
+// One workgroup of four waves per (16 queries, head), everything in f32 (v_mfma_f32_16x16x4_f32, f32
+// softmax). Wave w computes the scores of key blocks w and w + 4 (16 keys each) straight from the QKV
+// GEMM's splits, then the output columns 16 w .. + 15. The 64 products of a score run over d = 16 kq + i
+// so that a lane's share of a q or k row is 64 contiguous bytes. The kernel is latency-bound (77 keys:
+// at most 52 MFMAs a wave), so the loads of q, k and V of every split go out in one sequence,
+// so that all of them wait together (once per 4 splits): MT 16-key blocks at most.
+template <int MT>
+__global__ __launch_bounds__(256, 1) void enc_attn_kernel(const EncAttnArgs a) {
+    constexpr int KB = (MT + 3) / 4;   // key blocks of a wave
+    __shared__ __attribute__((aligned(16))) float Vs[16 * MT * EA_VP];
+    __shared__ __attribute__((aligned(16))) float P[EA_Q * EA_PP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, kq = lane >> 4;
+    // workgroups go to the 8 XCDs in turn: the query tiles of a head run on one XCD, whose L2 then serves
+    // the head's k and v to all but the first of them
+    const int S = a.S, H = a.nh * EA_HD, N = 3 * H, nkb = (S + 15) >> 4, idx = blockIdx.x >> 3;
+    const int h = idx / nkb * 8 + (blockIdx.x & 7), q0 = idx % nkb * EA_Q;
+    if (h >= a.nh) return;
+    // q row q0 + r16 and k rows 16 kb + r16, columns 16 kq .. + 15 of the head; V: 4 columns of rows
+    // tid / 16 + 16 i. Rows past the context repeat its last one: masked, or never stored.
+    constexpr int NV = 4 + 4 * KB + MT;
+    int off[NV];
+    float4 x[NV];
+    const int ch = h * EA_HD + 16 * kq, cv = 2 * H + h * EA_HD + (tid & 15) * 4;
+#pragma unroll
+    for (int i = 0; i < 4 + 4 * KB; ++i) {
+        const int row = i < 4 ? q0 + r16 : 16 * (wave + 4 * (i / 4 - 1)) + r16;
+        off[i] = min(row, S - 1) * N + (i < 4 ? 0 : H) + ch + 4 * (i & 3);
     }
-    {
-        const int q = tid >> 4, d = (tid & 15) * 4;
-        *(float4 *)&Qs[q * EA_HD + d] = q0 + q < S
-            ? *(const float4 *)(a.qkv + (long long)(q0 + q) * a.ld + a.q_off + h * EA_HD + d)
-            : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) off[4 + 4 * KB + i] = min((tid >> 4) + 16 * i, S - 1) * N + cv;
+    float4 bias[3][4];   // CLIP: q and k columns, and V's (bias[2][0])
+    if (a.qkv.bias) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            bias[0][i] = *(const float4 *)(a.qkv.bias + ch + 4 * i);
+            bias[1][i] = *(const float4 *)(a.qkv.bias + H + ch + 4 * i);
+        }
+        bias[2][0] = *(const float4 *)(a.qkv.bias + cv);
+    }
+    parts_sum<NV, MT <= 5 ? 4 : 2>(a.qkv, off, x);
+    if (a.qkv.bias) {
+#pragma unroll
+        for (int i = 0; i < 4 + 4 * KB; ++i) x[i] = add4(x[i], bias[i < 4 ? 0 : 1][i & 3]);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) x[4 + 4 * KB + i] = add4(x[4 + 4 * KB + i], bias[2][0]);
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+        *(float4 *)&Vs[((tid >> 4) + 16 * i) * EA_VP + (tid & 15) * 4] = x[4 + 4 * KB + i];
+    const int q = q0 + r16;
+#pragma unroll
+    for (int b = 0; b < KB; ++b) {
+        const int kb = wave + 4 * b;
+        if (kb >= nkb) break;
+        floatx4_t s = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 kv = x[4 + 4 * b + i], qv = x[i];
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.x, qv.x, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.y, qv.y, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.z, qv.z, s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.w, qv.w, s, 0, 0, 0);
+        }
+        // lane: keys 16 kb + 4 kq + r of query q
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int k = 16 * kb + 4 * kq + r;
+            s[r] *= a.scale;
+            bool keep = k < S;
+            if (a.mode == 1) {   // T5: padded keys masked, else the head's bias of the distance k - q
+                keep = keep && (a.keys[k >> 5] >> (k & 31) & 1);
+                if (keep && q < S) s[r] += a.rel[h * (2 * S - 1) + k - q + S - 1];
+            } else {             // CLIP: causal, and nothing past the end-of-text token
+                keep = keep && k <= q && k <= a.eot;
+            }
+            if (!keep) s[r] = -INFINITY;
+        }
+        *(floatx4_t *)&P[r16 * EA_PP + 16 * kb + 4 * kq] = s;
     }
     __syncthreads();
-    const int q = tid >> 4, t16 = tid & 15, qg = q0 + q;
-    {
-        float4 qv[EA_HD / 4];
+    // softmax: wave w takes queries 4 w .. + 3, one lane per key and 64 keys at a time
 #pragma unroll
-        for (int i = 0; i < EA_HD / 4; ++i) qv[i] = *(const float4 *)&Qs[q * EA_HD + 4 * i];
-        for (int k = t16; k < S; k += 16) {
-            const float *kr = &Ks[k * EA_KP];
-            float s = 0.0f;
+    for (int r = 0; r < 4; ++r) {
+        float *pr = P + (4 * wave + r) * EA_PP;
+        const int n = nkb * 16;
+        const float s0 = lane < n ? pr[lane] : -INFINITY, s1 = lane + 64 < n ? pr[lane + 64] : -INFINITY;
+        const float mx = wave_max(fmaxf(s0, s1));
+        const float e0 = expf(s0 - mx), e1 = expf(s1 - mx);
+        const float inv = 1.0f / wave_sum(e0 + e1);
+        if (lane < n) pr[lane] = e0 * inv;
+        if (lane + 64 < n) pr[lane + 64] = e1 * inv;
+    }
+    __syncthreads();
+    // V^T is the first operand: a lane holds columns 16 wave + 4 kq .. + 3 of query q
+    floatx4_t o[2] = {floatx4_t{0.f, 0.f, 0.f, 0.f}, floatx4_t{0.f, 0.f, 0.f, 0.f}};
+    for (int kb = 0; kb < nkb; ++kb)
 #pragma unroll
-            for (int i = 0; i < EA_HD / 4; ++i) {
-                const float4 kv = *(const float4 *)(kr + 4 * i);
-                s += qv[i].x * kv.x;
-                s += qv[i].y * kv.y;
-                s += qv[i].z * kv.z;
-                s += qv[i].w * kv.w;
+        for (int i = 0; i < 4; ++i) {
+            const int k = 16 * kb + 4 * i + kq;
+            o[i & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(Vs[k * EA_VP + 16 * wave + r16], P[r16 * EA_PP + k],
+                                                            o[i & 1], 0, 0, 0);
+        }
+    if (q >= S) return;
+    const floatx4_t y = o[0] + o[1];
+    const float f = pow2_recip(a.odiv[0]);
+    const float y4[4] = {y[0] * f, y[1] * f, y[2] * f, y[3] * f};
+    pack_parts4(a.Ap, a.mt, q, h * EA_HD + 16 * wave + 4 * kq, y4);
+}
+
+// The FFN activation of a GEMM's result as the next GEMM's operand, one workgroup per row (its largest
+// magnitude sets the scale): quick GELU of column c (shaders/ops_conv.metal:25-29), or gelu_tanh(column
+// c) * column F + c (GEGLU; tanh form, argument clamped to +-10: shaders/ops_conv.metal:15-24). A thread
+// has 4 columns of every 4096; those past the first 8192 are computed again when the scale is known.
+template <bool GEGLU>
+__global__ __launch_bounds__(1024) void enc_act_kernel(const EncParts p, half_t *Ap, float *adiv, int mt, int F) {
+    __shared__ float part[16];
+    const int tid = threadIdx.x, m = blockIdx.x;
+    auto act = [&](int c) {
+        constexpr int NV = GEGLU ? 2 : 1;
+        int off[NV];
+        float4 u[NV];
+#pragma unroll
+        for (int i = 0; i < NV; ++i) off[i] = m * p.N + i * F + c;
+        parts_sum<NV, 4>(p, off, u);
+        if (p.bias) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) u[i] = add4(u[i], *(const float4 *)(p.bias + i * F + c));
+        }
+        const float uv[4] = {u[0].x, u[0].y, u[0].z, u[0].w};
+        float y[4];
+        if constexpr (GEGLU) {
+            const float gv[4] = {u[1].x, u[1].y, u[1].z, u[1].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v = uv[e], t = 0.7978845608f * (v + 0.044715f * v * v * v);
+                y[e] = 0.5f * v * (1.0f + tanhf(fminf(fmaxf(t, -10.0f), 10.0f))) * gv[e];
             }
-            s *= a.scale;
-            if (a.mode == 1) {   // T5: padded keys masked, else the head's bias for the bucket of (q, k)
-                if (a.pad && a.pad[k] == 0) s = -INFINITY;
-                else if (qg < S) s += a.rel[a.bucket[qg * S + k] * a.nh + h];
-            } else if (a.mode == 2) {   // CLIP: causal, and nothing past the end-of-text token
-                if (!(k <= qg && k <= a.eot)) s = -INFINITY;
-            }
-            P[q * EA_PP + k] = s;
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[e] = uv[e] / (1.0f + expf(-1.702f * uv[e]));
+        }
+        return make_float4(y[0], y[1], y[2], y[3]);
+    };
+    float4 keep[2];
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int c = 4 * tid + 4096 * i;
+        if (c < F) {
+            keep[i] = act(c);
+            mx = fmaxf(mx, max4(keep[i]));
         }
     }
+    for (int c = 4 * tid + 8192; c < F; c += 4096) mx = fmaxf(mx, max4(act(c)));
+    mx = wave_max(mx);
+    if ((tid & 63) == 0) part[tid >> 6] = mx;
     __syncthreads();
-    {   // softmax: wave w takes rows w, w+4, w+8, w+12
-        const int lane = tid & 63, wave = tid >> 6;
-        for (int r = wave; r < EA_Q; r += 4) {
-            float *pr = P + r * EA_PP;
-            float mx = -INFINITY;
-            for (int k = lane; k < S; k += 64) mx = fmaxf(mx, pr[k]);
-            mx = wave_max(mx);
-            float sum = 0.0f;
-            for (int k = lane; k < S; k += 64) {
-                const float e = expf(pr[k] - mx);
-                pr[k] = e;
-                sum += e;
-            }
-            sum = wave_sum(sum);
-            const float inv = 1.0f / sum;
-            for (int k = lane; k < S; k += 64) pr[k] *= inv;
-        }
-    }
-    __syncthreads();
-    if (qg >= S) return;
-    const int d = t16 * 4;
-    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int k = 0; k < S; ++k) {
-        const float pk = P[q * EA_PP + k];
-        const float4 v = *(const float4 *)&Vs[k * EA_HD + d];
-        o.x += pk * v.x;
-        o.y += pk * v.y;
-        o.z += pk * v.z;
-        o.w += pk * v.w;
-    }
-    *(float4 *)(a.out + (long long)qg * a.ldo + h * EA_HD + d) = o;
+    mx = part[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, part[i]);
+    const float d = row_divisor(mx), f = pow2_recip(d);
+    if (tid == 0) adiv[m] = d;
+    auto pack = [&](int c, float4 y) {
+        const float y4[4] = {y.x * f, y.y * f, y.z * f, y.w * f};
+        pack_parts4(Ap, mt, m, c, y4);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        if (4 * tid + 4096 * i < F) pack(4 * tid + 4096 * i, keep[i]);
+    for (int c = 4 * tid + 8192; c < F; c += 4096) pack(c, act(c));
 }
 
-// y[r][c] = gelu_tanh(u[r][c]) * u[r][F + c] (tanh form, argument clamped to +-10: shaders/ops_conv.metal:15-24)
-__global__ void geglu_rows_kernel(const float *__restrict__ u, float *__restrict__ y, int rows, int F) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)rows * F) return;
-    const long long r = i / F;
-    const int c = (int)(i - r * F);
-    const float v = u[r * 2 * F + c], g = u[r * 2 * F + F + c];
-    const float t = 0.7978845608f * (v + 0.044715f * v * v * v);
-    y[i] = 0.5f * v * (1.0f + tanhf(fminf(fmaxf(t, -10.0f), 10.0f))) * g;
+// x[s][c] = tok[ids[s]][c] (+ pos[s][c]), one workgroup per row; the ids are kernel arguments, so the
+// call needs no copy to the device and no wait
+__global__ __launch_bounds__(256) void embed_rows_kernel(const EncIds ids, const float *__restrict__ tok,
+                                                         const float *__restrict__ pos, float *__restrict__ x, int H) {
+    const int s = blockIdx.x;
+    const float *t = tok + (long long)ids.id[s] * H;
+    for (int c = threadIdx.x * 4; c < H; c += 1024) {
+        float4 v = *(const float4 *)(t + c);
+        if (pos) v = add4(v, *(const float4 *)(pos + (long long)s * H + c));
+        *(float4 *)(x + (long long)s * H + c) = v;
+    }
 }
 
-// x[s][c] = tok[ids[s]][c] (+ pos[s][c])
-__global__ void embed_rows_kernel(const int32_t *__restrict__ ids, const float *__restrict__ tok,
-                                  const float *__restrict__ pos, float *__restrict__ x, int S, int H) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)S * H) return;
-    const int s = (int)(i / H), c = (int)(i - (long long)s * H);
-    float v = tok[(long long)ids[s] * H + c];
-    if (pos) v += pos[i];
-    x[i] = v;
-}
+bool aligned16(const void *p) { return (((uintptr_t)p) & 15) == 0; }
 
 } // namespace
 
-int launch_gemm_f32(const EncGemmArgs &gin, hipStream_t st) {
-    EncGemmArgs g = gin;
-    TSN_REQUIRE(g.A && g.W && g.Y && g.M > 0 && g.N > 0 && g.K > 0, "gemm_f32: null operand or empty shape");
-    TSN_REQUIRE(g.K % 4 == 0 && g.lda % 4 == 0 && g.ldw % 4 == 0 && g.lda >= g.K && g.ldw >= g.K && g.ldy >= g.N,
-                "gemm_f32: K and row strides multiples of 4, strides covering the rows");
-    TSN_REQUIRE((((uintptr_t)g.A) & 15) == 0 && (((uintptr_t)g.W) & 15) == 0, "gemm_f32: 16-byte aligned A and W");
-    TSN_REQUIRE(g.act == 0 || g.act == 1, "gemm_f32: activation 0 (none) or 1 (quick GELU)");
-    // The f32 MFMA bounds these GEMMs, so the K split balances K tiles per CU: estimated time in K
-    // tiles = rounds of 256 workgroups x K tiles per split, plus the partial sums written and read
-    // (about 8 MB per K-tile time) and a reduce launch. Splits are powers of two with at least 2 K
-    // tiles each, and the workspace must hold the partials.
-    const int tiles = ((g.N + FB_N - 1) / FB_N) * ((g.M + FB_M - 1) / FB_M);
-    const int nkt = (g.K + FB_K - 1) / FB_K;
-    int splits = 1;
-    double best = (double)((tiles + 255) / 256) * nkt;
-    for (int s = 2; g.ws && nkt / s >= 2 && (size_t)s * g.M * g.N * sizeof(float) <= g.ws_bytes; s *= 2) {
-        const double cost = (double)((tiles * s + 255) / 256) * ((nkt + s - 1) / s) + 1.0 +
-                            2.0 * s * g.M * (double)g.N * sizeof(float) / 8e6;
-        if (cost < best) {
-            best = cost;
-            splits = s;
-        }
-    }
-    g.kps = (nkt + splits - 1) / splits;
-    g.splits = (nkt + g.kps - 1) / g.kps;
-    TSN_LAUNCH(gemm_f32_kernel, dim3((g.N + FB_N - 1) / FB_N, (g.M + FB_M - 1) / FB_M, g.splits), dim3(256), 0, st, g);
+int enc_row_blocks(int M) { return M <= 32 ? 2 : M <= 80 ? 5 : 8; }
+size_t enc_operand_bytes(int M, int K) {   // whole 64-column steps
+    return (size_t)2 * enc_row_blocks(M) * 16 * ((K + 63) / 64 * 64) * sizeof(half_t);
+}
+
+size_t enc_weight_floats(int N, int K) { return (size_t)N * ((K + 63) / 64 * 64); }
+
+int launch_enc_weight_pack(const float *src, half_t *dst, float *div, int N, int K, hipStream_t st) {
+    TSN_REQUIRE(src && dst && div && N > 0 && K > 0 && N % 64 == 0 && K % 32 == 0 && aligned16(src) && aligned16(dst),
+                "enc_weight_pack: 16-byte aligned weights, N a multiple of 64, K of 32");
+    TSN_LAUNCH(enc_weight_scale_kernel, dim3(N), dim3(256), 0, st, src, div, K);
+    TSN_LAUNCH(enc_weight_pack_kernel, dim3((K + 63) / 64, N / 64), dim3(256), 0, st, src, div, dst, K);
     TSN_HIP_CHECK(hipGetLastError());
-    if (g.splits > 1) {
-        const long long n = (long long)g.M * g.N;
-        TSN_LAUNCH(enc_gemm_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, g);
-        TSN_HIP_CHECK(hipGetLastError());
-    }
     return TSN_OK;
 }
 
-int launch_enc_norm(const float *x, float *y, const float *w, const float *b, int rows, int H, float eps, bool ln,
-                    hipStream_t st) {
-    TSN_REQUIRE(x && y && w && rows > 0 && H > 0 && (!ln || b), "enc_norm: arguments");
-    TSN_REQUIRE(H % 4 == 0 && H <= 2048 && ((((uintptr_t)x) | ((uintptr_t)y) | ((uintptr_t)w) | ((uintptr_t)b)) & 15) == 0,
-                "enc_norm: rows of at most 2048 floats, a multiple of 4, 16-byte aligned");
-    if (ln) TSN_LAUNCH(enc_norm_kernel<true>, dim3(rows), dim3(256), 0, st, x, y, w, b, rows, H, eps);
-    else TSN_LAUNCH(enc_norm_kernel<false>, dim3(rows), dim3(256), 0, st, x, y, w, b, rows, H, eps);
+int launch_enc_gemm(EncGemmArgs &g, hipStream_t st) {
+    TSN_REQUIRE(g.Ap && g.adiv && g.W && g.wdiv && g.ws && g.M > 0 && g.M <= 128 && g.N > 0 && g.K > 0,
+                "enc_gemm: null operand, or rows outside 1..128");
+    TSN_REQUIRE(g.N % 64 == 0 && g.K % 32 == 0, "enc_gemm: N a multiple of 64, K of 32");
+    TSN_REQUIRE(aligned16(g.Ap) && aligned16(g.W) && aligned16(g.wdiv) && aligned16(g.ws), "enc_gemm: 16-byte aligned operands");
+    const int mt = enc_row_blocks(g.M);
+    TSN_REQUIRE((size_t)g.M * g.N * sizeof(float) <= g.ws_bytes, "enc_gemm: workspace");
+    // at most two workgroups per CU, of at least four steps each
+    const int tiles = g.N / 64, steps = (g.K + 63) / 64;
+    const int fit = (int)std::min<size_t>(std::max(1, steps / 4), g.ws_bytes / ((size_t)g.M * g.N * sizeof(float)));
+    const int want = std::max(1, std::min(std::min(fit, g.most), 512 / tiles));
+    g.kps = (steps + want - 1) / want;
+    g.splits = (steps + g.kps - 1) / g.kps;
+    const dim3 grid(tiles, g.splits, mt == 8 ? 2 : 1), block(256);   // more than 80 rows: two halves
+    if (mt == 2) TSN_LAUNCH((enc_gemm_kernel<2, 2>), grid, block, 0, st, g);
+    else if (mt == 5) TSN_LAUNCH((enc_gemm_kernel<5, 5>), grid, block, 0, st, g);
+    else TSN_LAUNCH((enc_gemm_kernel<4, 8>), grid, block, 0, st, g);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
+}
+
+int launch_enc_norm(const EncNormArgs &a, bool ln, hipStream_t st) {
+    TSN_REQUIRE(a.x && a.w && (a.y || a.Ap) && a.rows > 0 && a.H > 0 && (!ln || a.b), "enc_norm: arguments");
+    TSN_REQUIRE(!a.parts.ws || (a.xout && a.parts.splits > 0 && a.parts.N == a.H), "enc_norm: partial sums");
+    TSN_REQUIRE(!a.Ap || (a.adiv && a.rows <= 128 && a.H % 32 == 0), "enc_norm: packed rows");
+    TSN_REQUIRE(a.H % 4 == 0 && a.H <= 2048 && aligned16(a.x) && aligned16(a.y) && aligned16(a.w) && aligned16(a.b),
+                "enc_norm: rows of at most 2048 floats, a multiple of 4, 16-byte aligned");
+    if (ln && a.H <= 1024) TSN_LAUNCH((enc_norm_kernel<true, 1>), dim3(a.rows), dim3(256), 0, st, a);
+    else if (ln) TSN_LAUNCH((enc_norm_kernel<true, 2>), dim3(a.rows), dim3(256), 0, st, a);
+    else if (a.H <= 1024) TSN_LAUNCH((enc_norm_kernel<false, 1>), dim3(a.rows), dim3(256), 0, st, a);
+    else TSN_LAUNCH((enc_norm_kernel<false, 2>), dim3(a.rows), dim3(256), 0, st, a);
+    TSN_HIP_CHECK(hipGetLastError());
+    return TSN_OK;
+}
+
+int launch_enc_norm_rows(const float *x, float *y, const float *w, const float *b, int rows, int H, float eps, bool ln,
+                         hipStream_t st) {
+    TSN_REQUIRE(y, "enc_norm: arguments");
+    EncNormArgs a{};
+    a.x = x; a.y = y; a.w = w; a.b = b; a.rows = rows; a.H = H; a.eps = eps;
+    return launch_enc_norm(a, ln, st);
 }
 
 int launch_enc_attention(const EncAttnArgs &a, hipStream_t st) {
-    TSN_REQUIRE(a.qkv && a.out && a.S > 0 && a.S <= EA_SMAX && a.nh > 0 && a.hd == EA_HD,
-                "enc_attention: context 1..128, head width 64");
-    TSN_REQUIRE(a.mode == 0 || a.mode == 2 || (a.mode == 1 && a.rel && a.bucket), "enc_attention: mode and tables");
-    TSN_REQUIRE((((uintptr_t)a.qkv | (uintptr_t)a.out) & 15) == 0 && a.ld % 4 == 0 && a.ldo % 4 == 0 &&
-                    a.q_off % 4 == 0 && a.k_off % 4 == 0 && a.v_off % 4 == 0,
-                "enc_attention: 16-byte aligned rows (qkv, out, strides and offsets multiples of 4 floats)");
-    TSN_LAUNCH(enc_attn_kernel, dim3((a.S + EA_Q - 1) / EA_Q, a.nh), dim3(256), 0, st, a);
+    TSN_REQUIRE(a.qkv.ws && a.Ap && a.odiv && a.S > 0 && a.S <= EA_SMAX && a.nh > 0 && a.qkv.N == 3 * EA_HD * a.nh,
+                "enc_attention: context 1..128, rows of q, k and v with heads of 64");
+    TSN_REQUIRE((a.mode == 1 && a.rel) || a.mode == 2, "enc_attention: mode and tables");
+    const dim3 grid((a.nh + 7) / 8 * 8 * ((a.S + EA_Q - 1) / EA_Q)), block(256);
+    const int mt = enc_row_blocks(a.S);
+    if (mt == 2) TSN_LAUNCH(enc_attn_kernel<2>, grid, block, 0, st, a);
+    else if (mt == 5) TSN_LAUNCH(enc_attn_kernel<5>, grid, block, 0, st, a);
+    else TSN_LAUNCH(enc_attn_kernel<8>, grid, block, 0, st, a);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
 
-int launch_geglu_rows(const float *u, float *y, int rows, int F, hipStream_t st) {
-    TSN_REQUIRE(u && y && rows > 0 && F > 0, "geglu: arguments");
-    const long long n = (long long)rows * F;
-    TSN_LAUNCH(geglu_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, u, y, rows, F);
+int launch_enc_act(const EncParts &p, bool geglu, half_t *Ap, float *adiv, int rows, int F, hipStream_t st) {
+    TSN_REQUIRE(p.ws && Ap && adiv && rows > 0 && rows <= 128 && F > 0 && F % 32 == 0 && p.N == (geglu ? 2 * F : F),
+                "enc_act: arguments");
+    if (geglu) TSN_LAUNCH(enc_act_kernel<true>, dim3(rows), dim3(1024), 0, st, p, Ap, adiv, enc_row_blocks(rows), F);
+    else TSN_LAUNCH(enc_act_kernel<false>, dim3(rows), dim3(1024), 0, st, p, Ap, adiv, enc_row_blocks(rows), F);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
 
-int launch_embed_rows(const int32_t *ids, const float *tok, const float *pos, float *x, int S, int H, hipStream_t st) {
-    TSN_REQUIRE(ids && tok && x && S > 0 && H > 0, "embed: arguments");
-    const long long n = (long long)S * H;
-    TSN_LAUNCH(embed_rows_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, ids, tok, pos, x, S, H);
+int launch_embed_rows(const EncIds &ids, const float *tok, const float *pos, float *x, int S, int H, hipStream_t st) {
+    TSN_REQUIRE(tok && x && S > 0 && S <= EA_SMAX && H > 0 && H % 4 == 0, "embed: arguments");
+    TSN_LAUNCH(embed_rows_kernel, dim3(S), dim3(256), 0, st, ids, tok, pos, x, H);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }

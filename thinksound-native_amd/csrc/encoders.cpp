@@ -5,6 +5,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 
 #include "gguf.h"
@@ -151,6 +152,67 @@ std::vector<ManifestEntry> t5_manifest(const T5Spec &s) {
     return v;
 }
 
+// K splits of a QKV GEMM: attention reads every split of k and v in each of a head's workgroups (77 rows,
+// 1024 wide: attention 11.8 us with 4 splits, the GEMM 1.3 us less than with 2)
+constexpr int QKV_SPLITS = 4;
+
+int EncoderRunner::create_common(int ctx, int width, int ffn, int layers) {
+    TSN_TRY(alloc(enc_operand_bytes(ctx, width), (void **)&A_));
+    TSN_TRY(alloc(enc_operand_bytes(ctx, ffn), (void **)&F_));
+    TSN_TRY(alloc((size_t)ctx * 4, (void **)&adiv_));
+    TSN_TRY(alloc((size_t)ctx * 4, (void **)&fdiv_));
+    TSN_TRY(alloc((size_t)layers * ctx * 4, (void **)&odiv_));
+    return alloc(ENC_WS_BYTES, (void **)&ws_);
+}
+
+int EncoderRunner::gemm(const half_t *A, const float *adiv, const EncWeight &W, const float *b, int M, int N, int K,
+                        EncParts &out, int most) {
+    EncGemmArgs g{A, adiv, W.w, W.div, ws_, ENC_WS_BYTES, M, N, K, most, 1, 0};
+    TSN_TRY(run("enc_gemm_kernel", 2.0 * M * N * K, 4.0 * ((double)N * K + M * (double)N + M * (double)K),
+                [&] { return launch_enc_gemm(g, rt->dev.stream()); }));
+    out = EncParts{ws_, (long long)M * N, g.splits, N, b};
+    return TSN_OK;
+}
+
+int EncoderRunner::pack_weights(const std::vector<RawWeight> &ws) {
+    size_t most = 0, rows = 0;
+    for (const RawWeight &w : ws) {
+        most = std::max(most, (size_t)w.N * w.K * sizeof(float));
+        rows += (size_t)w.N;
+    }
+    void *tmp;
+    float *div;
+    TSN_TRY(alloc(rows * sizeof(float), (void **)&div));
+    TSN_TRY(alloc(most, &tmp));
+    const hipStream_t st = rt->dev.stream();
+    for (const RawWeight &w : ws) {
+        TSN_TRY(rt->dev.copy_d2d(tmp, w.p, (size_t)w.N * w.K * sizeof(float)));
+        TSN_TRY(launch_enc_weight_pack((const float *)tmp, (half_t *)w.p, div, w.N, w.K, st));
+        *w.out = EncWeight{(const half_t *)w.p, div};
+        div += w.N;
+    }
+    return release(tmp);
+}
+
+// An output of attention is a mean of v rows, and |v| <= |norm output| |row of Wv| + |bv| with
+// |norm output| <= sqrt(width) max|nw| + |nb|. The bound may be loose: values 2^-16 of it still keep 22 bits.
+int EncoderRunner::set_odiv(int layer, int ctx, int width, const float *wv, const float *bv, const float *nw, const float *nb) {
+    double row = 0.0, w = 0.0, b2 = 0.0, bias = 0.0;
+    for (int n = 0; n < width; ++n) {
+        double s = 0.0;
+        for (int k = 0; k < width; ++k) s += (double)wv[(size_t)n * width + k] * wv[(size_t)n * width + k];
+        row = std::max(row, s);
+        if (bv) bias = std::max(bias, fabs((double)bv[n]));
+        w = std::max(w, fabs((double)nw[n]));
+        if (nb) b2 += (double)nb[n] * nb[n];
+    }
+    const double bound = (sqrt((double)width) * w + sqrt(b2)) * sqrt(row) + bias;
+    // bound / div below 2^15; exponents as the device's row_divisor has them
+    const int e = bound > 0.0 && std::isfinite(bound) ? std::min(std::max(ilogb(bound), -95), 127) : 0;
+    const std::vector<float> div((size_t)ctx, ldexpf(1.0f, e - 14));
+    return rt->dev.upload(odiv_ + (size_t)layer * ctx, div.data(), div.size() * sizeof(float));
+}
+
 /* ---------------- CLIP ---------------- */
 
 int ClipModel::create(Runtime *r, const ClipSpec &sp) {
@@ -160,13 +222,7 @@ int ClipModel::create(Runtime *r, const ClipSpec &sp) {
     s = sp;
     const size_t n = s.ctx, H = s.H;
     TSN_TRY(alloc(n * H * 4, (void **)&X_));
-    TSN_TRY(alloc(n * H * 4, (void **)&R_));
-    TSN_TRY(alloc(n * 3 * H * 4, (void **)&QKV_));
-    TSN_TRY(alloc(n * H * 4, (void **)&ATT_));
-    TSN_TRY(alloc(n * 4 * H * 4, (void **)&FF_));
-    TSN_TRY(alloc(n * 4, (void **)&ids_));
-    TSN_TRY(alloc(ENC_WS_BYTES, (void **)&ws_));
-    return TSN_OK;
+    return create_common(s.ctx, s.H, 4 * s.H, s.NL);
 }
 
 int ClipModel::upload_weights(const float *host, size_t numel) { return upload(host, numel); }
@@ -194,7 +250,7 @@ int ClipModel::upload(const float *host, size_t numel) {
         const std::string leaf = stem.empty() ? n : n.substr(stem.size() + 1);
         if (leaf == "q.w" || leaf == "k.w" || leaf == "v.w") {   // one [3H][H] weight per layer
             const size_t j = leaf[0] == 'q' ? 0 : leaf[0] == 'k' ? 1 : 2;
-            if (j == 0) lay.put(stem + ".qkv.w", 3 * H * H);
+            if (j == 0) lay.put(stem + ".qkv.w", enc_weight_floats(3 * s.H, s.H));
             group[n] = {stem + ".qkv.w", j * H * H};
         } else if (leaf == "q.b" || leaf == "k.b" || leaf == "v.b") {
             const size_t j = leaf[0] == 'q' ? 0 : leaf[0] == 'k' ? 1 : 2;
@@ -211,15 +267,25 @@ int ClipModel::upload(const float *host, size_t numel) {
     tok_ = P("tok_emb");
     pos_ = P("pos_emb");
     L_.resize(s.NL);
+    std::vector<RawWeight> pw;
+    auto at = [&](const std::string &n) {   // host tensor
+        return host + std::find_if(man.begin(), man.end(), [&](const ManifestEntry &e) { return e.name == n; })->offset;
+    };
     for (int l = 0; l < s.NL; ++l) {
         const std::string b = "blk." + std::to_string(l);
-        L_[l] = Layer{P(b + ".ln1.w"), P(b + ".ln1.b"), P(b + ".qkv.w"), P(b + ".qkv.b"), P(b + ".out.w"),
-                      P(b + ".out.b"), P(b + ".ln2.w"), P(b + ".ln2.b"), P(b + ".fc1.w"), P(b + ".fc1.b"),
-                      P(b + ".fc2.w"), P(b + ".fc2.b")};
+        Layer &L = L_[l];
+        L.ln1w = P(b + ".ln1.w"); L.ln1b = P(b + ".ln1.b"); L.bqkv = P(b + ".qkv.b"); L.bo = P(b + ".out.b");
+        L.ln2w = P(b + ".ln2.w"); L.ln2b = P(b + ".ln2.b"); L.b1 = P(b + ".fc1.b"); L.b2 = P(b + ".fc2.b");
+        pw.push_back({dev + lay.at.at(b + ".qkv.w"), 3 * s.H, s.H, &L.Wqkv});
+        pw.push_back({dev + lay.at.at(b + ".out.w"), s.H, s.H, &L.Wo});
+        pw.push_back({dev + lay.at.at(b + ".fc1.w"), 4 * s.H, s.H, &L.W1});
+        pw.push_back({dev + lay.at.at(b + ".fc2.w"), s.H, 4 * s.H, &L.W2});
+        TSN_TRY(set_odiv(l, s.ctx, s.H, at(b + ".v.w"), at(b + ".v.b"), at(b + ".ln1.w"), at(b + ".ln1.b")));
     }
     lnw_ = P("out_ln.w");
     lnb_ = P("out_ln.b");
     proj_ = P("text_proj");
+    TSN_TRY(pack_weights(pw));
     ready_ = true;
     return TSN_OK;
 }
@@ -229,37 +295,45 @@ int ClipModel::encode(const int32_t *ids, float *per_token, float *global) {
     TSN_REQUIRE(ids && per_token && global, "clip: null ids or outputs");
     const int n = s.ctx, H = s.H;
     int eos = 0;
+    EncIds id{};
     for (int i = 0; i < n; ++i) {
         TSN_REQUIRE(ids[i] >= 0 && ids[i] < s.vocab, "clip: token id outside the vocabulary");
         if (ids[i] > ids[eos]) eos = i;   // first position of the largest id (src/clip.cpp:45-46)
+        id.id[i] = ids[i];
     }
-    TSN_TRY(rt->dev.upload(ids_, ids, (size_t)n * 4));
+    TSN_TRY(rt->dev.make_current());
     const hipStream_t st = rt->dev.stream();
-    auto gemm = [&](const float *A, int lda, const float *W, const float *b, float *Y, int ldy, int M, int N, int K,
-                    int resid, int act) {
-        EncGemmArgs g{A, lda, W, K, b, Y, ldy, M, N, K, resid, act, ws_, ENC_WS_BYTES, 1, 0};
-        return run("gemm_f32_kernel", 2.0 * M * N * K, 4.0 * ((double)N * K + (double)M * K + M * (double)N),
-                   [&] { return launch_gemm_f32(g, st); });
+    const int mt = enc_row_blocks(n);
+    // X += the pending GEMM result (if any), then LN into the operand A_ or, last, per_token
+    auto norm = [&](const EncParts &p, const float *w, const float *b, float *y) {
+        EncNormArgs a{X_, X_, p, w, b, y, y ? nullptr : A_, adiv_, mt, n, H, s.eps};
+        return run("enc_norm_kernel<true>", 0, 4.0 * n * H * (p.ws ? p.splits + 3 : 2),
+                   [&] { return launch_enc_norm(a, true, st); });
     };
-    auto norm = [&](const float *x, float *y, const float *w, const float *b) {
-        return run("enc_norm_kernel<true>", 0, 8.0 * n * H, [&] { return launch_enc_norm(x, y, w, b, n, H, s.eps, true, st); });
-    };
-    TSN_TRY(run("embed_rows_kernel", 0, 12.0 * n * H, [&] { return launch_embed_rows(ids_, tok_, pos_, X_, n, H, st); }));
+    EncParts p{}, none{};
+    TSN_TRY(run("embed_rows_kernel", 0, 12.0 * n * H, [&] { return launch_embed_rows(id, tok_, pos_, X_, n, H, st); }));
     for (int l = 0; l < s.NL; ++l) {
         const Layer &w = L_[l];
-        TSN_TRY(norm(X_, R_, w.ln1w, w.ln1b));
-        TSN_TRY(gemm(R_, H, w.Wqkv, w.bqkv, QKV_, 3 * H, n, 3 * H, H, 0, 0));
-        EncAttnArgs a{QKV_, 3 * H, 0, H, 2 * H, ATT_, H, n, s.NH, 64, 0.125f, 2, nullptr, nullptr, nullptr, eos};
-        TSN_TRY(run("enc_attn_kernel", 4.0 * s.NH * n * (double)n * 64, 16.0 * n * H,
+        const float *odiv = odiv_ + (size_t)l * n;
+        TSN_TRY(norm(l ? p : none, w.ln1w, w.ln1b, nullptr));
+        TSN_TRY(gemm(A_, adiv_, w.Wqkv, w.bqkv, n, 3 * H, H, p, QKV_SPLITS));
+        EncAttnArgs a{p, A_, odiv, mt, n, s.NH, 0.125f, 2, nullptr, {0, 0, 0, 0}, eos};
+        TSN_TRY(run("enc_attn_kernel", 4.0 * s.NH * n * (double)n * 64, 4.0 * n * H * (3 * p.splits + 1.5),
                     [&] { return launch_enc_attention(a, st); }));
-        TSN_TRY(gemm(ATT_, H, w.Wo, w.bo, X_, H, n, H, H, 1, 0));
-        TSN_TRY(norm(X_, R_, w.ln2w, w.ln2b));
-        TSN_TRY(gemm(R_, H, w.W1, w.b1, FF_, 4 * H, n, 4 * H, H, 0, 1));
-        TSN_TRY(gemm(FF_, 4 * H, w.W2, w.b2, X_, H, n, H, 4 * H, 1, 0));
+        TSN_TRY(gemm(A_, odiv, w.Wo, w.bo, n, H, H, p));
+        TSN_TRY(norm(p, w.ln2w, w.ln2b, nullptr));
+        TSN_TRY(gemm(A_, adiv_, w.W1, w.b1, n, 4 * H, H, p));
+        TSN_TRY(run("enc_act_kernel<false>", 0, 4.0 * n * 4 * H * (p.splits + 1.5),
+                    [&] { return launch_enc_act(p, false, F_, fdiv_, n, 4 * H, st); }));
+        TSN_TRY(gemm(F_, fdiv_, w.W2, w.b2, n, H, 4 * H, p));
     }
-    TSN_TRY(norm(X_, per_token, lnw_, lnb_));
+    TSN_TRY(norm(p, lnw_, lnb_, per_token));
     // pooled: text_proj · per_token[eos] (src/clip.cpp:88-91)
-    return gemm(per_token + (size_t)eos * H, H, proj_, nullptr, global, H, 1, H, H, 0, 0);
+    GemvArgs v;
+    memset(&v, 0, sizeof v);
+    v.W = proj_; v.ldw = H; v.wdt = DT_F32; v.X = per_token + (size_t)eos * H; v.ldx = H; v.Y = global; v.ldy = H;
+    v.N = H; v.K = H; v.nb = 1;
+    return run("gemv_kernel", 2.0 * H * H, 4.0 * H * H, [&] { return launch_gemv(v, st); });
 }
 
 /* ---------------- T5 ---------------- */
@@ -269,23 +343,10 @@ int T5Model::create(Runtime *r, const T5Spec &sp) {
     TSN_TRY(t5_spec_check(sp));
     rt = r;
     s = sp;
-    const size_t n = s.ctx, d = s.d, F = s.d_ff;
+    const size_t n = s.ctx, d = s.d;
     TSN_TRY(alloc(n * d * 4, (void **)&X_));
-    TSN_TRY(alloc(n * d * 4, (void **)&R_));
-    TSN_TRY(alloc(n * 3 * d * 4, (void **)&QKV_));
-    TSN_TRY(alloc(n * d * 4, (void **)&ATT_));
-    TSN_TRY(alloc(n * 2 * F * 4, (void **)&U_));
-    TSN_TRY(alloc(n * F * 4, (void **)&G_));
-    TSN_TRY(alloc(n * 4, (void **)&ids_));
-    TSN_TRY(alloc(n * 4, (void **)&pad_));
-    TSN_TRY(alloc(ENC_WS_BYTES, (void **)&ws_));
-    // bucket of (q, k) = bucket(k - q) (src/t5.cpp:47-53)
-    std::vector<int32_t> bk(n * n);
-    for (size_t q = 0; q < n; ++q)
-        for (size_t k = 0; k < n; ++k) bk[q * n + k] = t5_bucket((int)k - (int)q, s.n_bucket, s.max_dist);
-    TSN_TRY(alloc(bk.size() * 4, (void **)&bucket_));
-    TSN_TRY(rt->dev.upload(bucket_, bk.data(), bk.size() * 4));
-    return TSN_OK;
+    TSN_TRY(alloc((2 * n - 1) * s.NH * 4, (void **)&rel_));
+    return create_common(s.ctx, s.d, s.d_ff, s.NL);
 }
 
 int T5Model::upload_weights(const float *host, size_t numel) { return upload(host, numel); }
@@ -313,12 +374,14 @@ int T5Model::upload(const float *host, size_t numel) {
         const std::string leaf = stem.empty() ? n : n.substr(stem.size() + 1);
         if (leaf == "q" || leaf == "k" || leaf == "v") {
             const size_t j = leaf == "q" ? 0 : leaf == "k" ? 1 : 2;
-            if (j == 0) lay.put(stem + ".qkv", 3 * d * d);
+            if (j == 0) lay.put(stem + ".qkv", enc_weight_floats(3 * s.d, s.d));
             group[n] = {stem + ".qkv", j * d * d};
         } else if (leaf == "wi_0" || leaf == "wi_1") {   // one [2F][d] weight: wi_0 rows, then wi_1 rows
             const size_t j = leaf == "wi_0" ? 0 : 1;
-            if (j == 0) lay.put(stem + ".wi", 2 * F * d);
+            if (j == 0) lay.put(stem + ".wi", enc_weight_floats(2 * s.d_ff, s.d));
             group[n] = {stem + ".wi", j * F * d};
+        } else if (leaf == "wo") {
+            lay.put(n, enc_weight_floats(s.d, s.d_ff));
         } else {
             lay.put(n, (size_t)e.numel);
         }
@@ -329,12 +392,30 @@ int T5Model::upload(const float *host, size_t numel) {
     auto P = [&](const std::string &n) { return (const float *)(dev + lay.at.at(n)); };
     tok_ = P("tok_emb");
     L_.resize(s.NL);
+    std::vector<RawWeight> pw;
+    auto at = [&](const std::string &n) {   // host tensor
+        return host + std::find_if(man.begin(), man.end(), [&](const ManifestEntry &e) { return e.name == n; })->offset;
+    };
     for (int l = 0; l < s.NL; ++l) {
         const std::string b = "blk." + std::to_string(l);
-        L_[l] = Layer{P(b + ".attn_norm"), P(b + ".qkv"), P(b + ".o"), P(b + ".ffn_norm"), P(b + ".wi"), P(b + ".wo")};
+        Layer &L = L_[l];
+        L.an = P(b + ".attn_norm"); L.fn = P(b + ".ffn_norm");
+        pw.push_back({dev + lay.at.at(b + ".qkv"), 3 * s.d, s.d, &L.Wqkv});
+        pw.push_back({dev + lay.at.at(b + ".o"), s.d, s.d, &L.Wo});
+        pw.push_back({dev + lay.at.at(b + ".wi"), 2 * s.d_ff, s.d, &L.Wi});
+        pw.push_back({dev + lay.at.at(b + ".wo"), s.d, s.d_ff, &L.Wout});
+        TSN_TRY(set_odiv(l, s.ctx, s.d, at(b + ".v"), nullptr, at(b + ".attn_norm"), nullptr));
     }
-    rel_ = P("rel_bias");
     on_ = P("out_norm");
+    // the bias of each head by distance k - q in -(ctx - 1) .. ctx - 1: bucket(k - q) (src/t5.cpp:47-53)
+    const float *rb = at("rel_bias");
+    const int span = 2 * s.ctx - 1;
+    std::vector<float> rel((size_t)span * s.NH);
+    for (int h = 0; h < s.NH; ++h)
+        for (int i = 0; i < span; ++i)
+            rel[(size_t)h * span + i] = rb[(size_t)t5_bucket(i - (s.ctx - 1), s.n_bucket, s.max_dist) * s.NH + h];
+    TSN_TRY(rt->dev.upload(rel_, rel.data(), rel.size() * sizeof(float)));
+    TSN_TRY(pack_weights(pw));
     ready_ = true;
     return TSN_OK;
 }
@@ -343,39 +424,41 @@ int T5Model::encode(const int32_t *ids, float *out) {
     TSN_REQUIRE(ready_, "t5: weights not uploaded");
     TSN_REQUIRE(ids && out, "t5: null ids or output");
     const int n = s.ctx, d = s.d, F = s.d_ff;
-    std::vector<int32_t> pad((size_t)n);
+    EncIds id{};
+    uint32_t keys[4] = {0, 0, 0, 0};
     for (int i = 0; i < n; ++i) {
         TSN_REQUIRE(ids[i] >= 0 && ids[i] < s.vocab, "t5: token id outside the vocabulary");
-        pad[i] = ids[i] != 0;   // keys of id 0 (pad) masked (src/t5.cpp:90-94)
+        id.id[i] = ids[i];
+        if (ids[i] != 0) keys[i >> 5] |= 1u << (i & 31);   // keys of id 0 (pad) masked (src/t5.cpp:90-94)
     }
-    TSN_TRY(rt->dev.upload(ids_, ids, (size_t)n * 4));
-    TSN_TRY(rt->dev.upload(pad_, pad.data(), (size_t)n * 4));
+    TSN_TRY(rt->dev.make_current());
     const hipStream_t st = rt->dev.stream();
-    auto gemm = [&](const float *A, int lda, const float *W, float *Y, int ldy, int M, int N, int K, int resid) {
-        EncGemmArgs g{A, lda, W, K, nullptr, Y, ldy, M, N, K, resid, 0, ws_, ENC_WS_BYTES, 1, 0};
-        return run("gemm_f32_kernel", 2.0 * M * N * K, 4.0 * ((double)N * K + (double)M * K + M * (double)N),
-                   [&] { return launch_gemm_f32(g, st); });
+    const int mt = enc_row_blocks(n);
+    // X += the pending GEMM result (if any), then RMS into the operand A_ or, last, out
+    auto rms = [&](const EncParts &p, const float *w, float *y) {
+        EncNormArgs a{X_, X_, p, w, nullptr, y, y ? nullptr : A_, adiv_, mt, n, d, s.eps};
+        return run("enc_norm_kernel<false>", 0, 4.0 * n * d * (p.ws ? p.splits + 3 : 2),
+                   [&] { return launch_enc_norm(a, false, st); });
     };
-    auto rms = [&](const float *x, float *y, const float *w) {
-        return run("enc_norm_kernel<false>", 0, 8.0 * n * d,
-                   [&] { return launch_enc_norm(x, y, w, nullptr, n, d, s.eps, false, st); });
-    };
-    TSN_TRY(run("embed_rows_kernel", 0, 8.0 * n * d, [&] { return launch_embed_rows(ids_, tok_, nullptr, X_, n, d, st); }));
+    EncParts p{}, none{};
+    TSN_TRY(run("embed_rows_kernel", 0, 8.0 * n * d, [&] { return launch_embed_rows(id, tok_, nullptr, X_, n, d, st); }));
     for (int l = 0; l < s.NL; ++l) {
         const Layer &w = L_[l];
-        TSN_TRY(rms(X_, R_, w.an));
-        TSN_TRY(gemm(R_, d, w.Wqkv, QKV_, 3 * d, n, 3 * d, d, 0));
+        const float *odiv = odiv_ + (size_t)l * n;
+        TSN_TRY(rms(l ? p : none, w.an, nullptr));
+        TSN_TRY(gemm(A_, adiv_, w.Wqkv, nullptr, n, 3 * d, d, p, QKV_SPLITS));
         // scale 1: T5 folds 1/sqrt(d_kv) into q (src/t5.cpp:70)
-        EncAttnArgs a{QKV_, 3 * d, 0, d, 2 * d, ATT_, d, n, s.NH, 64, 1.0f, 1, bucket_, rel_, pad_, 0};
-        TSN_TRY(run("enc_attn_kernel", 4.0 * s.NH * n * (double)n * 64, 16.0 * n * d,
+        EncAttnArgs a{p, A_, odiv, mt, n, s.NH, 1.0f, 1, rel_, {keys[0], keys[1], keys[2], keys[3]}, 0};
+        TSN_TRY(run("enc_attn_kernel", 4.0 * s.NH * n * (double)n * 64, 4.0 * n * d * (3 * p.splits + 1.5),
                     [&] { return launch_enc_attention(a, st); }));
-        TSN_TRY(gemm(ATT_, d, w.Wo, X_, d, n, d, d, 1));
-        TSN_TRY(rms(X_, R_, w.fn));
-        TSN_TRY(gemm(R_, d, w.Wi, U_, 2 * F, n, 2 * F, d, 0));
-        TSN_TRY(run("geglu_rows_kernel", 0, 12.0 * n * F, [&] { return launch_geglu_rows(U_, G_, n, F, st); }));
-        TSN_TRY(gemm(G_, F, w.Wout, X_, d, n, d, F, 1));
+        TSN_TRY(gemm(A_, odiv, w.Wo, nullptr, n, d, d, p));
+        TSN_TRY(rms(p, w.fn, nullptr));
+        TSN_TRY(gemm(A_, adiv_, w.Wi, nullptr, n, 2 * F, d, p));
+        TSN_TRY(run("enc_act_kernel<true>", 0, 4.0 * n * F * (2 * p.splits + 1.5),
+                    [&] { return launch_enc_act(p, true, F_, fdiv_, n, F, st); }));
+        TSN_TRY(gemm(F_, fdiv_, w.Wout, nullptr, n, d, F, p));
     }
-    return rms(X_, out, on_);
+    return rms(p, on_, out);
 }
 
 } // namespace tsn

@@ -16,7 +16,7 @@
 
 namespace tsn {
 
-constexpr size_t ENC_WS_BYTES = (size_t)32 << 20;   // split-K partials of the f32 GEMMs
+constexpr size_t ENC_WS_BYTES = (size_t)32 << 20;   // K-split sums of one GEMM
 
 struct ClipSpec {   // field meaning documented in include/tsn.h (tsn_clip_spec)
     int H, NL, NH, ctx, vocab;
@@ -38,7 +38,34 @@ int t5_spec_from_gguf(const char *path, T5Spec *out);       // t5.* metadata
 // bidirectional bucket of relative position rel = k - q (src/t5.cpp:6-19)
 int t5_bucket(int rel, int n_bucket, int max_dist);
 
-class ClipModel : public GraphRunner {
+struct EncWeight {   // a packed [N][K] weight and its row divisors
+    const half_t *w;
+    const float *div;
+};
+
+class EncoderRunner : public GraphRunner {
+protected:
+    float *ws_ = nullptr;                        // ENC_WS_BYTES
+    half_t *A_ = nullptr, *F_ = nullptr;         // packed GEMM operands: width and FFN columns
+    float *adiv_ = nullptr, *fdiv_ = nullptr;    // their row divisors
+    float *odiv_ = nullptr;                      // [layers][ctx] divisors of the attention outputs
+    int create_common(int ctx, int width, int ffn, int layers);
+    // out = A·Wᵀ (+ b) as K-split sums in ws_, for the next kernel to read
+    int gemm(const half_t *A, const float *adiv, const EncWeight &W, const float *b, int M, int N, int K, EncParts &out,
+             int most = 1 << 20);
+    // row-major [N][K] weights at p, each in a region of enc_weight_floats, packed in place
+    struct RawWeight {
+        float *p;
+        int N, K;
+        EncWeight *out;
+    };
+    int pack_weights(const std::vector<RawWeight> &ws);
+    // odiv_ of a layer: a power of two that brings its v rows below the f16 range. wv [width][width]
+    // host rows, bv their bias, and the norm's weight and bias (null: none)
+    int set_odiv(int layer, int ctx, int width, const float *wv, const float *bv, const float *nw, const float *nb);
+};
+
+class ClipModel : public EncoderRunner {
 public:
     int create(Runtime *rt, const ClipSpec &s);
     int upload_weights(const float *host, size_t numel);   // flat f32, manifest order
@@ -50,17 +77,17 @@ public:
 
 private:
     struct Layer {
-        const float *ln1w, *ln1b, *Wqkv, *bqkv, *Wo, *bo, *ln2w, *ln2b, *W1, *b1, *W2, *b2;
+        const float *ln1w, *ln1b, *bqkv, *bo, *ln2w, *ln2b, *b1, *b2;
+        EncWeight Wqkv, Wo, W1, W2;
     };
     std::vector<Layer> L_;
     const float *tok_ = nullptr, *pos_ = nullptr, *lnw_ = nullptr, *lnb_ = nullptr, *proj_ = nullptr;
-    float *X_ = nullptr, *R_ = nullptr, *QKV_ = nullptr, *ATT_ = nullptr, *FF_ = nullptr, *ws_ = nullptr;
-    int32_t *ids_ = nullptr;
+    float *X_ = nullptr;
     bool ready_ = false;
     int upload(const float *host, size_t numel);
 };
 
-class T5Model : public GraphRunner {
+class T5Model : public EncoderRunner {
 public:
     int create(Runtime *rt, const T5Spec &s);
     int upload_weights(const float *host, size_t numel);   // flat f32, manifest order
@@ -72,12 +99,12 @@ public:
 
 private:
     struct Layer {
-        const float *an, *Wqkv, *Wo, *fn, *Wi, *Wout;
+        const float *an, *fn;
+        EncWeight Wqkv, Wo, Wi, Wout;
     };
     std::vector<Layer> L_;
-    const float *tok_ = nullptr, *rel_ = nullptr, *on_ = nullptr;
-    float *X_ = nullptr, *R_ = nullptr, *QKV_ = nullptr, *ATT_ = nullptr, *U_ = nullptr, *G_ = nullptr, *ws_ = nullptr;
-    int32_t *ids_ = nullptr, *pad_ = nullptr, *bucket_ = nullptr;
+    const float *tok_ = nullptr, *on_ = nullptr;
+    float *X_ = nullptr, *rel_ = nullptr;   // rel_: [NH][2 ctx - 1] bias by distance
     bool ready_ = false;
     int upload(const float *host, size_t numel);
 };

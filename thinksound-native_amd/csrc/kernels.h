@@ -360,42 +360,69 @@ int launch_split3(const float *x, long long rows, int C, half_t *out, hipStream_
 // y [T][OC] = conv(snake(x), W [OC][C][KK], pad), no bias; x [T][C] f32, OC in {1, 2, 4}, KK == 7, C % 8 == 0
 int launch_conv_out(const float *x, const float *ab, const float *W, float *y, int T, int C, int OC, int KK, int pad,
                     hipStream_t st);
-// Text encoders (enc.hip), all f32.
-// gemm_f32: Y[m*ldy + n] = act(sum_k A[m*lda + k] W[n*ldw + k] + bias[n]) (act 1: quick GELU), or with
-// resid set Y[m*ldy + n] += sum + bias[n]; K % 4 == 0, f32 MFMA. With a workspace the launcher may
-// split K (partials reduced in split order by a second kernel it launches); splits and kps are its own.
+// Text encoders (enc.hip). GEMM operands are pairs of f16 parts of rows divided by a power of two, packed
+// by their producer; a GEMM leaves the sums of its K splits, which the next kernel adds in order.
+// 16-row blocks of a packed operand of M <= 128 rows, and its size for K columns
+int enc_row_blocks(int M);
+size_t enc_operand_bytes(int M, int K);
+// size in floats of a packed [N][K] weight (K in whole 64-column steps), and the packing of a row-major
+// one, with its row divisors div[N]
+size_t enc_weight_floats(int N, int K);
+int launch_enc_weight_pack(const float *src, half_t *dst, float *div, int N, int K, hipStream_t st);
+// ws[z][M][N] = the sums over K split z of A[M][K] W[N][K]^T; M <= 128, N % 64 == 0, K % 32 == 0.
+// The launcher chooses at most `most` splits, and kps (64-column K steps per split).
 struct EncGemmArgs {
-    const float *A; int lda;
-    const float *W; int ldw;
-    const float *bias;
-    float *Y; int ldy;
-    int M, N, K;
-    int resid, act;
+    const half_t *Ap; const float *adiv;   // rows and their divisors
+    const half_t *W; const float *wdiv;
     float *ws; size_t ws_bytes;
+    int M, N, K;
+    int most;
     int splits, kps;
 };
-int launch_gemm_f32(const EncGemmArgs &g, hipStream_t st);
-// LayerNorm with weight and bias (ln) or RMSNorm with weight, rows of H floats
-int launch_enc_norm(const float *x, float *y, const float *w, const float *b, int rows, int H, float eps, bool ln,
-                    hipStream_t st);
-// attention over one context of S <= 128 rows, heads of 64: q, k, v at column offsets q_off/k_off/v_off
-// + 64h of qkv rows (stride ld), output at column 64h of out rows (stride ldo);
-// mode 0 none, 1 T5 (keys with pad[k] == 0 masked, else + rel[bucket[q*S + k]*nh + h]),
+int launch_enc_gemm(EncGemmArgs &g, hipStream_t st);
+// a GEMM's result as its reader takes it: the sum of splits [M][N] arrays, stride floats apart, + bias[N]
+struct EncParts {
+    const float *ws;
+    long long stride;
+    int splits, N;
+    const float *bias;
+};
+// xout = x + parts (when parts.ws), then LayerNorm with weight and bias (ln) or RMSNorm with weight,
+// rows of H floats, as f32 rows y or the packed operand Ap with its divisors adiv
+struct EncNormArgs {
+    const float *x; float *xout;
+    EncParts parts;
+    const float *w, *b;
+    float *y;
+    half_t *Ap; float *adiv; int mt;
+    int rows, H;
+    float eps;
+};
+int launch_enc_norm(const EncNormArgs &a, bool ln, hipStream_t st);
+int launch_enc_norm_rows(const float *x, float *y, const float *w, const float *b, int rows, int H, float eps, bool ln,
+                         hipStream_t st);
+// attention over one context of S <= 128 rows [q | k | v] of nh heads of 64, output packed, every row
+// divided by odiv[0] (a bound of the values: an output is a mean of v rows);
+// mode 1 T5 (keys whose bit of `keys` is clear masked, else + rel[h*(2S - 1) + k - q + S - 1]),
 // 2 CLIP (keys k > q or k > eot masked)
 struct EncAttnArgs {
-    const float *qkv; int ld, q_off, k_off, v_off;
-    float *out; int ldo;
-    int S, nh, hd;
+    EncParts qkv;
+    half_t *Ap; const float *odiv; int mt;
+    int S, nh;
     float scale;
     int mode;
-    const int32_t *bucket; const float *rel; const int32_t *pad;
+    const float *rel;
+    uint32_t keys[4];
     int eot;
 };
 int launch_enc_attention(const EncAttnArgs &a, hipStream_t st);
-// y[r][c] = gelu_tanh(u[r][c]) * u[r][F + c], u rows of 2F
-int launch_geglu_rows(const float *u, float *y, int rows, int F, hipStream_t st);
-// x[s][:] = tok[ids[s]][:] (+ pos[s][:]); ids on the device, each inside tok's rows
-int launch_embed_rows(const int32_t *ids, const float *tok, const float *pos, float *x, int S, int H, hipStream_t st);
+// packed operand of F columns: quick GELU of the F result columns, or gelu_tanh(column c) * column F + c
+int launch_enc_act(const EncParts &p, bool geglu, half_t *Ap, float *adiv, int rows, int F, hipStream_t st);
+// x[s][:] = tok[ids[s]][:] (+ pos[s][:]); each id inside tok's rows
+struct EncIds {
+    int32_t id[128];
+};
+int launch_embed_rows(const EncIds &ids, const float *tok, const float *pos, float *x, int S, int H, hipStream_t st);
 // dst[i][:] = src[idx[i]][:] for rows x H floats (idx on the device, every entry a valid src row)
 int launch_gather_rows(const float *src, const int32_t *idx, float *dst, int rows, int H, hipStream_t st);
 // out[c] = mean over rows of x[r][c], rows summed in order (src/net.mm Runtime::mean_cols)

@@ -373,11 +373,11 @@ int Runtime::ln_plain(const float *x, float *y, uint32_t S, uint32_t H, float ep
 int Runtime::ln_wb(const float *x, float *y, const float *w, const float *b, uint32_t S, uint32_t H, float eps) {
     TSN_REQUIRE(b, "ln_wb: null bias");
     TSN_TRY(dev.make_current());
-    return launch_enc_norm(x, y, w, b, (int)S, (int)H, eps, true, dev.stream());
+    return launch_enc_norm_rows(x, y, w, b, (int)S, (int)H, eps, true, dev.stream());
 }
 int Runtime::rms_w(const float *x, float *y, const float *w, uint32_t S, uint32_t H, float eps) {
     TSN_TRY(dev.make_current());
-    return launch_enc_norm(x, y, w, nullptr, (int)S, (int)H, eps, false, dev.stream());
+    return launch_enc_norm_rows(x, y, w, nullptr, (int)S, (int)H, eps, false, dev.stream());
 }
 int Runtime::mean_cols(const float *x, float *y, uint32_t S, uint32_t H) {
     TSN_TRY(dev.make_current());
