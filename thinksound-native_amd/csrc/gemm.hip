@@ -1837,7 +1837,7 @@ __global__ __launch_bounds__(512) void gemm_fixup_kernel(const GemmBatch bt) {
 
 // split-K reduction + epilogue, one thread per 4 columns; partials summed in split order
 // (deterministic). EPI_RESID: R[rmap(m)][n] += gate[m/gate_L][n] * (sum + bias[n]);
-// EPI_STORE: Y[ymap(m)][n] = act(sum + bias[n]) as f16 or f32.
+// EPI_STORE: Y[ymap(m)][n] = act(sum + bias[n]) as f16, f16 pairs or f32.
 template <int EPI>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmBatch bt) {
     long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1896,7 +1896,14 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmBatch bt) 
     } else {
         if (P.silu) { v.x = silu_f(v.x); v.y = silu_f(v.y); v.z = silu_f(v.z); v.w = silu_f(v.w); }
         const long long o = rowmap_phys(P.ymap, m) * (long long)P.ldy + n;
-        if (P.y_f16) *(half4 *)((half_t *)P.Y + o) = half4{(half_t)v.x, (half_t)v.y, (half_t)v.z, (half_t)v.w};
+        if (P.y_pair) {
+            const float e[4] = {v.x, v.y, v.z, v.w};
+            half4 hi, lo;
+            split_parts4(e, hi, lo);
+            half_t *y = (half_t *)P.Y + o + pair_col(n) - n;
+            *(half4 *)y = hi;
+            *(half4 *)(y + PAIR) = lo;
+        } else if (P.y_f16) *(half4 *)((half_t *)P.Y + o) = half4{(half_t)v.x, (half_t)v.y, (half_t)v.z, (half_t)v.w};
         else *(float4 *)((float *)P.Y + o) = v;
     }
 }
@@ -1968,14 +1975,12 @@ void gemm_problem_init(GemmProblem &p) {
 // adds its partial sums written and read (about 2.15 MB per 128-row K tile) and split_overhead K tiles.
 static bool hl2_plan(GemmBatch &b, int epi) {
     static const int cost[5] = {0, 281, 375, 470, 562};   // clocks per K tile, by MB / 2
-    bool lo = false;
     int nkmin = 1 << 30;
     for (int i = 0; i < b.nprob; ++i) {
         if (!b.p[i].w_half) return false;
-        lo = lo || b.p[i].y_pair;
         nkmin = std::min(nkmin, b.p[i].K / BK);
     }
-    const bool can_split = b.ws && !lo && (epi == EPI_RESID || epi == EPI_STORE);
+    const bool can_split = b.ws && (epi == EPI_RESID || epi == EPI_STORE);
     double best = 1e30;
     int best_mb = 0, best_s = 1;
     for (int mb = 2; mb <= 8; mb += 2)

@@ -99,8 +99,7 @@ int RefCondModel::create(Runtime *r, const RefCondSpec &sp) {
     TSN_TRY(alloc((size_t)s.sync_S * H * sizeof(float), (void **)&SMID_));
     TSN_TRY(alloc(H * sizeof(float), (void **)&cmean_));
     TSN_TRY(alloc(H * sizeof(float), (void **)&fc_));
-    TSN_TRY(alloc(F * sizeof(float), (void **)&ga_));
-    TSN_TRY(alloc(F * sizeof(float), (void **)&gb_));
+    TSN_TRY(alloc(2 * F * sizeof(float), (void **)&ga_));
     ws_bytes_ = (size_t)40 << 20;
     TSN_TRY(alloc(ws_bytes_, (void **)&ws_));
     TSN_TRY(alloc_skcnt());
@@ -182,8 +181,11 @@ int RefCondModel::upload(const void *host, bool src_f32, size_t numel) {
     TSN_TRY(swiglu_w("text_input_proj.2", 1, &W13t_, &W2t_));
     TSN_TRY(f16w("text_cond_proj.weight", H, s.gtext_dim, 1, &Wtfc_));
     TSN_TRY(f32v("text_cond_proj.bias", H, &btfc_));
-    TSN_TRY(f16w("global_cond_mlp.w1.weight", F, H, 1, &Wg1_));
-    TSN_TRY(f16w("global_cond_mlp.w3.weight", F, H, 1, &Wg3_));
+    half_t *g13;   // [w1; w3]: one GEMV for both
+    TSN_TRY(alloc((size_t)2 * F * H * 2, (void **)&g13));
+    TSN_TRY(prep("global_cond_mlp.w1.weight", F, H, 1, 1, 0, 1, 0, g13, F, 0));
+    TSN_TRY(prep("global_cond_mlp.w3.weight", F, H, 1, 1, 0, 1, 0, g13 + (size_t)F * H, F, 0));
+    Wg13_ = g13;
     TSN_TRY(f16w("global_cond_mlp.w2.weight", H, F, 1, &Wg2_));
     TSN_TRY(rt->dev.sync());
     TSN_TRY(release(wraw_));
@@ -284,9 +286,8 @@ int RefCondModel::enqueue_prep_text_arm(const float *text_cat, const float *gtex
         return run(K_GEMV, 2.0 * N * K, 2.0 * N * K, [&] { return launch_gemv(g, st); });
     };
     TSN_TRY(gemv(Wtfc_, H, s.gtext_dim, gtext, fc_, btfc_, clip_fc));
-    TSN_TRY(gemv(Wg1_, F, H, fc_, ga_, nullptr, nullptr));
-    TSN_TRY(gemv(Wg3_, F, H, fc_, gb_, nullptr, nullptr));
-    TSN_TRY(run("swiglu_kernel", 0, 12.0 * F, [&] { return launch_swiglu(ga_, gb_, ga_, (size_t)F, st); }));
+    TSN_TRY(gemv(Wg13_, 2 * F, H, fc_, ga_, nullptr, nullptr));
+    TSN_TRY(run("swiglu_kernel", 0, 12.0 * F, [&] { return launch_swiglu(ga_, ga_ + F, ga_, (size_t)F, st); }));
     return gemv(Wg2_, H, F, ga_, gcmlp, nullptr, nullptr);
 }
 

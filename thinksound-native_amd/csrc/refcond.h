@@ -58,10 +58,10 @@ private:
     const half_t *Ws0_ = nullptr, *W13s_ = nullptr, *W2s_ = nullptr;
     const half_t *Wc0_ = nullptr, *W13c_ = nullptr, *W2c_ = nullptr, *Wcfc_ = nullptr;
     const half_t *Wt0_ = nullptr, *W13t_ = nullptr, *W2t_ = nullptr, *Wtfc_ = nullptr;
-    const half_t *Wg1_ = nullptr, *Wg3_ = nullptr, *Wg2_ = nullptr;
+    const half_t *Wg13_ = nullptr, *Wg2_ = nullptr;
     const float *bs0_ = nullptr, *bc0_ = nullptr, *bcfc_ = nullptr, *bt0_ = nullptr, *btfc_ = nullptr;
     half_t *IN_ = nullptr, *XA_ = nullptr, *HF_ = nullptr;
-    float *SMID_ = nullptr, *cmean_ = nullptr, *fc_ = nullptr, *ga_ = nullptr, *gb_ = nullptr;
+    float *SMID_ = nullptr, *cmean_ = nullptr, *fc_ = nullptr, *ga_ = nullptr;
     int32_t *idx_ = nullptr;   // sync row gathered for each latent row
     float *ws_ = nullptr;
     size_t ws_bytes_ = 0;
