@@ -512,12 +512,22 @@ __global__ void gather_rows_kernel(const float *src, const int32_t *idx, float *
     for (int c = threadIdx.x; c < H; c += blockDim.x) d[c] = s[c];
 }
 
-// out[c] = (sum over rows r in order of x[r][c]) / rows: one thread per column, fixed order
-__global__ void mean_rows_kernel(const float *x, int rows, int H, float *out) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= H) return;
+// out[c] = (sum over rows of x[r][c]) / rows. A workgroup has 32 columns; group g of 8 sums rows g, g + 8, ...
+// eight loads at a time, and the groups' sums are added in order. (One thread per column, one row after
+// the other, waited for memory once per row on 4 CUs: 64 x 1024 16.1 us.)
+__global__ __launch_bounds__(256) void mean_rows_kernel(const float *x, int rows, int H, float *out) {
+    __shared__ float part[8][32];
+    const int l = threadIdx.x & 31, g = threadIdx.x >> 5, c = blockIdx.x * 32 + l;
     float acc = 0.0f;
-    for (int r = 0; r < rows; ++r) acc += x[(long long)r * H + c];
+    if (c < H) {
+#pragma unroll 8
+        for (int r = g; r < rows; r += 8) acc += x[(long long)r * H + c];
+    }
+    part[g][l] = acc;
+    __syncthreads();
+    if (g > 0 || c >= H) return;
+#pragma unroll
+    for (int i = 1; i < 8; ++i) acc += part[i][l];
     out[c] = acc / (float)rows;
 }
 
@@ -526,9 +536,16 @@ __global__ void silu_kernel(float *x, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) x[i] = x[i] / (1.0f + expf(-x[i]));
 }
+// VEC: four floats a thread (16-byte aligned x and y), the last n % 4 by one further thread. 6504448 floats:
+// 13.7 us with one float a thread.
+template <bool VEC>
 __global__ void copy_kernel(const float *x, float *y, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) y[i] = x[i];
+    if constexpr (VEC) {
+        if (i < n / 4) ((float4 *)y)[i] = ((const float4 *)x)[i];
+        else if (i == n / 4)
+            for (size_t k = i * 4; k < n; ++k) y[k] = x[k];
+    } else if (i < n) y[i] = x[i];
 }
 __global__ void swiglu_kernel(const float *a, const float *b, float *y, size_t n) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -964,7 +981,7 @@ int launch_gather_rows(const float *src, const int32_t *idx, float *dst, int row
 }
 int launch_mean_rows(const float *x, int rows, int H, float *out, hipStream_t st) {
     TSN_REQUIRE(x && out && rows > 0 && H > 0, "mean_rows: arguments");
-    TSN_LAUNCH(mean_rows_kernel, dim3((H + 255) / 256), dim3(256), 0, st, x, rows, H, out);
+    TSN_LAUNCH(mean_rows_kernel, dim3((H + 31) / 32), dim3(256), 0, st, x, rows, H, out);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
@@ -978,7 +995,8 @@ int launch_silu(float *x, size_t n, hipStream_t st) {
 int launch_copy(const float *x, float *y, size_t n, hipStream_t st) {
     TSN_REQUIRE((x && y) || n == 0, "copy: null");
     if (n == 0) return TSN_OK;
-    TSN_LAUNCH(copy_kernel, dim3(blocks_for(n)), dim3(256), 0, st, x, y, n);
+    if (((((uintptr_t)x) | ((uintptr_t)y)) & 15) == 0) TSN_LAUNCH(copy_kernel<true>, dim3(blocks_for(n / 4 + 1)), dim3(256), 0, st, x, y, n);
+    else TSN_LAUNCH(copy_kernel<false>, dim3(blocks_for(n)), dim3(256), 0, st, x, y, n);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
