@@ -460,3 +460,46 @@ def test_launcher_surface_rest(tsn, rt, orc):
     dd = rt.array(dst0)
     rt.qkv_split3(rt.array(src), dd, rows, Hq, off); rt.sync()
     assert np.array_equal(dd.numpy(), orc.qkv_split3(src, dst0, off))
+
+
+@pytest.mark.parametrize("S", [1, 63, 64, 65, 130])
+def test_attention_pack_alignment(tsn, rt, S):
+    """The operand packing with 16-byte loads and with single ones (odd strides and offsets): the same
+    values in both layouts give bit-identical outputs."""
+    nh, H = 3, 192
+    q = rng(S).standard_normal((S, 3 * H)).astype(np.float32)
+    odd = np.zeros((S, 3 * H + 7), np.float32)
+    for i, off in enumerate((1, H + 3, 2 * H + 6)):
+        odd[:, off:off + H] = q[:, i * H:(i + 1) * H]
+    a, b = rt.empty((S, H)), rt.empty((S, H))
+    rt.attention(rt.array(q), a, S, nh, 64, 3 * H, H, 0, H, 2 * H, 0, 0.125)
+    rt.attention(rt.array(odd), b, S, nh, 64, 3 * H + 7, H, 1, H + 3, 2 * H + 6, 0, 0.125)
+    rt.sync()
+    assert np.array_equal(a.numpy().view(np.uint32), b.numpy().view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 1023, 1024, 1027])
+def test_copy_and_mean_edges(tsn, rt, n):
+    """Copies of every n % 4 at 16-byte and 4-byte alignment that leave the element after them alone; row
+    means around the groups of 8 rows and 32 columns. The mean of n f32 values: n roundings of 2^-24."""
+    x = rng(n).standard_normal(n + 5).astype(np.float32)
+    dx = rt.array(x)
+
+    class At:
+        def __init__(self, arr, elems):
+            self.p = arr.offset(elems)
+
+    for off in (0, 1):
+        y = rt.array(np.full(n + 5, 7.0, np.float32))
+        rt.copy(At(dx, off), At(y, off), n)
+        rt.sync()
+        got = y.numpy()
+        assert np.array_equal(got[off:off + n], x[off:off + n])
+        assert np.all(got[:off] == 7.0) and np.all(got[off + n:] == 7.0)
+    for rows, H in ((1, n), (7, 33), (8, 32), (9, 31), (n, 40)):
+        m = rng(rows + H).standard_normal((rows, H)).astype(np.float32)
+        out = rt.empty((H,))
+        rt.mean_cols(rt.array(m), out, rows, H)
+        rt.sync()
+        bound = rows * 2.0 ** -24 * np.abs(m).mean(0) + 1e-7 * np.abs(m.mean(0))
+        assert np.all(np.abs(out.numpy() - m.astype(np.float64).mean(0)) <= bound + 1e-30)
