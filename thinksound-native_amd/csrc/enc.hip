@@ -347,64 +347,59 @@ constexpr int EA_HD = 64;
 constexpr int EA_PP = EA_SMAX + 4;   // pitches (floats): the four k groups and sixteen rows or columns that
 constexpr int EA_VP = EA_HD + 16;    // one MFMA operand read touches lie in distinct banks
 
-// One workgroup of four waves per (16 queries, head), everything in f32 (v_mfma_f32_16x16x4_f32, f32
-// softmax). Wave w computes the scores of key blocks w and w + 4 (16 keys each) straight from the QKV
-// GEMM's splits, then the output columns 16 w .. + 15. The 64 products of a score run over d = 16 kq + i
-// so that a lane's share of a q or k row is 64 contiguous bytes. The kernel is latency-bound (77 keys:
-// at most 52 MFMAs a wave), so the loads of q, k and V of every split go out in one sequence,
-// so that all of them wait together (once per 4 splits): MT 16-key blocks at most.
+// One workgroup per (16 queries, head), everything in f32 (v_mfma_f32_16x16x4_f32, f32 softmax). Wave w
+// computes the scores of key block w (16 keys, MT of them at most) with k straight from the QKV GEMM's
+// splits, then waves 0 to 3 the output columns 16 w .. + 15. The 64 products of a score run over
+// d = 16 kq + i, so a lane's share of a k row is 64 contiguous bytes. The kernel is as long as its loads
+// (77 keys, 4 splits: four waves with two key blocks and a q tile each 11.8 us, nine loads a thread and
+// split instead of seventeen 9.2 us): q, k and v of up to 4 splits go out in one sequence.
 template <int MT>
-__global__ __launch_bounds__(256, 1) void enc_attn_kernel(const EncAttnArgs a) {
-    constexpr int KB = (MT + 3) / 4;   // key blocks of a wave
+__global__ __launch_bounds__(64 * (MT < 4 ? 4 : MT), 1) void enc_attn_kernel(const EncAttnArgs a) {
+    constexpr int NW = MT < 4 ? 4 : MT, NT = 64 * NW, VR = 256 * MT / NT;   // waves, threads, v rows of a thread
+    constexpr int QP = EA_HD + 4;
     __shared__ __attribute__((aligned(16))) float Vs[16 * MT * EA_VP];
     __shared__ __attribute__((aligned(16))) float P[EA_Q * EA_PP];
+    __shared__ __attribute__((aligned(16))) float Qs[EA_Q * QP];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, kq = lane >> 4;
     // workgroups go to the 8 XCDs in turn: the query tiles of a head run on one XCD, whose L2 then serves
     // the head's k and v to all but the first of them
     const int S = a.S, H = a.nh * EA_HD, N = 3 * H, nkb = (S + 15) >> 4, idx = blockIdx.x >> 3;
     const int h = idx / nkb * 8 + (blockIdx.x & 7), q0 = idx % nkb * EA_Q;
     if (h >= a.nh) return;
-    // q row q0 + r16 and k rows 16 kb + r16, columns 16 kq .. + 15 of the head; V: 4 columns of rows
-    // tid / 16 + 16 i. Rows past the context repeat its last one: masked, or never stored.
-    constexpr int NV = 4 + 4 * KB + MT;
+    // q and v: 4 columns of row tid / 16 (of 16; + 4 NW i), k: columns 16 kq .. + 15 of row 16 wave + r16. Rows
+    // past the context repeat its last one: masked, or never stored.
+    constexpr int NV = 5 + VR;
     int off[NV];
     float4 x[NV];
-    const int ch = h * EA_HD + 16 * kq, cv = 2 * H + h * EA_HD + (tid & 15) * 4;
+    const int c4 = h * EA_HD + (tid & 15) * 4, ck = H + h * EA_HD + 16 * kq, cv = 2 * H + c4;
+    off[0] = min(q0 + ((tid >> 4) & 15), S - 1) * N + c4;
 #pragma unroll
-    for (int i = 0; i < 4 + 4 * KB; ++i) {
-        const int row = i < 4 ? q0 + r16 : 16 * (wave + 4 * (i / 4 - 1)) + r16;
-        off[i] = min(row, S - 1) * N + (i < 4 ? 0 : H) + ch + 4 * (i & 3);
+    for (int i = 0; i < 4; ++i) off[1 + i] = min(16 * wave + r16, S - 1) * N + ck + 4 * i;
+#pragma unroll
+    for (int i = 0; i < VR; ++i) off[5 + i] = min((tid >> 4) + 4 * NW * i, S - 1) * N + cv;
+    float4 bias[6];   // CLIP: q's, k's and v's columns
+    if (a.qkv.bias) {
+        bias[0] = *(const float4 *)(a.qkv.bias + c4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) bias[1 + i] = *(const float4 *)(a.qkv.bias + ck + 4 * i);
+        bias[5] = *(const float4 *)(a.qkv.bias + cv);
     }
-#pragma unroll
-    for (int i = 0; i < MT; ++i) off[4 + 4 * KB + i] = min((tid >> 4) + 16 * i, S - 1) * N + cv;
-    float4 bias[3][4];   // CLIP: q and k columns, and V's (bias[2][0])
+    parts_sum<NV, 4>(a.qkv, off, x);
     if (a.qkv.bias) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            bias[0][i] = *(const float4 *)(a.qkv.bias + ch + 4 * i);
-            bias[1][i] = *(const float4 *)(a.qkv.bias + H + ch + 4 * i);
-        }
-        bias[2][0] = *(const float4 *)(a.qkv.bias + cv);
+        for (int i = 0; i < NV; ++i) x[i] = add4(x[i], bias[i < 5 ? i : 5]);
     }
-    parts_sum<NV, MT <= 5 ? 4 : 2>(a.qkv, off, x);
-    if (a.qkv.bias) {
+    if (tid < 256) *(float4 *)&Qs[(tid >> 4) * QP + (tid & 15) * 4] = x[0];
 #pragma unroll
-        for (int i = 0; i < 4 + 4 * KB; ++i) x[i] = add4(x[i], bias[i < 4 ? 0 : 1][i & 3]);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) x[4 + 4 * KB + i] = add4(x[4 + 4 * KB + i], bias[2][0]);
-    }
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-        *(float4 *)&Vs[((tid >> 4) + 16 * i) * EA_VP + (tid & 15) * 4] = x[4 + 4 * KB + i];
+    for (int i = 0; i < VR; ++i) *(float4 *)&Vs[((tid >> 4) + 4 * NW * i) * EA_VP + (tid & 15) * 4] = x[5 + i];
+    __syncthreads();
     const int q = q0 + r16;
-#pragma unroll
-    for (int b = 0; b < KB; ++b) {
-        const int kb = wave + 4 * b;
-        if (kb >= nkb) break;
+    if (wave < nkb) {
+        const int kb = wave;
         floatx4_t s = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float4 kv = x[4 + 4 * b + i], qv = x[i];
+            const float4 kv = x[1 + i], qv = *(const float4 *)&Qs[r16 * QP + 16 * kq + 4 * i];
             s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.x, qv.x, s, 0, 0, 0);
             s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.y, qv.y, s, 0, 0, 0);
             s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv.z, qv.z, s, 0, 0, 0);
@@ -427,10 +422,9 @@ __global__ __launch_bounds__(256, 1) void enc_attn_kernel(const EncAttnArgs a) {
         *(floatx4_t *)&P[r16 * EA_PP + 16 * kb + 4 * kq] = s;
     }
     __syncthreads();
-    // softmax: wave w takes queries 4 w .. + 3, one lane per key and 64 keys at a time
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        float *pr = P + (4 * wave + r) * EA_PP;
+    // softmax: wave w takes queries w, w + NW, ..., one lane per key and 64 keys at a time
+    for (int r = wave; r < EA_Q; r += NW) {
+        float *pr = P + r * EA_PP;
         const int n = nkb * 16;
         const float s0 = lane < n ? pr[lane] : -INFINITY, s1 = lane + 64 < n ? pr[lane + 64] : -INFINITY;
         const float mx = wave_max(fmaxf(s0, s1));
@@ -440,6 +434,7 @@ __global__ __launch_bounds__(256, 1) void enc_attn_kernel(const EncAttnArgs a) {
         if (lane + 64 < n) pr[lane + 64] = e1 * inv;
     }
     __syncthreads();
+    if (wave >= 4) return;
     // V^T is the first operand: a lane holds columns 16 wave + 4 kq .. + 3 of query q
     floatx4_t o[2] = {floatx4_t{0.f, 0.f, 0.f, 0.f}, floatx4_t{0.f, 0.f, 0.f, 0.f}};
     for (int kb = 0; kb < nkb; ++kb)
@@ -599,11 +594,11 @@ int launch_enc_attention(const EncAttnArgs &a, hipStream_t st) {
     TSN_REQUIRE(a.qkv.ws && a.Ap && a.odiv && a.S > 0 && a.S <= EA_SMAX && a.nh > 0 && a.qkv.N == 3 * EA_HD * a.nh,
                 "enc_attention: context 1..128, rows of q, k and v with heads of 64");
     TSN_REQUIRE((a.mode == 1 && a.rel) || a.mode == 2, "enc_attention: mode and tables");
-    const dim3 grid((a.nh + 7) / 8 * 8 * ((a.S + EA_Q - 1) / EA_Q)), block(256);
+    const dim3 grid((a.nh + 7) / 8 * 8 * ((a.S + EA_Q - 1) / EA_Q));
     const int mt = enc_row_blocks(a.S);
-    if (mt == 2) TSN_LAUNCH(enc_attn_kernel<2>, grid, block, 0, st, a);
-    else if (mt == 5) TSN_LAUNCH(enc_attn_kernel<5>, grid, block, 0, st, a);
-    else TSN_LAUNCH(enc_attn_kernel<8>, grid, block, 0, st, a);
+    if (mt == 2) TSN_LAUNCH(enc_attn_kernel<2>, grid, dim3(256), 0, st, a);
+    else if (mt == 5) TSN_LAUNCH(enc_attn_kernel<5>, grid, dim3(320), 0, st, a);
+    else TSN_LAUNCH(enc_attn_kernel<8>, grid, dim3(512), 0, st, a);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
