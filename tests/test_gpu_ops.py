@@ -503,3 +503,20 @@ def test_copy_and_mean_edges(tsn, rt, n):
         rt.sync()
         bound = rows * 2.0 ** -24 * np.abs(m).mean(0) + 1e-7 * np.abs(m.mean(0))
         assert np.all(np.abs(out.numpy() - m.astype(np.float64).mean(0)) <= bound + 1e-30)
+
+
+@pytest.mark.parametrize("M", [1, 31, 33, 64, 65, 96, 97, 128, 129])
+@pytest.mark.parametrize("N,K", [(8, 64), (128, 128), (136, 1088), (1024, 4096)])
+def test_gemm_hilo_one_round_edges(tsn, rt, M, N, K):
+    """One-round hi|lo grids around the 32- to 128-row tiles, one K step, an odd number of steps, a ragged
+    column tile and (N = 1024) K splits. Against 64 bits: the parts carry 22 bits (2.4e-7 of a value),
+    and 32-bit sums of K / 32 terms add less than 3e-7 here."""
+    r = rng(M * 7 + K)
+    X = r.standard_normal((M, K)).astype(np.float32)
+    W = (r.standard_normal((N, K)) * 0.03).astype(np.float16)
+    b = r.standard_normal(N).astype(np.float32)
+    Y = rt.empty((M, N))
+    rt.gemm(tsn.F16, rt.array(W), rt.array(X), tsn.F32, Y, tsn.F32, rt.array(b), M, N, K)
+    rt.sync()
+    ref = X.astype(np.float64) @ W.astype(np.float64).T + b
+    assert rel_l2(Y.numpy(), ref) < 1e-6
