@@ -152,8 +152,9 @@ std::vector<ManifestEntry> t5_manifest(const T5Spec &s) {
     return v;
 }
 
-// K splits of a QKV GEMM: attention reads every split of k and v in each of a head's workgroups (77 rows,
-// 1024 wide: attention 11.8 us with 4 splits when it was measured against 8.5 with 2, the GEMM 1.6 us less)
+// K splits of a QKV GEMM: attention reads every split of k and v in each of a head's workgroups. 77 rows, 1024
+// wide: 4 splits 1.48 ms a prompt, 2 splits 1.51 (the GEMM 9.2 -> 10.8 us); 2048 wide: 2.27 ms with 4 and 2,
+// 2.30 with 5.
 constexpr int QKV_SPLITS = 4;
 
 int EncoderRunner::create_common(int ctx, int width, int ffn, int layers) {
