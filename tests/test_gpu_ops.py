@@ -520,3 +520,34 @@ def test_gemm_hilo_one_round_edges(tsn, rt, M, N, K):
     rt.sync()
     ref = X.astype(np.float64) @ W.astype(np.float64).T + b
     assert rel_l2(Y.numpy(), ref) < 1e-6
+
+
+@pytest.mark.parametrize("ln", [False, True])
+def test_weighted_norm_past_2_31_floats(tsn, rt, orc, ln):
+    """Norm rows whose element offset needs more than 31 bits (8 GiB of f32 rows): the first and the last
+    rows equal the same rows normalised by themselves."""
+    H, rows, n = 2048, (1 << 20) + 3, 4
+
+    class At:
+        def __init__(self, arr, elems):
+            self.p = arr.offset(elems)
+
+    r = rng(81 + ln)
+    x = r.standard_normal((n, H)).astype(np.float32)
+    w, b = rt.array(r.standard_normal(H).astype(np.float32)), rt.array(r.standard_normal(H).astype(np.float32))
+    small, out = rt.array(x), rt.empty((n, H))
+    big = rt.empty((rows, H))
+    try:
+        norm = (lambda a, y, S: rt.ln_wb(a, y, w, b, S, H, 1e-5)) if ln else (lambda a, y, S: rt.rms_w(a, y, w, S, H, 1e-6))
+        norm(small, out, n)
+        for first in (0, rows - n):
+            rt.copy(small, At(big, first * H), n * H)
+        norm(big, big, rows)   # in place: a row is read whole before it is written
+        rt.sync()
+        want = out.numpy()
+        for first in (0, rows - n):
+            rt.copy(At(big, first * H), out, n * H)
+            rt.sync()
+            assert np.array_equal(out.numpy().view(np.uint32), want.view(np.uint32)), first
+    finally:
+        big.free()

@@ -269,14 +269,14 @@ __global__ __launch_bounds__(256) void enc_norm_kernel(const EncNormArgs a) {
     // the row in registers: columns 4*tid + 1024*j .. + 3; all loads ahead of the first barrier
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 v[NJ], wv[NJ], bv[NJ];
-    int off[NJ];
+    int off[NJ];   // of the GEMM's result, at most 128 rows; x and y may have any number (launch_enc_norm_rows)
     bool in[NJ];
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const int c = 4 * tid + 1024 * j;
         in[j] = c < H;
-        off[j] = row * H + (in[j] ? c : 0);
+        off[j] = a.parts.ws ? row * H + (in[j] ? c : 0) : 0;
         v[j] = in[j] ? *(const float4 *)(a.x + (long long)row * H + c) : zero;
         wv[j] = in[j] ? *(const float4 *)(a.w + c) : zero;
         bv[j] = LN && in[j] ? *(const float4 *)(a.b + c) : zero;
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(256) void enc_norm_kernel(const EncNormArgs a) {
     } else {
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
-            if (in[j]) *(float4 *)(a.y + off[j]) = o[j];
+            if (in[j]) *(float4 *)(a.y + (long long)row * H + 4 * tid + 1024 * j) = o[j];
     }
 }
 
@@ -570,7 +570,7 @@ int launch_enc_gemm(EncGemmArgs &g, hipStream_t st) {
 
 int launch_enc_norm(const EncNormArgs &a, bool ln, hipStream_t st) {
     TSN_REQUIRE(a.x && a.w && (a.y || a.Ap) && a.rows > 0 && a.H > 0 && (!ln || a.b), "enc_norm: arguments");
-    TSN_REQUIRE(!a.parts.ws || (a.xout && a.parts.splits > 0 && a.parts.N == a.H), "enc_norm: partial sums");
+    TSN_REQUIRE(!a.parts.ws || (a.xout && a.rows <= 128 && a.parts.splits > 0 && a.parts.N == a.H), "enc_norm: partial sums");
     TSN_REQUIRE(!a.Ap || (a.adiv && a.rows <= 128 && a.H % 32 == 0), "enc_norm: packed rows");
     TSN_REQUIRE(a.H % 4 == 0 && a.H <= 2048 && aligned16(a.x) && aligned16(a.y) && aligned16(a.w) && aligned16(a.b),
                 "enc_norm: rows of at most 2048 floats, a multiple of 4, 16-byte aligned");
