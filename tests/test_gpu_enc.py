@@ -179,3 +179,23 @@ def test_encoder_gemm_edges(tsn, rt, orc, ctx, scale):
     finally:
         t.close()
         c.close()
+
+
+@pytest.mark.parametrize("ctx,d_ff", [(128, 32768), (128, 32800), (77, 65536)])
+def test_t5_wide_ffn(tsn, rt, orc, ctx, d_ff):
+    """FFN widths around and past the point where one [ctx][2 d_ff] result fills 32 MB: any multiple of 32 is
+    accepted."""
+    spec = tsn.t5_spec_default().copy(d=64, d_ff=d_ff, NL=1, NH=1, ctx=ctx, vocab=50)
+    w = tsn.t5_synth_weights(spec, 41)
+    ids = rng(ctx).integers(1, 50, ctx).astype(np.int32)
+    m = tsn.T5Model(rt, spec)
+    try:
+        m.upload_weights(w)
+        out = rt.empty((ctx, spec.d))
+        m.encode(ids, out)
+        rt.sync()
+        e = rel_l2(out.numpy(), orc.t5_encode(spec.as_dict(), w, ids))
+        print("t5 d_ff %d: %.3g" % (d_ff, e))
+        assert e <= 3e-6   # f32 against f32, one layer
+    finally:
+        m.close()

@@ -456,15 +456,16 @@ __global__ __launch_bounds__(64 * (MT < 4 ? 4 : MT), 1) void enc_attn_kernel(con
 // c) * column F + c (GEGLU; tanh form, argument clamped to +-10: shaders/ops_conv.metal:15-24). A thread
 // has 4 columns of every 4096; those past the first 8192 are computed again when the scale is known.
 template <bool GEGLU>
-__global__ __launch_bounds__(1024) void enc_act_kernel(const EncParts p, half_t *Ap, float *adiv, int mt, int F) {
+__global__ __launch_bounds__(1024) void enc_act_kernel(EncParts p, half_t *Ap, float *adiv, int mt, int F) {
     __shared__ float part[16];
     const int tid = threadIdx.x, m = blockIdx.x;
+    p.ws += (long long)m * p.N;
     auto act = [&](int c) {
         constexpr int NV = GEGLU ? 2 : 1;
         int off[NV];
         float4 u[NV];
 #pragma unroll
-        for (int i = 0; i < NV; ++i) off[i] = m * p.N + i * F + c;
+        for (int i = 0; i < NV; ++i) off[i] = i * F + c;
         parts_sum<NV, 4>(p, off, u);
         if (p.bias) {
 #pragma unroll

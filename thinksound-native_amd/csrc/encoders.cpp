@@ -157,18 +157,19 @@ std::vector<ManifestEntry> t5_manifest(const T5Spec &s) {
 // 2.30 with 5.
 constexpr int QKV_SPLITS = 4;
 
-int EncoderRunner::create_common(int ctx, int width, int ffn, int layers) {
+int EncoderRunner::create_common(int ctx, int width, int ffn, int ffn_cols, int layers) {
     TSN_TRY(alloc(enc_operand_bytes(ctx, width), (void **)&A_));
     TSN_TRY(alloc(enc_operand_bytes(ctx, ffn), (void **)&F_));
     TSN_TRY(alloc((size_t)ctx * 4, (void **)&adiv_));
     TSN_TRY(alloc((size_t)ctx * 4, (void **)&fdiv_));
     TSN_TRY(alloc((size_t)layers * ctx * 4, (void **)&odiv_));
-    return alloc(ENC_WS_BYTES, (void **)&ws_);
+    ws_bytes_ = std::max(ENC_WS_BYTES, (size_t)ctx * std::max(3 * (size_t)width, (size_t)ffn_cols) * sizeof(float));
+    return alloc(ws_bytes_, (void **)&ws_);
 }
 
 int EncoderRunner::gemm(const half_t *A, const float *adiv, const EncWeight &W, const float *b, int M, int N, int K,
                         EncParts &out, int most) {
-    EncGemmArgs g{A, adiv, W.w, W.div, ws_, ENC_WS_BYTES, M, N, K, most, 1, 0};
+    EncGemmArgs g{A, adiv, W.w, W.div, ws_, ws_bytes_, M, N, K, most, 1, 0};
     TSN_TRY(run("enc_gemm_kernel", 2.0 * M * N * K, 4.0 * ((double)N * K + M * (double)N + M * (double)K),
                 [&] { return launch_enc_gemm(g, rt->dev.stream()); }));
     out = EncParts{ws_, (long long)M * N, g.splits, N, b};
@@ -223,7 +224,7 @@ int ClipModel::create(Runtime *r, const ClipSpec &sp) {
     s = sp;
     const size_t n = s.ctx, H = s.H;
     TSN_TRY(alloc(n * H * 4, (void **)&X_));
-    return create_common(s.ctx, s.H, 4 * s.H, s.NL);
+    return create_common(s.ctx, s.H, 4 * s.H, 4 * s.H, s.NL);
 }
 
 int ClipModel::upload_weights(const float *host, size_t numel) { return upload(host, numel); }
@@ -347,7 +348,7 @@ int T5Model::create(Runtime *r, const T5Spec &sp) {
     const size_t n = s.ctx, d = s.d;
     TSN_TRY(alloc(n * d * 4, (void **)&X_));
     TSN_TRY(alloc((2 * n - 1) * s.NH * 4, (void **)&rel_));
-    return create_common(s.ctx, s.d, s.d_ff, s.NL);
+    return create_common(s.ctx, s.d, s.d_ff, 2 * s.d_ff, s.NL);
 }
 
 int T5Model::upload_weights(const float *host, size_t numel) { return upload(host, numel); }

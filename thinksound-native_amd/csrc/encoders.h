@@ -16,7 +16,7 @@
 
 namespace tsn {
 
-constexpr size_t ENC_WS_BYTES = (size_t)32 << 20;   // K-split sums of one GEMM
+constexpr size_t ENC_WS_BYTES = (size_t)32 << 20;   // K-split sums of one GEMM: at least this, and one sum of the widest
 
 struct ClipSpec {   // field meaning documented in include/tsn.h (tsn_clip_spec)
     int H, NL, NH, ctx, vocab;
@@ -45,11 +45,13 @@ struct EncWeight {   // a packed [N][K] weight and its row divisors
 
 class EncoderRunner : public GraphRunner {
 protected:
-    float *ws_ = nullptr;                        // ENC_WS_BYTES
+    float *ws_ = nullptr;                        // ws_bytes_
+    size_t ws_bytes_ = 0;
     half_t *A_ = nullptr, *F_ = nullptr;         // packed GEMM operands: width and FFN columns
     float *adiv_ = nullptr, *fdiv_ = nullptr;    // their row divisors
     float *odiv_ = nullptr;                      // [layers][ctx] divisors of the attention outputs
-    int create_common(int ctx, int width, int ffn, int layers);
+    // ffn_cols: columns of the first FFN GEMM's result
+    int create_common(int ctx, int width, int ffn, int ffn_cols, int layers);
     // out = A·Wᵀ (+ b) as K-split sums in ws_, for the next kernel to read
     int gemm(const half_t *A, const float *adiv, const EncWeight &W, const float *b, int M, int N, int K, EncParts &out,
              int most = 1 << 20);
