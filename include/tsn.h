@@ -345,7 +345,8 @@ int tsn_vae_profile_decode(tsn_vae *v, const float *latent, float *audio, tsn_ke
                            int *n_stats);
 
 /* ---------------- text encoders: tn::ClipModel, tn::T5Model (src/models.h:24-52) ----------------
- * f32 throughout, as the reference loads both (src/clip.cpp:7, src/t5.cpp:22): GEMMs on f16 hi + lo pairs, f32
+ * f32 throughout, as the reference loads both (src/clip.cpp:7, src/t5.cpp:22): GEMMs on the bf16 MFMA with every
+ * f32 operand as the exact sum of three bf16 parts, f32
  * attention over the 77-token context. ids are host arrays (the reference's std::vector<int32_t>);
  * outputs are device pointers enqueued on the runtime's stream. */
 typedef struct {

@@ -199,3 +199,67 @@ def test_t5_wide_ffn(tsn, rt, orc, ctx, d_ff):
         assert e <= 3e-6   # f32 against f32, one layer
     finally:
         m.close()
+
+
+def _views(manifest, w):
+    """name -> writable flat view of w"""
+    return {n: w[o:o + k] for n, k, o in manifest}
+
+
+@pytest.mark.parametrize("ctx", [9, 77, 100])
+@pytest.mark.parametrize("k", [-20, 14, 20, 40])
+def test_encoders_keep_f32_operands(tsn, rt, ctx, k):
+    """Powers of two moved between the two operands of a product (a channel of a norm weight or of a hidden row
+    against its column of the next weight, the v rows of a head against its columns of the output
+    projection, q rows against k rows) leave every f32 product and sum as it was, so the encoders'
+    outputs stay the same to the last bit, whatever the range of values inside a row: no operand is held
+    in fewer than 24 bits or in a narrower range."""
+    f = np.float32(2.0) ** k
+    inv = np.float32(1.0) / f
+    ts = tsn.t5_spec_default().copy(d=192, d_ff=352, NL=2, NH=3, ctx=ctx, vocab=200)
+    cs = tsn.clip_spec_default().copy(H=192, NL=2, NH=3, ctx=ctx, vocab=300)
+    tw, cw = tsn.t5_synth_weights(ts, 51).copy(), tsn.clip_synth_weights(cs, 52).copy()
+    tw2, cw2 = tw.copy(), cw.copy()
+    t, c = _views(tsn.t5_manifest(ts), tw2), _views(tsn.clip_manifest(cs), cw2)
+    for l in range(2):
+        b = "blk.%d." % l
+        for norm, nexts, ch in ((".attn_norm", ("q", "k", "v"), 5), (".ffn_norm", ("wi_0", "wi_1"), 70)):
+            t[b[:-1] + norm][ch] *= f
+            for n in nexts:
+                t[b + n].reshape(-1, ts.d)[:, ch] *= inv
+        t[b + "wi_1"].reshape(-1, ts.d)[11] *= f                 # one hidden channel of the GEGLU's linear half
+        t[b + "wo"].reshape(-1, ts.d_ff)[:, 11] *= inv
+        t[b + "v"].reshape(-1, ts.d)[64:128] *= inv              # head 1
+        t[b + "o"].reshape(-1, ts.d)[:, 64:128] *= f
+        t[b + "k"].reshape(-1, ts.d)[:64] *= inv                 # head 0
+        t[b + "q"].reshape(-1, ts.d)[:64] *= f
+        for n in ("ln1.w", "ln1.b"):
+            c[b + n][7] *= f
+        for n in ("q.w", "k.w", "v.w"):
+            c[b + n].reshape(-1, cs.H)[:, 7] *= inv
+        for n in ("ln2.w", "ln2.b"):
+            c[b + n][100] *= f
+        c[b + "fc1.w"].reshape(-1, cs.H)[:, 100] *= inv
+        c[b + "v.w"].reshape(-1, cs.H)[128:] *= inv              # head 2
+        c[b + "v.b"][128:] *= inv
+        c[b + "out.w"].reshape(-1, cs.H)[:, 128:] *= f
+    r = rng(ctx)
+    tids, cids = r.integers(2, 200, ctx).astype(np.int32), r.integers(0, 300, ctx).astype(np.int32)
+    outs = []
+    for a, d in ((tw, cw), (tw2, cw2)):
+        tm, cm = tsn.T5Model(rt, ts), tsn.ClipModel(rt, cs)
+        try:
+            tm.upload_weights(a)
+            cm.upload_weights(d)
+            out, pt, g = rt.empty((ctx, ts.d)), rt.empty((ctx, cs.H)), rt.empty((cs.H,))
+            tm.encode(tids, out)
+            cm.encode(cids, pt, g)
+            rt.sync()
+            outs.append((out.numpy(), pt.numpy(), g.numpy()))
+        finally:
+            tm.close()
+            cm.close()
+    e = [rel_l2(y, x) for x, y in zip(*outs)]
+    print("ctx %d 2^%d: t5 %.3g clip %.3g pooled %.3g" % ((ctx, k) + tuple(e)))
+    for x, y in zip(*outs):
+        assert np.isfinite(x).all() and np.array_equal(x.view(np.uint32), y.view(np.uint32))

@@ -1,9 +1,9 @@
-// enc.hip — kernels of the text encoders (src/clip.cpp, src/t5.cpp): f32-accurate GEMM over streamed f32
-// weights, LayerNorm with weight and bias, RMSNorm with weight, attention over one short context with the
+// enc.hip — kernels of the text encoders (src/clip.cpp, src/t5.cpp): f32 GEMM over streamed f32 weights,
+// LayerNorm with weight and bias, RMSNorm with weight, attention over one short context with the
 // CLIP causal/EOT mask or the T5 bucketed relative bias and padding mask, quick GELU / GEGLU, and the
-// token (+ position) embedding gather. GEMM operands are pairs of f16 parts (hi + lo) of values scaled by
-// a power of two, per row of activations and per row of a weight, because T5's activations leave the
-// f16 range; everything else is f32.
+// token (+ position) embedding gather. GEMM operands are sums of three bf16 parts, which hold all 24 bits of
+// an f32 value over f32's range of exponents (T5's activations leave the f16 range, and a row's values
+// may lie any number of powers of two apart); everything else is f32.
 //
 // Per layer: norm -> QKV GEMM -> attention -> out GEMM -> norm -> FFN GEMM -> activation -> FFN GEMM.
 // A GEMM leaves the raw sums of its K splits in the workspace; the kernel that reads them adds the
@@ -23,34 +23,44 @@ namespace {
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 typedef unsigned uintx4_t __attribute__((ext_vector_type(4)));
 
-// 2^(e - 14) for 2^e <= v < 2^(e + 1): a row of largest magnitude v divided by it lies below 2^15, and
-// parts of its values down to 2^-16 of the largest are exact to 22 bits (smaller ones to 2^-39 of the
-// largest). Zero and denormal rows take the smallest exponent that keeps the divisor's reciprocal finite.
-__device__ __forceinline__ float row_divisor(float v) {
-    return __uint_as_float((max(__float_as_uint(v) >> 23, 32u) - 14u) << 23);
-}
-__device__ __forceinline__ float pow2_recip(float v) { return __uint_as_float((254u << 23) - __float_as_uint(v)); }
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float floatx2_t __attribute__((ext_vector_type(2)));
 
-// A GEMM operand with M <= 16 mt rows, packed for enc_gemm_kernel: per 32-wide K step the hi and the lo
-// parts one after the other, each mt blocks of 16 rows x 32 columns (1 KB). A block is the 64 16-byte
+// The three parts of N values: p[0] = bf16(v), p[1] = bf16(v - p[0]), p[2] = the rest, exact (8 + 8 + 8 bits).
+// Two values a 32-bit word.
+template <int N>
+__device__ __forceinline__ void split_bf16(const float (&v)[N], unsigned (&p)[3][N / 2]) {
+#pragma unroll
+    for (int e = 0; e < N; e += 2) {
+        floatx2_t r = {v[e], v[e + 1]};
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector(r, bf16x2_t));
+            p[c][e / 2] = u;
+            r[0] -= __uint_as_float(u << 16);
+            r[1] -= __uint_as_float(u & 0xFFFF0000u);
+        }
+    }
+}
+
+// A GEMM operand with M <= 16 mt rows, packed for enc_gemm_kernel: per 32-wide K step the three parts one
+// after the other, each mt blocks of 16 rows x 32 columns (1 KB). A block is the 64 16-byte
 // operands of one MFMA: row r (0..15), columns 8 kq .. + 7 (kq 0..3) at slot 4 r + (kq ^ (r / 2 % 4)).
 // The slots of one row are 64 contiguous bytes (producers write one row), and the xor makes the reads of
 // 8 lanes cover 128 contiguous bytes.
 __device__ __forceinline__ int pack_slot(int r, int kq) { return 4 * r + (kq ^ ((r >> 1) & 3)); }
 // columns k .. k + 3 (k % 4 == 0) of row m
-__device__ __forceinline__ void pack_parts4(half_t *Ap, int mt, int m, int k, const float (&v)[4]) {
-    half4 hi, lo;
-    split_parts4(v, hi, lo);
-    half_t *d = Ap + (((long long)(k >> 5) * 2 * mt + (m >> 4)) * 64 + pack_slot(m & 15, (k & 31) >> 3)) * 8 + (k & 4);
-    *(half4 *)d = hi;
-    *(half4 *)(d + mt * 512) = lo;
+__device__ __forceinline__ void pack_parts4(uint16_t *Ap, int mt, int m, int k, const float (&v)[4]) {
+    unsigned p[3][2];
+    split_bf16<4>(v, p);
+    uint16_t *d = Ap + (((long long)(k >> 5) * 3 * mt + (m >> 4)) * 64 + pack_slot(m & 15, (k & 31) >> 3)) * 8 + (k & 4);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) *(uint2 *)(d + c * mt * 512) = make_uint2(p[c][0], p[c][1]);
 }
 
 __device__ __forceinline__ float4 add4(float4 a, float4 b) {
     return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
-}
-__device__ __forceinline__ float max4(float4 v) {   // largest magnitude
-    return fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
 }
 // v[i] = the sum over the splits, in order, of the 4 columns at element off[i] of a GEMM's result. B splits
 // are loaded at a time (past the last one, that one again, not added), so a reader waits for memory
@@ -76,150 +86,140 @@ __device__ __forceinline__ void parts_sum(const EncParts &p, const int (&off)[NV
     }
 }
 
-// div[n] = row_divisor of the largest magnitude of row n
-__global__ __launch_bounds__(256) void enc_weight_scale_kernel(const float *__restrict__ src, float *__restrict__ div, int K) {
-    __shared__ float part[4];
-    const int n = blockIdx.x, tid = threadIdx.x;
-    float mx = 0.0f;
-    for (int k = tid * 4; k < K; k += 1024) {
-        const float4 v = *(const float4 *)(src + (long long)n * K + k);
-        mx = fmaxf(mx, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
-    }
-    mx = wave_max(mx);
-    if ((tid & 63) == 0) part[tid >> 6] = mx;
-    __syncthreads();
-    if (tid == 0) div[n] = row_divisor(fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3])));
-}
-
-// Weights in the order the GEMM reads them, 4 bytes each: blocks of 64 rows (output columns) x 64 columns
-// of K, 16 KB each, K innermost. Inside a block, each of 4 waves has 4 KB (32 rows, 32 columns) as its
-// four 1 KB loads: rows 16 j .. + 15, part p (hi, lo), lane: row lane % 16, columns 8 (lane / 16) .. + 7.
-// Row-major weights took 8% more time: rows of 4 or 8 KB put the 64 rows that a workgroup touches at
-// once on a few memory channels.
-__global__ __launch_bounds__(256) void enc_weight_pack_kernel(const float *__restrict__ src, const float *__restrict__ div,
-                                                              half_t *__restrict__ dst, int K) {
+// Weights in the order the GEMM reads them: blocks of 64 rows (output columns) x 64 columns of K, 16 KB
+// each, K innermost. Inside a block, each of 4 waves has 4 KB (32 rows, 32 columns) as its four 1 KB loads:
+// rows 16 j .. + 15, lane: row lane % 16, columns 8 (lane / 16) + 4 q .. + 3. Row-major weights took 8% more
+// time: rows of 4 or 8 KB put the 64 rows that a workgroup touches at once on a few memory channels.
+__global__ __launch_bounds__(256) void enc_weight_pack_kernel(const float *__restrict__ src, float *__restrict__ dst, int K) {
     const int s = blockIdx.x, t = blockIdx.y, nkt = gridDim.x;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    half_t *d = dst + (((long long)t * nkt + s) * 4 + wave) * 2048 + lane * 8;
+    float *d = dst + (((long long)t * nkt + s) * 4 + wave) * 1024 + lane * 4;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int row = t * 64 + (wave & 1) * 32 + j * 16 + (lane & 15);
         const int k = s * 64 + (wave >> 1) * 32 + (lane >> 4) * 8;
-        const float f = pow2_recip(div[row]);
-        float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = k < K ? src[(long long)row * K + k + e] * f : 0.0f;
-        half8 hi, lo;
-        split_parts8(v, hi, lo);
-        *(half8 *)(d + j * 1024) = hi;
-        *(half8 *)(d + j * 1024 + 512) = lo;
+        for (int q = 0; q < 2; ++q)
+            *(float4 *)(d + (j * 2 + q) * 256) = k < K ? *(const float4 *)(src + (long long)row * K + k + 4 * q)
+                                                       : make_float4(0.f, 0.f, 0.f, 0.f);
     }
 }
 
-// ws[z][M][N] = sums over K split z of A[M][K] W[N][K]^T, A and W packed, times adiv[m] wdiv[n].
+// ws[z][M][N] = sums over K split z of A[M][K] W[N][K]^T, A and W packed.
 //
 // The bound is the weight stream: each weight is read once up to 80 rows (one tile holds them all; twice up to 128), so the
 // design keeps HBM loads in flight and everything else under them. Weights go straight from global
-// memory to the registers of the lane that multiplies them (no LDS), three steps ahead. Three
-// v_mfma_f32_16x16x32_f16 products (hi hi, hi lo, lo hi) replace eight f32 MFMAs of the same 32 columns
-// of K at 3/16 of their matrix-core time. The dropped lo lo is below 2^-22 of a product. The hi hi sums
-// and the others have accumulators of their own, added at the end, so the main sum rounds once
-// per 32 products instead of eight times. (Three bf16 parts a value, split from f32 weights in the
-// loop, need no scales, but six products and five vector instructions a weight, which this core does not
-// overlap with MFMAs of the same wave: 10240 x 2048 at 77 rows 27.6 us.)
+// memory to the registers of the lane that multiplies them (no LDS), three steps ahead, and are split
+// there. Six v_mfma_f32_16x16x32_bf16 products (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi) replace eight
+// f32 MFMAs of the same 32 columns of K at 3/8 of their matrix-core time; the dropped ones lie below 2^-24 of a
+// product. The hi hi sums and the others have accumulators of their own, added at the end, so the
+// main sum rounds once per 32 products instead of eight times: error against 64 bits of a T5 prompt
+// 4.8e-7, 1.1e-6 on the f32 MFMA (CLIP 2.6e-7, 5.1e-7). 77 rows x 10240 x 2048: 28.8 us, 2.9 TB/s of weights.
+// (Two f16 parts of rows scaled by a power of two took 23.1 us, but lost every bit of values 2^-39 of
+// their row's largest, and splitting in the shadow of the MFMAs of the same wave took 31.4.)
 //
 // A step is 64 columns of K. 4 waves: wave w owns columns 32 (w & 1) .. + 31 of a 64-column tile and
 // K half w >> 1 of every step, and the two halves' sums are added through LDS at the end, so each
-// fragment of A read from LDS feeds two of W. A steps (4 KB per 16 rows) are shared by the waves through
-// two LDS buffers, loaded two steps ahead. Fetches past the split's end take its last step again, so
-// every wait in the loop has a fixed count of younger loads to leave in flight. (Eight waves with four
-// K ranges and half the K splits measured the same at 77 rows x 6144 x 2048 and 1.5 to 2 us a launch more
-// at a width of 1024; fragments read one step ahead of their products measured slower on both.)
+// fragment of A read from LDS feeds two of W. A steps (6 KB per 16 rows) are shared by the waves through
+// two LDS buffers, loaded one step ahead. Fetches past the split's end take its last step again, so
+// every wait in the loop has a fixed count of younger loads to leave in flight.
 //
 // MTP: the operand's row blocks; with MTP > MT, blockIdx.z picks the MT of them that the workgroup takes.
 template <int MT, int MTP>
 __global__ __launch_bounds__(256, 2) void enc_gemm_kernel(const EncGemmArgs g) {
-    constexpr int CH = 2 * 2 * MT * 64, NA = CH / 256;   // 16-byte chunks of an A step, per thread
+    constexpr int CH = 2 * 3 * MT * 64, NA = (CH + 255) / 256;   // 16-byte chunks of an A step, per thread
     __shared__ __attribute__((aligned(16))) uintx4_t As[2][CH];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, kq = lane >> 4, wn = wave & 1, kh = wave >> 1;
     const int n0 = blockIdx.x * 64 + wn * 32, z = blockIdx.y, mb = MTP > MT ? blockIdx.z * MT : 0;
     const int nkt = (g.K + 63) >> 6;
     const int kt0 = z * g.kps, kt1 = min(nkt, kt0 + g.kps);
-    const half_t *wb = g.W + ((long long)blockIdx.x * nkt * 4 + wave) * 2048;   // wave-uniform
-    uintx4_t w[4][4], a[2][NA];
-    auto fetch_w = [&](int kt, uintx4_t (&d)[4]) {
-        const uintx4_t *p = (const uintx4_t *)(wb + (long long)min(kt, kt1 - 1) * 8192);
+    const float *wb = g.W + ((long long)blockIdx.x * nkt * 4 + wave) * 1024;   // wave-uniform
+    floatx4_t w[3][4];
+    uintx4_t a[NA];
+    auto fetch_w = [&](int kt, floatx4_t (&d)[4]) {
+        const floatx4_t *p = (const floatx4_t *)(wb + (long long)min(kt, kt1 - 1) * 4096);
 #pragma unroll
         for (int q = 0; q < 4; ++q) d[q] = p[(unsigned)(q * 64 + lane)];
     };
-    auto fetch_a = [&](int kt, uintx4_t (&d)[NA]) {
-        const uintx4_t *p = (const uintx4_t *)g.Ap + ((long long)min(kt, kt1 - 1) * 4 * MTP + mb) * 64;
+    auto full = [&](int i) { return CH % 256 == 0 || i < NA - 1 || wave < CH % 256 / 64; };   // wave-uniform
+    auto fetch_a = [&](int kt) {
+        const uintx4_t *p = (const uintx4_t *)g.Ap + ((long long)min(kt, kt1 - 1) * 6 * MTP + mb) * 64;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int c = tid + 256 * i;
-            d[i] = p[(unsigned)(MTP > MT ? c / (64 * MT) * (64 * MTP) + c % (64 * MT) : c)];
+            if (full(i)) a[i] = p[(unsigned)(MTP > MT ? c / (64 * MT) * (64 * MTP) + c % (64 * MT) : c)];
         }
     };
-    auto stash_a = [&](int b, const uintx4_t (&d)[NA]) {
+    auto stash_a = [&](int b) {
 #pragma unroll
-        for (int i = 0; i < NA; ++i) As[b][tid + 256 * i] = d[i];
+        for (int i = 0; i < NA; ++i)
+            if (full(i)) As[b][tid + 256 * i] = a[i];
     };
     floatx4_t acc[2][MT], low[2][MT];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int i = 0; i < MT; ++i) acc[j][i] = low[j][i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    const int slot = kh * 2 * MT * 64 + pack_slot(r16, kq);
-    auto multiply = [&](int b, const uintx4_t (&o)[4]) {
-        half8 f[2][MT];
+    const int slot = kh * 3 * MT * 64 + pack_slot(r16, kq);
+    auto split_w = [&](const floatx4_t (&d)[4], bf16x8_t (&o)[2][3]) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+        for (int j = 0; j < 2; ++j) {
+            const floatx4_t x = d[2 * j], y = d[2 * j + 1];
+            const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
+            unsigned p[3][4];
+            split_bf16<8>(v, p);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) f[c][i] = __builtin_bit_cast(half8, As[b][(c * MT + i) * 64 + slot]);
-#pragma unroll
-        for (int c = 0; c < 3; ++c)   // A's hi with W's hi, hi with lo, lo with hi
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) {
-                    floatx4_t &d = c == 0 ? acc[j][i] : low[j][i];
-                    d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, o[2 * j + (c == 1)]), f[c == 2][i], d, 0, 0, 0);
-                }
+            for (int c = 0; c < 3; ++c) o[j][c] = __builtin_bit_cast(bf16x8_t, uintx4_t{p[c][0], p[c][1], p[c][2], p[c][3]});
+        }
     };
-    // Issue order A(kt + 2), W(kt + 3): when A(kt + 1) has to be in LDS, two weight steps and one A step
-    // issued after it are still in flight. LDS buffer (kt - kt0) & 1 holds A(kt); the other one was last
-    // read in step kt - 1, before the barrier that ended it.
-    fetch_a(kt0, a[0]);
+    auto multiply = [&](int b, const bf16x8_t (&o)[2][3]) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {   // part c of A with parts 0 .. 2 - c of W
+            bf16x8_t f[MT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) f[i] = __builtin_bit_cast(bf16x8_t, As[b][(c * MT + i) * 64 + slot]);
+#pragma unroll
+            for (int e = 0; e < 3 - c; ++e)
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        floatx4_t &d = c + e == 0 ? acc[j][i] : low[j][i];
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o[j][e], f[i], d, 0, 0, 0);
+                    }
+        }
+    };
+    // Step kt issues A(kt + 1), then W(kt + 3) into the registers that W(kt) leaves: A(kt + 1) has to be in LDS
+    // at the step's end, with W(kt + 3) still in flight. LDS buffer (kt - kt0) & 1 holds A(kt); the other
+    // one was last read in step kt - 1, before the barrier that ended it.
+    fetch_a(kt0);
     fetch_w(kt0, w[0]);
     fetch_w(kt0 + 1, w[1]);
-    fetch_a(kt0 + 1, a[1]);
+    stash_a(0);
     fetch_w(kt0 + 2, w[2]);
-    stash_a(0, a[0]);
     __syncthreads();
-    int kt = kt0;
-    for (; kt + 4 < kt1; kt += 4) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            fetch_a(kt + j + 2, a[j & 1]);
-            fetch_w(kt + j + 3, w[(j + 3) & 3]);
-            multiply(j & 1, w[j]);
-            stash_a((j + 1) & 1, a[(j + 1) & 1]);
-            __syncthreads();
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {   // the last one to four steps
-        if (j < 2) fetch_a(kt + j + 2, a[j & 1]);
-        if (j < 1) fetch_w(kt + j + 3, w[3]);
-        multiply(j & 1, w[j]);
-        if (kt + j + 1 >= kt1) break;
-        stash_a((j + 1) & 1, a[(j + 1) & 1]);
+    int kt = kt0, b = 0;
+    auto step = [&](floatx4_t (&d)[4]) {
+        bf16x8_t o[2][3];
+        fetch_a(kt + 1);
+        split_w(d, o);
+        fetch_w(kt + 3, d);
+        multiply(b, o);
+        stash_a(b ^ 1);
         __syncthreads();
+        b ^= 1;
+        ++kt;
+    };
+    while (kt + 3 <= kt1) {
+        step(w[0]);
+        step(w[1]);
+        step(w[2]);
     }
-    // the weights are the first operand: a lane holds columns n0 + 16 j + 4 kq .. + 3 of row 16 i + r16
-    __syncthreads();
-    // 4 MT KB of the buffers' 8 MT
+    if (kt < kt1) step(w[0]);
+    if (kt < kt1) step(w[1]);
+    // the weights are the first operand: a lane holds columns n0 + 16 j + 4 kq .. + 3 of row 16 i + r16;
+    // 4 MT KB of the buffers' 12 MT
     floatx4_t *sum = (floatx4_t *)&As[0][0] + wn * 2 * MT * 64 + lane;
     if (kh > 0) {
 #pragma unroll
@@ -229,18 +229,13 @@ __global__ __launch_bounds__(256, 2) void enc_gemm_kernel(const EncGemmArgs g) {
     }
     __syncthreads();
     if (kh > 0) return;
-    floatx4_t wd[2];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) wd[j] = *(const floatx4_t *)(g.wdiv + n0 + 16 * j + 4 * kq);
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const int m = 16 * (mb + i) + r16;
         if (m >= g.M) continue;
-        const float ad = g.adiv[m];
         float *y = g.ws + ((long long)z * g.M + m) * g.N + n0 + 4 * kq;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
-            *(floatx4_t *)(y + 16 * j) = ((acc[j][i] + low[j][i]) + sum[(j * MT + i) * 64]) * wd[j] * ad;
+        for (int j = 0; j < 2; ++j) *(floatx4_t *)(y + 16 * j) = (acc[j][i] + low[j][i]) + sum[(j * MT + i) * 64];
     }
 }
 
@@ -258,13 +253,6 @@ __global__ __launch_bounds__(256) void enc_norm_kernel(const EncNormArgs a) {
         if (lane == 0) part[wave] = v;
         __syncthreads();
         return ((part[0] + part[1]) + part[2]) + part[3];
-    };
-    auto block_max = [&](float v) {
-        v = wave_max(v);
-        __syncthreads();
-        if (lane == 0) part[wave] = v;
-        __syncthreads();
-        return fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
     };
     // the row in registers: columns 4*tid + 1024*j .. + 3; all loads ahead of the first barrier
     const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -314,30 +302,21 @@ __global__ __launch_bounds__(256) void enc_norm_kernel(const EncNormArgs a) {
     } else {
         inv = 1.0f / sqrtf(s / (float)H + a.eps);
     }
-    float4 o[NJ];
-    float mx = 0.0f;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {   // columns past H: zero
+    for (int j = 0; j < NJ; ++j) {
+        const int c = 4 * tid + 1024 * j;
+        if (!in[j]) continue;
+        float4 o;
         if (LN) {
-            o[j] = make_float4((v[j].x - mean) * inv * wv[j].x + bv[j].x, (v[j].y - mean) * inv * wv[j].y + bv[j].y,
-                               (v[j].z - mean) * inv * wv[j].z + bv[j].z, (v[j].w - mean) * inv * wv[j].w + bv[j].w);
+            o = make_float4((v[j].x - mean) * inv * wv[j].x + bv[j].x, (v[j].y - mean) * inv * wv[j].y + bv[j].y,
+                            (v[j].z - mean) * inv * wv[j].z + bv[j].z, (v[j].w - mean) * inv * wv[j].w + bv[j].w);
         } else {
-            o[j] = make_float4(v[j].x * inv * wv[j].x, v[j].y * inv * wv[j].y, v[j].z * inv * wv[j].z, v[j].w * inv * wv[j].w);
+            o = make_float4(v[j].x * inv * wv[j].x, v[j].y * inv * wv[j].y, v[j].z * inv * wv[j].z, v[j].w * inv * wv[j].w);
         }
-        mx = fmaxf(mx, max4(o[j]));
-    }
-    if (a.Ap) {
-        const float d = row_divisor(block_max(mx)), f = pow2_recip(d);
-        if (tid == 0) a.adiv[row] = d;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const float o4[4] = {o[j].x * f, o[j].y * f, o[j].z * f, o[j].w * f};
-            if (in[j]) pack_parts4(a.Ap, a.mt, row, 4 * tid + 1024 * j, o4);
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-            if (in[j]) *(float4 *)(a.y + (long long)row * H + 4 * tid + 1024 * j) = o[j];
+        if (a.Ap) {
+            const float o4[4] = {o.x, o.y, o.z, o.w};
+            pack_parts4(a.Ap, a.mt, row, c, o4);
+        } else *(float4 *)(a.y + (long long)row * H + c) = o;
     }
 }
 
@@ -446,73 +425,42 @@ __global__ __launch_bounds__(64 * (MT < 4 ? 4 : MT), 1) void enc_attn_kernel(con
         }
     if (q >= S) return;
     const floatx4_t y = o[0] + o[1];
-    const float f = pow2_recip(a.odiv[0]);
-    const float y4[4] = {y[0] * f, y[1] * f, y[2] * f, y[3] * f};
+    const float y4[4] = {y[0], y[1], y[2], y[3]};
     pack_parts4(a.Ap, a.mt, q, h * EA_HD + 16 * wave + 4 * kq, y4);
 }
 
-// The FFN activation of a GEMM's result as the next GEMM's operand, one workgroup per row (its largest
-// magnitude sets the scale): quick GELU of column c (shaders/ops_conv.metal:25-29), or gelu_tanh(column
-// c) * column F + c (GEGLU; tanh form, argument clamped to +-10: shaders/ops_conv.metal:15-24). A thread
-// has 4 columns of every 4096; those past the first 8192 are computed again when the scale is known.
+// The FFN activation of a GEMM's result as the next GEMM's operand, four columns a thread: quick GELU of
+// column c (shaders/ops_conv.metal:25-29), or gelu_tanh(column c) * column F + c (GEGLU; tanh form, argument
+// clamped to +-10: shaders/ops_conv.metal:15-24).
 template <bool GEGLU>
-__global__ __launch_bounds__(1024) void enc_act_kernel(EncParts p, half_t *Ap, float *adiv, int mt, int F) {
-    __shared__ float part[16];
-    const int tid = threadIdx.x, m = blockIdx.x;
+__global__ __launch_bounds__(256) void enc_act_kernel(EncParts p, uint16_t *Ap, int mt, int F) {
+    constexpr int NV = GEGLU ? 2 : 1;
+    const int m = blockIdx.y, c = 4 * (blockIdx.x * 256 + threadIdx.x);
+    if (c >= F) return;
     p.ws += (long long)m * p.N;
-    auto act = [&](int c) {
-        constexpr int NV = GEGLU ? 2 : 1;
-        int off[NV];
-        float4 u[NV];
+    int off[NV];
+    float4 u[NV];
 #pragma unroll
-        for (int i = 0; i < NV; ++i) off[i] = i * F + c;
-        parts_sum<NV, 4>(p, off, u);
-        if (p.bias) {
+    for (int i = 0; i < NV; ++i) off[i] = i * F + c;
+    parts_sum<NV, 4>(p, off, u);
+    if (p.bias) {
 #pragma unroll
-            for (int i = 0; i < NV; ++i) u[i] = add4(u[i], *(const float4 *)(p.bias + i * F + c));
-        }
-        const float uv[4] = {u[0].x, u[0].y, u[0].z, u[0].w};
-        float y[4];
-        if constexpr (GEGLU) {
-            const float gv[4] = {u[1].x, u[1].y, u[1].z, u[1].w};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float v = uv[e], t = 0.7978845608f * (v + 0.044715f * v * v * v);
-                y[e] = 0.5f * v * (1.0f + tanhf(fminf(fmaxf(t, -10.0f), 10.0f))) * gv[e];
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) y[e] = uv[e] / (1.0f + expf(-1.702f * uv[e]));
-        }
-        return make_float4(y[0], y[1], y[2], y[3]);
-    };
-    float4 keep[2];
-    float mx = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int c = 4 * tid + 4096 * i;
-        if (c < F) {
-            keep[i] = act(c);
-            mx = fmaxf(mx, max4(keep[i]));
-        }
+        for (int i = 0; i < NV; ++i) u[i] = add4(u[i], *(const float4 *)(p.bias + i * F + c));
     }
-    for (int c = 4 * tid + 8192; c < F; c += 4096) mx = fmaxf(mx, max4(act(c)));
-    mx = wave_max(mx);
-    if ((tid & 63) == 0) part[tid >> 6] = mx;
-    __syncthreads();
-    mx = part[0];
+    const float uv[4] = {u[0].x, u[0].y, u[0].z, u[0].w};
+    float y[4];
+    if constexpr (GEGLU) {
+        const float gv[4] = {u[1].x, u[1].y, u[1].z, u[1].w};
 #pragma unroll
-    for (int i = 1; i < 16; ++i) mx = fmaxf(mx, part[i]);
-    const float d = row_divisor(mx), f = pow2_recip(d);
-    if (tid == 0) adiv[m] = d;
-    auto pack = [&](int c, float4 y) {
-        const float y4[4] = {y.x * f, y.y * f, y.z * f, y.w * f};
-        pack_parts4(Ap, mt, m, c, y4);
-    };
+        for (int e = 0; e < 4; ++e) {
+            const float v = uv[e], t = 0.7978845608f * (v + 0.044715f * v * v * v);
+            y[e] = 0.5f * v * (1.0f + tanhf(fminf(fmaxf(t, -10.0f), 10.0f))) * gv[e];
+        }
+    } else {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-        if (4 * tid + 4096 * i < F) pack(4 * tid + 4096 * i, keep[i]);
-    for (int c = 4 * tid + 8192; c < F; c += 4096) pack(c, act(c));
+        for (int e = 0; e < 4; ++e) y[e] = uv[e] / (1.0f + expf(-1.702f * uv[e]));
+    }
+    pack_parts4(Ap, mt, m, c, y);
 }
 
 // x[s][c] = tok[ids[s]][c] (+ pos[s][c]), one workgroup per row; the ids are kernel arguments, so the
@@ -534,25 +482,30 @@ bool aligned16(const void *p) { return (((uintptr_t)p) & 15) == 0; }
 
 int enc_row_blocks(int M) { return M <= 32 ? 2 : M <= 80 ? 5 : 8; }
 size_t enc_operand_bytes(int M, int K) {   // whole 64-column steps
-    return (size_t)2 * enc_row_blocks(M) * 16 * ((K + 63) / 64 * 64) * sizeof(half_t);
+    return (size_t)3 * enc_row_blocks(M) * 16 * ((K + 63) / 64 * 64) * sizeof(uint16_t);
 }
 
 size_t enc_weight_floats(int N, int K) { return (size_t)N * ((K + 63) / 64 * 64); }
 
-int launch_enc_weight_pack(const float *src, half_t *dst, float *div, int N, int K, hipStream_t st) {
-    TSN_REQUIRE(src && dst && div && N > 0 && K > 0 && N % 64 == 0 && K % 32 == 0 && aligned16(src) && aligned16(dst),
+int launch_enc_weight_pack(const float *src, float *dst, int N, int K, hipStream_t st) {
+    TSN_REQUIRE(src && dst && N > 0 && K > 0 && N % 64 == 0 && K % 32 == 0 && aligned16(src) && aligned16(dst),
                 "enc_weight_pack: 16-byte aligned weights, N a multiple of 64, K of 32");
-    TSN_LAUNCH(enc_weight_scale_kernel, dim3(N), dim3(256), 0, st, src, div, K);
-    TSN_LAUNCH(enc_weight_pack_kernel, dim3((K + 63) / 64, N / 64), dim3(256), 0, st, src, div, dst, K);
+    // blocks of N in groups that the grid's second dimension takes
+    const int nkt = (K + 63) / 64;
+    for (int t0 = 0; t0 < N / 64; t0 += 65535) {
+        const int n = std::min(65535, N / 64 - t0);
+        TSN_LAUNCH(enc_weight_pack_kernel, dim3(nkt, n), dim3(256), 0, st, src + (size_t)t0 * 64 * K,
+                   dst + (size_t)t0 * nkt * 4096, K);
+    }
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }
 
 int launch_enc_gemm(EncGemmArgs &g, hipStream_t st) {
-    TSN_REQUIRE(g.Ap && g.adiv && g.W && g.wdiv && g.ws && g.M > 0 && g.M <= 128 && g.N > 0 && g.K > 0,
+    TSN_REQUIRE(g.Ap && g.W && g.ws && g.M > 0 && g.M <= 128 && g.N > 0 && g.K > 0,
                 "enc_gemm: null operand, or rows outside 1..128");
     TSN_REQUIRE(g.N % 64 == 0 && g.K % 32 == 0, "enc_gemm: N a multiple of 64, K of 32");
-    TSN_REQUIRE(aligned16(g.Ap) && aligned16(g.W) && aligned16(g.wdiv) && aligned16(g.ws), "enc_gemm: 16-byte aligned operands");
+    TSN_REQUIRE(aligned16(g.Ap) && aligned16(g.W) && aligned16(g.ws), "enc_gemm: 16-byte aligned operands");
     const int mt = enc_row_blocks(g.M);
     TSN_REQUIRE((size_t)g.M * g.N * sizeof(float) <= g.ws_bytes, "enc_gemm: workspace");
     // at most two workgroups per CU, of at least four steps each
@@ -572,7 +525,7 @@ int launch_enc_gemm(EncGemmArgs &g, hipStream_t st) {
 int launch_enc_norm(const EncNormArgs &a, bool ln, hipStream_t st) {
     TSN_REQUIRE(a.x && a.w && (a.y || a.Ap) && a.rows > 0 && a.H > 0 && (!ln || a.b), "enc_norm: arguments");
     TSN_REQUIRE(!a.parts.ws || (a.xout && a.rows <= 128 && a.parts.splits > 0 && a.parts.N == a.H), "enc_norm: partial sums");
-    TSN_REQUIRE(!a.Ap || (a.adiv && a.rows <= 128 && a.H % 32 == 0), "enc_norm: packed rows");
+    TSN_REQUIRE(!a.Ap || (a.rows <= 128 && a.H % 32 == 0), "enc_norm: packed rows");
     TSN_REQUIRE(a.H % 4 == 0 && a.H <= 2048 && aligned16(a.x) && aligned16(a.y) && aligned16(a.w) && aligned16(a.b),
                 "enc_norm: rows of at most 2048 floats, a multiple of 4, 16-byte aligned");
     if (ln && a.H <= 1024) TSN_LAUNCH((enc_norm_kernel<true, 1>), dim3(a.rows), dim3(256), 0, st, a);
@@ -592,7 +545,7 @@ int launch_enc_norm_rows(const float *x, float *y, const float *w, const float *
 }
 
 int launch_enc_attention(const EncAttnArgs &a, hipStream_t st) {
-    TSN_REQUIRE(a.qkv.ws && a.Ap && a.odiv && a.S > 0 && a.S <= EA_SMAX && a.nh > 0 && a.qkv.N == 3 * EA_HD * a.nh,
+    TSN_REQUIRE(a.qkv.ws && a.Ap && a.S > 0 && a.S <= EA_SMAX && a.nh > 0 && a.qkv.N == 3 * EA_HD * a.nh,
                 "enc_attention: context 1..128, rows of q, k and v with heads of 64");
     TSN_REQUIRE((a.mode == 1 && a.rel) || a.mode == 2, "enc_attention: mode and tables");
     const dim3 grid((a.nh + 7) / 8 * 8 * ((a.S + EA_Q - 1) / EA_Q));
@@ -604,11 +557,12 @@ int launch_enc_attention(const EncAttnArgs &a, hipStream_t st) {
     return TSN_OK;
 }
 
-int launch_enc_act(const EncParts &p, bool geglu, half_t *Ap, float *adiv, int rows, int F, hipStream_t st) {
-    TSN_REQUIRE(p.ws && Ap && adiv && rows > 0 && rows <= 128 && F > 0 && F % 32 == 0 && p.N == (geglu ? 2 * F : F),
+int launch_enc_act(const EncParts &p, bool geglu, uint16_t *Ap, int rows, int F, hipStream_t st) {
+    TSN_REQUIRE(p.ws && Ap && rows > 0 && rows <= 128 && F > 0 && F % 32 == 0 && p.N == (geglu ? 2 * F : F),
                 "enc_act: arguments");
-    if (geglu) TSN_LAUNCH(enc_act_kernel<true>, dim3(rows), dim3(1024), 0, st, p, Ap, adiv, enc_row_blocks(rows), F);
-    else TSN_LAUNCH(enc_act_kernel<false>, dim3(rows), dim3(1024), 0, st, p, Ap, adiv, enc_row_blocks(rows), F);
+    const dim3 grid((F + 1023) / 1024, rows), block(256);
+    if (geglu) TSN_LAUNCH(enc_act_kernel<true>, grid, block, 0, st, p, Ap, enc_row_blocks(rows), F);
+    else TSN_LAUNCH(enc_act_kernel<false>, grid, block, 0, st, p, Ap, enc_row_blocks(rows), F);
     TSN_HIP_CHECK(hipGetLastError());
     return TSN_OK;
 }

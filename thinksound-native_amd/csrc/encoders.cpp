@@ -5,7 +5,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <cmath>
 #include <map>
 
 #include "gguf.h"
@@ -153,66 +152,35 @@ std::vector<ManifestEntry> t5_manifest(const T5Spec &s) {
 }
 
 // K splits of a QKV GEMM: attention reads every split of k and v in each of a head's workgroups. 77 rows, 1024
-// wide: 4 splits 1.48 ms a prompt, 2 splits 1.51 (the GEMM 9.2 -> 10.8 us); 2048 wide: 2.27 ms with 4 and 2,
-// 2.30 with 5.
+// wide: 4 splits 1.42 ms a prompt, 2 splits 1.48; 2048 wide: 2.49 ms with 4 and 2, 2.54 with 5.
 constexpr int QKV_SPLITS = 4;
 
-int EncoderRunner::create_common(int ctx, int width, int ffn, int ffn_cols, int layers) {
+int EncoderRunner::create_common(int ctx, int width, int ffn, int ffn_cols) {
     TSN_TRY(alloc(enc_operand_bytes(ctx, width), (void **)&A_));
     TSN_TRY(alloc(enc_operand_bytes(ctx, ffn), (void **)&F_));
-    TSN_TRY(alloc((size_t)ctx * 4, (void **)&adiv_));
-    TSN_TRY(alloc((size_t)ctx * 4, (void **)&fdiv_));
-    TSN_TRY(alloc((size_t)layers * ctx * 4, (void **)&odiv_));
     ws_bytes_ = std::max(ENC_WS_BYTES, (size_t)ctx * std::max(3 * (size_t)width, (size_t)ffn_cols) * sizeof(float));
     return alloc(ws_bytes_, (void **)&ws_);
 }
 
-int EncoderRunner::gemm(const half_t *A, const float *adiv, const EncWeight &W, const float *b, int M, int N, int K,
-                        EncParts &out, int most) {
-    EncGemmArgs g{A, adiv, W.w, W.div, ws_, ws_bytes_, M, N, K, most, 1, 0};
-    TSN_TRY(run("enc_gemm_kernel", 2.0 * M * N * K, 4.0 * ((double)N * K + M * (double)N + M * (double)K),
+int EncoderRunner::gemm(const uint16_t *A, const float *W, const float *b, int M, int N, int K, EncParts &out, int most) {
+    EncGemmArgs g{A, W, ws_, ws_bytes_, M, N, K, most, 1, 0};
+    TSN_TRY(run("enc_gemm_kernel", 2.0 * M * N * K, 4.0 * ((double)N * K + M * (double)N) + 6.0 * M * (double)K,
                 [&] { return launch_enc_gemm(g, rt->dev.stream()); }));
     out = EncParts{ws_, (long long)M * N, g.splits, N, b};
     return TSN_OK;
 }
 
 int EncoderRunner::pack_weights(const std::vector<RawWeight> &ws) {
-    size_t most = 0, rows = 0;
-    for (const RawWeight &w : ws) {
-        most = std::max(most, (size_t)w.N * w.K * sizeof(float));
-        rows += (size_t)w.N;
-    }
+    size_t most = 0;
+    for (const RawWeight &w : ws) most = std::max(most, (size_t)w.N * w.K * sizeof(float));
     void *tmp;
-    float *div;
-    TSN_TRY(alloc(rows * sizeof(float), (void **)&div));
     TSN_TRY(alloc(most, &tmp));
     const hipStream_t st = rt->dev.stream();
     for (const RawWeight &w : ws) {
         TSN_TRY(rt->dev.copy_d2d(tmp, w.p, (size_t)w.N * w.K * sizeof(float)));
-        TSN_TRY(launch_enc_weight_pack((const float *)tmp, (half_t *)w.p, div, w.N, w.K, st));
-        *w.out = EncWeight{(const half_t *)w.p, div};
-        div += w.N;
+        TSN_TRY(launch_enc_weight_pack((const float *)tmp, w.p, w.N, w.K, st));
     }
     return release(tmp);
-}
-
-// An output of attention is a mean of v rows, and |v| <= |norm output| |row of Wv| + |bv| with
-// |norm output| <= sqrt(width) max|nw| + |nb|. The bound may be loose: values 2^-16 of it still keep 22 bits.
-int EncoderRunner::set_odiv(int layer, int ctx, int width, const float *wv, const float *bv, const float *nw, const float *nb) {
-    double row = 0.0, w = 0.0, b2 = 0.0, bias = 0.0;
-    for (int n = 0; n < width; ++n) {
-        double s = 0.0;
-        for (int k = 0; k < width; ++k) s += (double)wv[(size_t)n * width + k] * wv[(size_t)n * width + k];
-        row = std::max(row, s);
-        if (bv) bias = std::max(bias, fabs((double)bv[n]));
-        w = std::max(w, fabs((double)nw[n]));
-        if (nb) b2 += (double)nb[n] * nb[n];
-    }
-    const double bound = (sqrt((double)width) * w + sqrt(b2)) * sqrt(row) + bias;
-    // bound / div below 2^15; exponents as the device's row_divisor has them
-    const int e = bound > 0.0 && std::isfinite(bound) ? std::min(std::max(ilogb(bound), -95), 127) : 0;
-    const std::vector<float> div((size_t)ctx, ldexpf(1.0f, e - 14));
-    return rt->dev.upload(odiv_ + (size_t)layer * ctx, div.data(), div.size() * sizeof(float));
 }
 
 /* ---------------- CLIP ---------------- */
@@ -224,7 +192,7 @@ int ClipModel::create(Runtime *r, const ClipSpec &sp) {
     s = sp;
     const size_t n = s.ctx, H = s.H;
     TSN_TRY(alloc(n * H * 4, (void **)&X_));
-    return create_common(s.ctx, s.H, 4 * s.H, 4 * s.H, s.NL);
+    return create_common(s.ctx, s.H, 4 * s.H, 4 * s.H);
 }
 
 int ClipModel::upload_weights(const float *host, size_t numel) { return upload(host, numel); }
@@ -270,19 +238,16 @@ int ClipModel::upload(const float *host, size_t numel) {
     pos_ = P("pos_emb");
     L_.resize(s.NL);
     std::vector<RawWeight> pw;
-    auto at = [&](const std::string &n) {   // host tensor
-        return host + std::find_if(man.begin(), man.end(), [&](const ManifestEntry &e) { return e.name == n; })->offset;
-    };
     for (int l = 0; l < s.NL; ++l) {
         const std::string b = "blk." + std::to_string(l);
         Layer &L = L_[l];
         L.ln1w = P(b + ".ln1.w"); L.ln1b = P(b + ".ln1.b"); L.bqkv = P(b + ".qkv.b"); L.bo = P(b + ".out.b");
         L.ln2w = P(b + ".ln2.w"); L.ln2b = P(b + ".ln2.b"); L.b1 = P(b + ".fc1.b"); L.b2 = P(b + ".fc2.b");
-        pw.push_back({dev + lay.at.at(b + ".qkv.w"), 3 * s.H, s.H, &L.Wqkv});
-        pw.push_back({dev + lay.at.at(b + ".out.w"), s.H, s.H, &L.Wo});
-        pw.push_back({dev + lay.at.at(b + ".fc1.w"), 4 * s.H, s.H, &L.W1});
-        pw.push_back({dev + lay.at.at(b + ".fc2.w"), s.H, 4 * s.H, &L.W2});
-        TSN_TRY(set_odiv(l, s.ctx, s.H, at(b + ".v.w"), at(b + ".v.b"), at(b + ".ln1.w"), at(b + ".ln1.b")));
+        L.Wqkv = P(b + ".qkv.w"); L.Wo = P(b + ".out.w"); L.W1 = P(b + ".fc1.w"); L.W2 = P(b + ".fc2.w");
+        pw.push_back({dev + lay.at.at(b + ".qkv.w"), 3 * s.H, s.H});
+        pw.push_back({dev + lay.at.at(b + ".out.w"), s.H, s.H});
+        pw.push_back({dev + lay.at.at(b + ".fc1.w"), 4 * s.H, s.H});
+        pw.push_back({dev + lay.at.at(b + ".fc2.w"), s.H, 4 * s.H});
     }
     lnw_ = P("out_ln.w");
     lnb_ = P("out_ln.b");
@@ -308,7 +273,7 @@ int ClipModel::encode(const int32_t *ids, float *per_token, float *global) {
     const int mt = enc_row_blocks(n);
     // X += the pending GEMM result (if any), then LN into the operand A_ or, last, per_token
     auto norm = [&](const EncParts &p, const float *w, const float *b, float *y) {
-        EncNormArgs a{X_, X_, p, w, b, y, y ? nullptr : A_, adiv_, mt, n, H, s.eps};
+        EncNormArgs a{X_, X_, p, w, b, y, y ? nullptr : A_, mt, n, H, s.eps};
         return run("enc_norm_kernel<true>", 0, 4.0 * n * H * (p.ws ? p.splits + 3 : 2),
                    [&] { return launch_enc_norm(a, true, st); });
     };
@@ -316,18 +281,17 @@ int ClipModel::encode(const int32_t *ids, float *per_token, float *global) {
     TSN_TRY(run("embed_rows_kernel", 0, 12.0 * n * H, [&] { return launch_embed_rows(id, tok_, pos_, X_, n, H, st); }));
     for (int l = 0; l < s.NL; ++l) {
         const Layer &w = L_[l];
-        const float *odiv = odiv_ + (size_t)l * n;
         TSN_TRY(norm(l ? p : none, w.ln1w, w.ln1b, nullptr));
-        TSN_TRY(gemm(A_, adiv_, w.Wqkv, w.bqkv, n, 3 * H, H, p, QKV_SPLITS));
-        EncAttnArgs a{p, A_, odiv, mt, n, s.NH, 0.125f, 2, nullptr, {0, 0, 0, 0}, eos};
+        TSN_TRY(gemm(A_, w.Wqkv, w.bqkv, n, 3 * H, H, p, QKV_SPLITS));
+        EncAttnArgs a{p, A_, mt, n, s.NH, 0.125f, 2, nullptr, {0, 0, 0, 0}, eos};
         TSN_TRY(run("enc_attn_kernel", 4.0 * s.NH * n * (double)n * 64, 4.0 * n * H * (3 * p.splits + 1.5),
                     [&] { return launch_enc_attention(a, st); }));
-        TSN_TRY(gemm(A_, odiv, w.Wo, w.bo, n, H, H, p));
+        TSN_TRY(gemm(A_, w.Wo, w.bo, n, H, H, p));
         TSN_TRY(norm(p, w.ln2w, w.ln2b, nullptr));
-        TSN_TRY(gemm(A_, adiv_, w.W1, w.b1, n, 4 * H, H, p));
+        TSN_TRY(gemm(A_, w.W1, w.b1, n, 4 * H, H, p));
         TSN_TRY(run("enc_act_kernel<false>", 0, 4.0 * n * 4 * H * (p.splits + 1.5),
-                    [&] { return launch_enc_act(p, false, F_, fdiv_, n, 4 * H, st); }));
-        TSN_TRY(gemm(F_, fdiv_, w.W2, w.b2, n, H, 4 * H, p));
+                    [&] { return launch_enc_act(p, false, F_, n, 4 * H, st); }));
+        TSN_TRY(gemm(F_, w.W2, w.b2, n, H, 4 * H, p));
     }
     TSN_TRY(norm(p, lnw_, lnb_, per_token));
     // pooled: text_proj · per_token[eos] (src/clip.cpp:88-91)
@@ -348,7 +312,7 @@ int T5Model::create(Runtime *r, const T5Spec &sp) {
     const size_t n = s.ctx, d = s.d;
     TSN_TRY(alloc(n * d * 4, (void **)&X_));
     TSN_TRY(alloc((2 * n - 1) * s.NH * 4, (void **)&rel_));
-    return create_common(s.ctx, s.d, s.d_ff, 2 * s.d_ff, s.NL);
+    return create_common(s.ctx, s.d, s.d_ff, 2 * s.d_ff);
 }
 
 int T5Model::upload_weights(const float *host, size_t numel) { return upload(host, numel); }
@@ -402,11 +366,11 @@ int T5Model::upload(const float *host, size_t numel) {
         const std::string b = "blk." + std::to_string(l);
         Layer &L = L_[l];
         L.an = P(b + ".attn_norm"); L.fn = P(b + ".ffn_norm");
-        pw.push_back({dev + lay.at.at(b + ".qkv"), 3 * s.d, s.d, &L.Wqkv});
-        pw.push_back({dev + lay.at.at(b + ".o"), s.d, s.d, &L.Wo});
-        pw.push_back({dev + lay.at.at(b + ".wi"), 2 * s.d_ff, s.d, &L.Wi});
-        pw.push_back({dev + lay.at.at(b + ".wo"), s.d, s.d_ff, &L.Wout});
-        TSN_TRY(set_odiv(l, s.ctx, s.d, at(b + ".v"), nullptr, at(b + ".attn_norm"), nullptr));
+        L.Wqkv = P(b + ".qkv"); L.Wo = P(b + ".o"); L.Wi = P(b + ".wi"); L.Wout = P(b + ".wo");
+        pw.push_back({dev + lay.at.at(b + ".qkv"), 3 * s.d, s.d});
+        pw.push_back({dev + lay.at.at(b + ".o"), s.d, s.d});
+        pw.push_back({dev + lay.at.at(b + ".wi"), 2 * s.d_ff, s.d});
+        pw.push_back({dev + lay.at.at(b + ".wo"), s.d, s.d_ff});
     }
     on_ = P("out_norm");
     // the bias of each head by distance k - q in -(ctx - 1) .. ctx - 1: bucket(k - q) (src/t5.cpp:47-53)
@@ -438,7 +402,7 @@ int T5Model::encode(const int32_t *ids, float *out) {
     const int mt = enc_row_blocks(n);
     // X += the pending GEMM result (if any), then RMS into the operand A_ or, last, out
     auto rms = [&](const EncParts &p, const float *w, float *y) {
-        EncNormArgs a{X_, X_, p, w, nullptr, y, y ? nullptr : A_, adiv_, mt, n, d, s.eps};
+        EncNormArgs a{X_, X_, p, w, nullptr, y, y ? nullptr : A_, mt, n, d, s.eps};
         return run("enc_norm_kernel<false>", 0, 4.0 * n * d * (p.ws ? p.splits + 3 : 2),
                    [&] { return launch_enc_norm(a, false, st); });
     };
@@ -446,19 +410,18 @@ int T5Model::encode(const int32_t *ids, float *out) {
     TSN_TRY(run("embed_rows_kernel", 0, 8.0 * n * d, [&] { return launch_embed_rows(id, tok_, nullptr, X_, n, d, st); }));
     for (int l = 0; l < s.NL; ++l) {
         const Layer &w = L_[l];
-        const float *odiv = odiv_ + (size_t)l * n;
         TSN_TRY(rms(l ? p : none, w.an, nullptr));
-        TSN_TRY(gemm(A_, adiv_, w.Wqkv, nullptr, n, 3 * d, d, p, QKV_SPLITS));
+        TSN_TRY(gemm(A_, w.Wqkv, nullptr, n, 3 * d, d, p, QKV_SPLITS));
         // scale 1: T5 folds 1/sqrt(d_kv) into q (src/t5.cpp:70)
-        EncAttnArgs a{p, A_, odiv, mt, n, s.NH, 1.0f, 1, rel_, {keys[0], keys[1], keys[2], keys[3]}, 0};
+        EncAttnArgs a{p, A_, mt, n, s.NH, 1.0f, 1, rel_, {keys[0], keys[1], keys[2], keys[3]}, 0};
         TSN_TRY(run("enc_attn_kernel", 4.0 * s.NH * n * (double)n * 64, 4.0 * n * d * (3 * p.splits + 1.5),
                     [&] { return launch_enc_attention(a, st); }));
-        TSN_TRY(gemm(A_, odiv, w.Wo, nullptr, n, d, d, p));
+        TSN_TRY(gemm(A_, w.Wo, nullptr, n, d, d, p));
         TSN_TRY(rms(p, w.fn, nullptr));
-        TSN_TRY(gemm(A_, adiv_, w.Wi, nullptr, n, 2 * F, d, p));
+        TSN_TRY(gemm(A_, w.Wi, nullptr, n, 2 * F, d, p));
         TSN_TRY(run("enc_act_kernel<true>", 0, 4.0 * n * F * (2 * p.splits + 1.5),
-                    [&] { return launch_enc_act(p, true, F_, fdiv_, n, F, st); }));
-        TSN_TRY(gemm(F_, fdiv_, w.Wout, nullptr, n, d, F, p));
+                    [&] { return launch_enc_act(p, true, F_, n, F, st); }));
+        TSN_TRY(gemm(F_, w.Wout, nullptr, n, d, F, p));
     }
     return rms(p, on_, out);
 }

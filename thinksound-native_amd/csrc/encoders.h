@@ -38,33 +38,21 @@ int t5_spec_from_gguf(const char *path, T5Spec *out);       // t5.* metadata
 // bidirectional bucket of relative position rel = k - q (src/t5.cpp:6-19)
 int t5_bucket(int rel, int n_bucket, int max_dist);
 
-struct EncWeight {   // a packed [N][K] weight and its row divisors
-    const half_t *w;
-    const float *div;
-};
-
 class EncoderRunner : public GraphRunner {
 protected:
     float *ws_ = nullptr;                        // ws_bytes_
     size_t ws_bytes_ = 0;
-    half_t *A_ = nullptr, *F_ = nullptr;         // packed GEMM operands: width and FFN columns
-    float *adiv_ = nullptr, *fdiv_ = nullptr;    // their row divisors
-    float *odiv_ = nullptr;                      // [layers][ctx] divisors of the attention outputs
+    uint16_t *A_ = nullptr, *F_ = nullptr;       // packed GEMM operands: width and FFN columns
     // ffn_cols: columns of the first FFN GEMM's result
-    int create_common(int ctx, int width, int ffn, int ffn_cols, int layers);
+    int create_common(int ctx, int width, int ffn, int ffn_cols);
     // out = A·Wᵀ (+ b) as K-split sums in ws_, for the next kernel to read
-    int gemm(const half_t *A, const float *adiv, const EncWeight &W, const float *b, int M, int N, int K, EncParts &out,
-             int most = 1 << 20);
+    int gemm(const uint16_t *A, const float *W, const float *b, int M, int N, int K, EncParts &out, int most = 1 << 20);
     // row-major [N][K] weights at p, each in a region of enc_weight_floats, packed in place
     struct RawWeight {
         float *p;
         int N, K;
-        EncWeight *out;
     };
     int pack_weights(const std::vector<RawWeight> &ws);
-    // odiv_ of a layer: a power of two that brings its v rows below the f16 range. wv [width][width]
-    // host rows, bv their bias, and the norm's weight and bias (null: none)
-    int set_odiv(int layer, int ctx, int width, const float *wv, const float *bv, const float *nw, const float *nb);
 };
 
 class ClipModel : public EncoderRunner {
@@ -80,7 +68,7 @@ public:
 private:
     struct Layer {
         const float *ln1w, *ln1b, *bqkv, *bo, *ln2w, *ln2b, *b1, *b2;
-        EncWeight Wqkv, Wo, W1, W2;
+        const float *Wqkv, *Wo, *W1, *W2;   // packed
     };
     std::vector<Layer> L_;
     const float *tok_ = nullptr, *pos_ = nullptr, *lnw_ = nullptr, *lnb_ = nullptr, *proj_ = nullptr;
@@ -102,7 +90,7 @@ public:
 private:
     struct Layer {
         const float *an, *fn;
-        EncWeight Wqkv, Wo, Wi, Wout;
+        const float *Wqkv, *Wo, *Wi, *Wout;   // packed
     };
     std::vector<Layer> L_;
     const float *tok_ = nullptr, *on_ = nullptr;

@@ -360,20 +360,19 @@ int launch_split3(const float *x, long long rows, int C, half_t *out, hipStream_
 // y [T][OC] = conv(snake(x), W [OC][C][KK], pad), no bias; x [T][C] f32, OC in {1, 2, 4}, KK == 7, C % 8 == 0
 int launch_conv_out(const float *x, const float *ab, const float *W, float *y, int T, int C, int OC, int KK, int pad,
                     hipStream_t st);
-// Text encoders (enc.hip). GEMM operands are pairs of f16 parts of rows divided by a power of two, packed
-// by their producer; a GEMM leaves the sums of its K splits, which the next kernel adds in order.
+// Text encoders (enc.hip). GEMM operands are f32 values as three bf16 parts (exact), packed by their
+// producer; a GEMM leaves the sums of its K splits, which the next kernel adds in order.
 // 16-row blocks of a packed operand of M <= 128 rows, and its size for K columns
 int enc_row_blocks(int M);
 size_t enc_operand_bytes(int M, int K);
-// size in floats of a packed [N][K] weight (K in whole 64-column steps), and the packing of a row-major
-// one, with its row divisors div[N]
+// size of a packed [N][K] f32 weight (K in whole 64-column steps), and the packing of a row-major one
 size_t enc_weight_floats(int N, int K);
-int launch_enc_weight_pack(const float *src, half_t *dst, float *div, int N, int K, hipStream_t st);
+int launch_enc_weight_pack(const float *src, float *dst, int N, int K, hipStream_t st);
 // ws[z][M][N] = the sums over K split z of A[M][K] W[N][K]^T; M <= 128, N % 64 == 0, K % 32 == 0.
 // The launcher chooses at most `most` splits, and kps (64-column K steps per split).
 struct EncGemmArgs {
-    const half_t *Ap; const float *adiv;   // rows and their divisors
-    const half_t *W; const float *wdiv;
+    const uint16_t *Ap;
+    const float *W;
     float *ws; size_t ws_bytes;
     int M, N, K;
     int most;
@@ -388,26 +387,25 @@ struct EncParts {
     const float *bias;
 };
 // xout = x + parts (when parts.ws), then LayerNorm with weight and bias (ln) or RMSNorm with weight,
-// rows of H floats, as f32 rows y or the packed operand Ap with its divisors adiv
+// rows of H floats, as f32 rows y or the packed operand Ap
 struct EncNormArgs {
     const float *x; float *xout;
     EncParts parts;
     const float *w, *b;
     float *y;
-    half_t *Ap; float *adiv; int mt;
+    uint16_t *Ap; int mt;
     int rows, H;
     float eps;
 };
 int launch_enc_norm(const EncNormArgs &a, bool ln, hipStream_t st);
 int launch_enc_norm_rows(const float *x, float *y, const float *w, const float *b, int rows, int H, float eps, bool ln,
                          hipStream_t st);
-// attention over one context of S <= 128 rows [q | k | v] of nh heads of 64, output packed, every row
-// divided by odiv[0] (a bound of the values: an output is a mean of v rows);
+// attention over one context of S <= 128 rows [q | k | v] of nh heads of 64, output packed;
 // mode 1 T5 (keys whose bit of `keys` is clear masked, else + rel[h*(2S - 1) + k - q + S - 1]),
 // 2 CLIP (keys k > q or k > eot masked)
 struct EncAttnArgs {
     EncParts qkv;
-    half_t *Ap; const float *odiv; int mt;
+    uint16_t *Ap; int mt;
     int S, nh;
     float scale;
     int mode;
@@ -417,7 +415,7 @@ struct EncAttnArgs {
 };
 int launch_enc_attention(const EncAttnArgs &a, hipStream_t st);
 // packed operand of F columns: quick GELU of the F result columns, or gelu_tanh(column c) * column F + c
-int launch_enc_act(const EncParts &p, bool geglu, half_t *Ap, float *adiv, int rows, int F, hipStream_t st);
+int launch_enc_act(const EncParts &p, bool geglu, uint16_t *Ap, int rows, int F, hipStream_t st);
 // x[s][:] = tok[ids[s]][:] (+ pos[s][:]); each id inside tok's rows
 struct EncIds {
     int32_t id[128];
