@@ -481,7 +481,8 @@ def test_attention_pack_alignment(tsn, rt, S):
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 1023, 1024, 1027])
 def test_copy_and_mean_edges(tsn, rt, n):
     """Copies of every n % 4 at 16-byte and 4-byte alignment that leave the element after them alone; row
-    means around the groups of 8 rows and 32 columns. The mean of n f32 values: n roundings of 2^-24."""
+    means around the 64 rows and 32 columns of a step, rows summed in order: every bit that of the f32 sum
+    row after row."""
     x = rng(n).standard_normal(n + 5).astype(np.float32)
     dx = rt.array(x)
 
@@ -496,13 +497,15 @@ def test_copy_and_mean_edges(tsn, rt, n):
         got = y.numpy()
         assert np.array_equal(got[off:off + n], x[off:off + n])
         assert np.all(got[:off] == 7.0) and np.all(got[off + n:] == 7.0)
-    for rows, H in ((1, n), (7, 33), (8, 32), (9, 31), (n, 40)):
+    for rows, H in ((1, n), (7, 33), (8, 32), (9, 31), (63, 40), (64, 64), (65, 40), (129, 33), (n, 40)):
         m = rng(rows + H).standard_normal((rows, H)).astype(np.float32)
         out = rt.empty((H,))
         rt.mean_cols(rt.array(m), out, rows, H)
         rt.sync()
-        bound = rows * 2.0 ** -24 * np.abs(m).mean(0) + 1e-7 * np.abs(m.mean(0))
-        assert np.all(np.abs(out.numpy() - m.astype(np.float64).mean(0)) <= bound + 1e-30)
+        acc = np.zeros(H, np.float32)
+        for row in m:
+            acc += row
+        assert np.array_equal(out.numpy().view(np.uint32), (acc / np.float32(rows)).view(np.uint32)), (rows, H)
 
 
 @pytest.mark.parametrize("M", [1, 31, 33, 64, 65, 96, 97, 128, 129])
