@@ -28,6 +28,14 @@ def orc():
 
 
 @pytest.fixture(scope="session")
+def plan(tsn, tmp_path_factory):
+    """gemm_plan on the host (tests/gemm_plan.cpp)"""
+    import gemm_plan
+    exe = gemm_plan.build(tmp_path_factory.mktemp("plan"))
+    return lambda *a, **k: gemm_plan.ask(exe, *a, **k)
+
+
+@pytest.fixture(scope="session")
 def rt(tsn):
     r = tsn.Runtime(0)
     yield r

@@ -1984,7 +1984,7 @@ static bool hl2_plan(GemmBatch &b, int epi) {
     double best = 1e30;
     int best_mb = 0, best_s = 1;
     for (int mb = 2; mb <= 8; mb += 2)
-        for (int s = 1; s <= (can_split ? nkmin / 8 : 1); ++s) {
+        for (int s = 1; s <= std::max(1, can_split ? nkmin / 8 : 1); ++s) {   // a K too short to split is planned whole
             long long wg = 0;
             int nk = 0;
             double part = 0;
