@@ -115,3 +115,43 @@ def test_vae_gguf_load(tsn, rt, tmp_path):
     finally:
         a_m.close()
         b_m.close()
+
+
+def test_vae_conv_sums_keep_the_small_products(tsn, rt):
+    """A decoder that is the identity (stride 1, one unit tap, snakes of zero amplitude) up to its last k1
+    conv, whose sums are one large product and 63 of about 2^-4. The f16 remainders of either operand add
+    0.375 ulp of the large sum per 32 channels, 1.5 ulp in all: they have to be summed on their own, not each
+    lost in the large sum. Two roundings of half an ulp (the two sums together, the residual)."""
+    C = 64
+    spec = tsn.vae_spec_for_duration(1).copy(T=3, latent=C, width=[C] * 6, stride=[1] * 5, kt=[2] * 5)
+    w = np.zeros(sum(k for _, k, _ in tsn.vae_manifest(spec)), np.float32)
+    v = {n: w[o:o + k] for n, k, o in tsn.vae_manifest(spec)}
+    eye, small = np.eye(C, dtype=np.float32), np.float32(1 + 0.75 * 2.0 ** -11)
+    for n, a in v.items():
+        if n.endswith(".beta"):
+            a[:] = 200.0   # exp(-200): no snake
+    v["decoder.layers.0.weight"].reshape(C, C, 7)[:, :, 3] = eye
+    for n in range(1, 6):
+        v["decoder.layers.%d.layers.1.weight" % n].reshape(C, C, 2)[:, :, 1] = eye
+    v["decoder.layers.5.layers.4.layers.1.weight"].reshape(C, C, 7)[:, :, 3] = eye
+    last = v["decoder.layers.5.layers.4.layers.3.weight"].reshape(C, C)
+    last[1:3] = small
+    last[1:3, 0] = 1.0
+    out = v["decoder.layers.7.weight"].reshape(2, C, 7)
+    out[0, 1, 3] = out[1, 2, 3] = 1.0   # the audio is channels 1 and 2
+    x = np.full((3, C), small / 16, np.float32)
+    x[:, 0] = 2.0 ** 14
+    x[1] *= -1
+    x64 = x.astype(np.float64)
+    want = (x64 + x64 @ last.astype(np.float64).T)[:, 1:3]
+    m = tsn.VaeModel(rt, spec)
+    try:
+        m.upload_weights(w)
+        audio = rt.empty((3, 2))
+        m.decode(rt.array(x), audio)
+        rt.sync()
+        err = np.abs(audio.numpy() - want) / 2.0 ** -9   # ulps of 2^14 .. 2^15
+        print("ulps", err.ravel())
+        assert err.max() <= 1.0
+    finally:
+        m.close()

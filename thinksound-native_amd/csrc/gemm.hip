@@ -791,7 +791,9 @@ __device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, i
     // [W_hi | W_hi | W_lo] every part that enters two products was staged and read from LDS twice
     // (18 fragments and 48 KB per 24 MFMAs of a wave against 12 and 32 KB now), and the loop is bound
     // by those: 8 s decode 4.40 -> 3.41 ms, 1 s 1.07 -> 0.89 ms (same box; operand rows also shrink
-    // from 6 to 4 bytes a value).
+    // from 6 to 4 bytes a value). Products with a lo part have accumulators of their own, so the sum of
+    // the hi products rounds once per 32 channels: error of a decode against 64 bits 4.5e-6 -> 4.2e-6
+    // (three parts: 4.4e-6), same time.
     constexpr bool chunk_major = EPI == EPI_SNAKE || EPI == EPI_RSNAKE, pairs = chunk_major;
     const int dil = EPI == EPI_SNAKE ? P.dil : 1;   // dilated taps only in the snake-conv kernels
     const int taps = P.taps;
@@ -854,10 +856,11 @@ __device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, i
         }
     };
 
+    floatx4 low[2][4];   // pairs: the products with a lo part
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 4; ++j) acc[i][j] = low[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     const int wm = wave >> 1, wn = wave & 1;
     // operand read offsets (halves) inside a stage, per half kh of the 64 staged columns: slot
@@ -893,8 +896,10 @@ __device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, i
 #pragma unroll
                 for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[q == 1][i], bf[q / 2][j], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < 4; ++j) {
+                        floatx4 &d = pairs && q > 0 ? low[i][j] : acc[i][j];
+                        d = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[q == 1][i], bf[q / 2][j], d, 0, 0, 0);
+                    }
             return;
         }
 #pragma unroll
@@ -954,6 +959,12 @@ __device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, i
             block_barrier();
             if (kt + NST < nk) issue(kt + NST, st);
         }
+    }
+    if constexpr (pairs) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[i][j] += low[i][j];
     }
 }
 
@@ -1114,9 +1125,10 @@ template <int EPI>
 __global__ __launch_bounds__(512, 2) void gemm_pipe2_bf16_kernel(const GemmBatch bt) {
     pipe_dp<EPI, false, 2, true>(bt);
 }
-// two LDS stages, two workgroups per CU (grids of several rounds)
+// two LDS stages, two workgroups per CU (grids of several rounds), which is at most 128 registers: the
+// snake kernels, with two accumulators, are held to that
 template <int EPI>
-__global__ __launch_bounds__(512, 2) void gemm_pipe2_kernel(const GemmBatch bt) {
+__global__ __launch_bounds__(512, EPI == EPI_SNAKE || EPI == EPI_RSNAKE ? 4 : 2) void gemm_pipe2_kernel(const GemmBatch bt) {
     pipe_dp<EPI, false, 2>(bt);
 }
 template <int EPI>
