@@ -747,7 +747,8 @@ constexpr int hl_stages(int nsx) { return nsx == 2 ? 3 : 6; }
 // fragment reads per 16 MFMAs of a wave.
 template <int EPI, bool HLP, int NSX, bool BF>
 __device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, int m0, int n0, int kbeg, int nk, int tid,
-                                           floatx4 (&acc)[2][4]) {
+                                           floatx4 (&out)[2][4]) {
+    floatx4 acc[2][4];
     constexpr int NST = HLP ? hl_stages(NSX) : NSX;          // stages
     constexpr int WST = HLP ? STAGE / 2 : STAGE;             // halves of a W stage
     constexpr int LPT = HLP ? 3 : 4;                         // DMAs per wave per K tile
@@ -845,7 +846,8 @@ __device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, i
             nt_trow += dil;
             nt_kw += Kc;
         }
-        const unsigned sa = ldsa + stage * STAGE * 2, sb = ldsb + stage * WST * 2;
+        // plain tiles: both operands from one base
+        const unsigned sa = ldsa + stage * STAGE * 2, sb = HLP ? ldsb + stage * WST * 2 : ldsa + (NST + stage) * STAGE * 2;
 #pragma unroll
         for (int i = 0; i < 2; ++i) dma16s(rsa, va[i], (unsigned)kin * 2, sa + i * 1024);
 #pragma unroll
@@ -960,12 +962,10 @@ __device__ __forceinline__ void pipe_kloop(const GemmProblem &P, half_t *smem, i
             if (kt + NST < nk) issue(kt + NST, st);
         }
     }
-    if constexpr (pairs) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] += low[i][j];
-    }
+        for (int j = 0; j < 4; ++j) out[i][j] = pairs ? acc[i][j] + low[i][j] : acc[i][j];
 }
 
 // One C tile over the K tiles [kbeg, kbeg + nk): the K loop,
