@@ -157,6 +157,27 @@ __device__ inline int attn_xcd_remap(int bid, int nwg) {
     return (xcd < rem ? xcd * (base + 1) : rem * (base + 1) + (xcd - rem) * base) + idx;
 }
 
+// Columns d0 .. d0 + 3 of query q's head (column hc on) at element e of O. Whether any row is paired is the same
+// for every workgroup of a launch, so launches without one branch past the per-lane test.
+__device__ __forceinline__ void store_o4(const AttnArgs &a, long long e, int hc, int d0, int q, float y0, float y1, float y2,
+                                         float y3) {
+    if (a.o_f32) {
+        *(float4 *)((float *)a.O + e) = make_float4(y0, y1, y2, y3);
+        return;
+    }
+    half_t *op = (half_t *)a.O + e;
+    if (a.o_pair && q < a.o_pair) {   // paired row: the head's 64 columns are 128 halves, the f16 remainder PAIR further
+        const float y4[4] = {y0, y1, y2, y3};
+        half4 hi, lo;
+        split_parts4(y4, hi, lo);
+        op += hc + (d0 & PAIR);
+        *(half4 *)op = hi;
+        *(half4 *)(op + PAIR) = lo;
+    } else {
+        *(half4 *)op = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
+    }
+}
+
 // NSTG stages of two key blocks each: 4 (128 KB, one workgroup per CU; up to 512 keys, all loaded
 // at once) or 2 (a 64 KB ring, two workgroups per CU, one pair of key blocks in flight while the
 // other is multiplied; for longer contexts, where the second workgroup covers the load latency)
@@ -453,23 +474,7 @@ __global__ __launch_bounds__(512, NSTG == 2 ? 2 : 1) void flash_attn_kernel(cons
             const int dt = 2 * half + j;
             const float (&od)[4] = om[j];
             const int d0 = dt * 16 + g * 4;
-            if (a.o_f32) {
-                float *op = (float *)a.O + orow + d0;
-                *(float4 *)op = make_float4(od[0] * inv, od[1] * inv, od[2] * inv, od[3] * inv);
-            } else {
-                const bool pair = q < a.o_pair;   // paired row: head h's 64 columns are 128 halves
-                half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
-                const float y0 = od[0] * inv, y1 = od[1] * inv, y2 = od[2] * inv, y3 = od[3] * inv;
-                if (pair) {   // the f16 remainder: hi + lo carries the f32 value
-                    const float y4[4] = {y0, y1, y2, y3};
-                    half4 hi, lo;
-                    split_parts4(y4, hi, lo);
-                    *(half4 *)op = hi;
-                    *(half4 *)(op + PAIR) = lo;
-                } else {
-                    *(half4 *)op = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-                }
-            }
+            store_o4(a, orow + d0, h * 64, d0, q, od[0] * inv, od[1] * inv, od[2] * inv, od[3] * inv);
         }
     }
 }
@@ -610,23 +615,7 @@ __global__ __launch_bounds__(256, 3) void flash_attn4_kernel(const AttnArgs a) {
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) {
             const int d0 = dt * 16 + g * 4;
-            if (a.o_f32) {
-                float *op = (float *)a.O + orow + d0;
-                *(float4 *)op = make_float4(o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
-            } else {
-                const bool pair = q < a.o_pair;
-                half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
-                const float y0 = o[dt][0] * inv, y1 = o[dt][1] * inv, y2 = o[dt][2] * inv, y3 = o[dt][3] * inv;
-                if (pair) {
-                    const float y4[4] = {y0, y1, y2, y3};
-                    half4 hi, lo;
-                    split_parts4(y4, hi, lo);
-                    *(half4 *)op = hi;
-                    *(half4 *)(op + PAIR) = lo;
-                } else {
-                    *(half4 *)op = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-                }
-            }
+            store_o4(a, orow + d0, h * 64, d0, q, o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
         }
     }
 }
@@ -776,23 +765,7 @@ __global__ __launch_bounds__(256, 3) void flash_attn4q2_kernel(const AttnArgs a)
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) {
             const int d0 = dt * 16 + g * 4;
-            if (a.o_f32) {
-                float *op = (float *)a.O + orow + d0;
-                *(float4 *)op = make_float4(o[u][dt][0] * inv, o[u][dt][1] * inv, o[u][dt][2] * inv, o[u][dt][3] * inv);
-            } else {
-                const bool pair = q[u] < a.o_pair;
-                half_t *op = (half_t *)a.O + orow + d0 + (pair ? h * 64 + (d0 & PAIR) : 0);
-                const float y0 = o[u][dt][0] * inv, y1 = o[u][dt][1] * inv, y2 = o[u][dt][2] * inv, y3 = o[u][dt][3] * inv;
-                if (pair) {
-                    const float y4[4] = {y0, y1, y2, y3};
-                    half4 hi, lo;
-                    split_parts4(y4, hi, lo);
-                    *(half4 *)op = hi;
-                    *(half4 *)(op + PAIR) = lo;
-                } else {
-                    *(half4 *)op = half4{(half_t)y0, (half_t)y1, (half_t)y2, (half_t)y3};
-                }
-            }
+            store_o4(a, orow + d0, h * 64, d0, q[u], o[u][dt][0] * inv, o[u][dt][1] * inv, o[u][dt][2] * inv, o[u][dt][3] * inv);
         }
     }
 }
