@@ -21,10 +21,10 @@ def build(out_dir):
 
 
 def ask(exe, epi, probs, ws=40 << 20, pair=0, half=1, split_waves=0, counters=1 << 16):
-    """Plan of a batch of (M, N, K, taps) problems; height: rows of a tile of the one-round hi|lo kernel, or 0."""
+    """Plan of a batch of (M, N, K, taps[, half, pair]) problems; height: rows of a tile of the one-round hi|lo kernel, or 0."""
     line = "%d %d %d %d %d" % (epi, ws, split_waves, counters, len(probs))
     for p in probs:
-        line += " %d %d %d %d %d %d" % (tuple(p) + (half, pair))
+        line += " %d %d %d %d %d %d" % (tuple(p) + (half, pair)[len(p) - 4:])
     r = subprocess.run([exe], input=line + "\n", capture_output=True, text=True, check=True)
     rc, name, hl2, sk, splits, tiles = r.stdout.split("\n")[0].rsplit(" ", 5)
     assert rc == "0", r.stdout

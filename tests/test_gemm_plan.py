@@ -1,6 +1,6 @@
 """The GEMM planner (gemm_plan) on the host: which kernel, tile height and K split a batch gets. The GPU tests of the
 kernels take their sizes from plans that are asserted here or there, so that they run what they name."""
-from gemm_plan import QKV, RESID, STORE, SWIGLU
+from gemm_plan import QKV, RSNAKE, SNAKE, STORE, SWIGLU
 
 
 def test_input_projection_fits_one_round(plan):
@@ -16,3 +16,17 @@ def test_one_step_fits_one_round(plan):
         for pair in (0, 1):
             p = plan(STORE, [(33, 128, 128, 1)], ws=ws, pair=pair)
             assert p.kernel == "gemm_hl2_kernel<0>" and p.splits == 1, (ws, pair, p)
+
+
+def test_stream_k_kernels(plan):
+    """Stream-K: plain batches run the kernel with the plain K loop alone, a batch with one half-width-W problem
+    the one with both; the snake convs never stream."""
+    for epi in (QKV, SWIGLU):   # 297 tiles: a second round of 41
+        p = plan(epi, [(384, 99 * 128, 1024, 1)], half=0)
+        assert p.sk == 1 and p.kernel == "gemm_sk_kernel<%d>" % epi, p
+    mixed = [(344, 5632, 2048 * 3, 3, 1, 1), (308, 5632, 1024, 1, 0, 0)]
+    p = plan(SWIGLU, mixed)
+    assert p.sk == 1 and p.kernel == "gemm_sk_hl_kernel<3>", p
+    for epi in (SNAKE, RSNAKE):
+        p = plan(epi, [(200, 1024, 8192, 1)], half=0)
+        assert p.sk == 0 and p.kernel == "gemm_pipe_kernel<%d>" % epi, p

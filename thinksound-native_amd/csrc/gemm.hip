@@ -22,7 +22,7 @@
 //    five (two workgroups per CU), three per group (one per CU) or three (three per CU, for grids
 //    past 512 tiles); residual epilogue in place or plain store, for GEMMs whose 128x128 grid
 //    cannot fill one round of the chip.
-//  * gemm_sk_kernel + gemm_fixup_kernel: stream-K over (tile, K tile) units, with the cut tiles
+//  * gemm_sk_kernel, gemm_sk_hl_kernel (batches with a half-width W) + gemm_fixup_kernel: stream-K over (tile, K tile) units, with the cut tiles
 //    finished in-kernel by their last contributor or by the fixup launch.
 //  * splitk_reduce_kernel: classic split-K sum in split order, then the epilogue.
 //  * gemm_f16_kernel: register-staged 256-thread kernel (4 waves of 64x64, two padded LDS stages)
@@ -1769,8 +1769,9 @@ __device__ __forceinline__ long long sk_owner(long long u, long long U, long lon
     return w;
 }
 
-template <int EPI>
-__global__ __launch_bounds__(512, 1) void gemm_sk_kernel(const GemmBatch bt) {
+// HL: the batch has a half-width-W problem (two K loops; plain batches keep the one they use)
+template <int EPI, bool HL>
+__device__ __forceinline__ void sk_tiles(const GemmBatch &bt) {
     const int tid = threadIdx.x;
     const int wg = xcd_remap(blockIdx.x, gridDim.x);
     const long long U = bt.sk_units, G = gridDim.x;
@@ -1799,12 +1800,21 @@ __global__ __launch_bounds__(512, 1) void gemm_sk_kernel(const GemmBatch bt) {
             fx.a = a;
             fx.w0 = sk_owner(a, U, G);
             fx.nc = (int)(sk_owner(b - 1, U, G) - fx.w0 + 1);
-            pipe_tile<EPI, true, true>(P, tm * BM, tn * BN, kbeg, nk, part, 0, tid, &fx);
+            pipe_tile<EPI, HL, true>(P, tm * BM, tn * BN, kbeg, nk, part, 0, tid, &fx);
         } else {
-            pipe_tile<EPI, true, true>(P, tm * BM, tn * BN, kbeg, nk, part, 0, tid);
+            pipe_tile<EPI, HL, true>(P, tm * BM, tn * BN, kbeg, nk, part, 0, tid);
         }
         u += nk;
     }
+}
+
+template <int EPI>
+__global__ __launch_bounds__(512, 1) void gemm_sk_kernel(const GemmBatch bt) {
+    sk_tiles<EPI, false>(bt);
+}
+template <int EPI>
+__global__ __launch_bounds__(512, 1) void gemm_sk_hl_kernel(const GemmBatch bt) {
+    sk_tiles<EPI, true>(bt);
 }
 
 // Stream-K fixup: one workgroup per tile of the batch; tiles cut by a workgroup boundary sum their
@@ -1934,8 +1944,6 @@ int launch_gemm_reduce(const GemmBatch &b, int epi, hipStream_t st) {
         if (epi == EPI_STORE) TSN_LAUNCH((gemm_fixup_kernel<EPI_STORE>), grid, block, 0, st, b);
         else if (epi == EPI_RESID) TSN_LAUNCH((gemm_fixup_kernel<EPI_RESID>), grid, block, 0, st, b);
         else if (epi == EPI_QKV) TSN_LAUNCH((gemm_fixup_kernel<EPI_QKV>), grid, block, 0, st, b);
-        else if (epi == EPI_SNAKE) TSN_LAUNCH((gemm_fixup_kernel<EPI_SNAKE>), grid, block, 0, st, b);
-        else if (epi == EPI_RSNAKE) TSN_LAUNCH((gemm_fixup_kernel<EPI_RSNAKE>), grid, block, 0, st, b);
         else TSN_LAUNCH((gemm_fixup_kernel<EPI_SWIGLU>), grid, block, 0, st, b);
         TSN_HIP_CHECK(hipGetLastError());
         return TSN_OK;
@@ -1964,8 +1972,7 @@ bool gemm_needs_reduce(const GemmBatch &b) {
 const char *gemm_reduce_name(const GemmBatch &b, int epi) {
     if (b.sk)
         return epi == EPI_STORE ? "gemm_fixup_kernel<0>" : epi == EPI_RESID ? "gemm_fixup_kernel<1>"
-               : epi == EPI_QKV ? "gemm_fixup_kernel<2>" : epi == EPI_SNAKE ? "gemm_fixup_kernel<4>"
-               : epi == EPI_RSNAKE ? "gemm_fixup_kernel<5>" : "gemm_fixup_kernel<3>";
+               : epi == EPI_QKV ? "gemm_fixup_kernel<2>" : "gemm_fixup_kernel<3>";
     return epi == EPI_RESID ? "splitk_reduce_kernel<1>" : epi == EPI_RSNAKE ? "splitk_reduce_kernel<5>"
            : epi == EPI_SNAKE ? "splitk_reduce_kernel<4>" : "splitk_reduce_kernel<0>";
 }
@@ -2276,8 +2283,9 @@ int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
     // Stream-K when the grid chosen above leaves CUs idle. Estimated critical path in K tiles:
     // that grid = waves * longest K range per workgroup (+2 for a split-K reduce); stream-K = units
     // per workgroup + pipeline fill, partial store and fixup.
+    // The snake convs never stream: a classic split keeps their long K's W and A tiles shared in L2.
     b.sk = 0;
-    if (pipe && b.ws && !b.split_waves) {
+    if (pipe && b.ws && !b.split_waves && !snake_epi) {
         long long units = 0, cur = 0;
         int nkmax = 0, split = 0;
         for (int i = 0; i < b.nprob; ++i) {
@@ -2312,9 +2320,10 @@ int gemm_plan(GemmBatch &b, int epi, bool a_f32) {
     b.pipe = pipe ? 1 : 0;
     b.hl = any_half ? 1 : 0;
     TSN_REQUIRE((epi != EPI_SNAKE && epi != EPI_RSNAKE) || !b.hl, "gemm snake: no half-width W");
-    b.kname = b.sk ? (epi == EPI_STORE ? "gemm_sk_kernel<0>" : epi == EPI_RESID ? "gemm_sk_kernel<1>"
-                      : epi == EPI_QKV ? "gemm_sk_kernel<2>" : epi == EPI_SNAKE ? "gemm_sk_kernel<4>"
-                      : epi == EPI_RSNAKE ? "gemm_sk_kernel<5>" : "gemm_sk_kernel<3>")
+    b.kname = b.sk && b.hl ? (epi == EPI_STORE ? "gemm_sk_hl_kernel<0>" : epi == EPI_RESID ? "gemm_sk_hl_kernel<1>"
+                              : epi == EPI_QKV ? "gemm_sk_hl_kernel<2>" : "gemm_sk_hl_kernel<3>")
+            : b.sk ? (epi == EPI_STORE ? "gemm_sk_kernel<0>" : epi == EPI_RESID ? "gemm_sk_kernel<1>"
+                      : epi == EPI_QKV ? "gemm_sk_kernel<2>" : "gemm_sk_kernel<3>")
             : pipe && b.hl ? (epi == EPI_STORE ? "gemm_pipe_hl_kernel<0>" : epi == EPI_RESID ? "gemm_pipe_hl_kernel<1>"
                               : epi == EPI_QKV ? "gemm_pipe_hl_kernel<2>" : "gemm_pipe_hl_kernel<3>")
             : pipe ? (epi == EPI_STORE ? "gemm_pipe_kernel<0>" : epi == EPI_RESID ? "gemm_pipe_kernel<1>"
@@ -2430,13 +2439,17 @@ int gemm_launch_planned(const GemmBatch &b, int epi, bool a_f32, hipStream_t st)
         return TSN_OK;
     }
     if (b.pipe) {
-        if (b.sk) {
+        if (b.sk && b.hl) {
+            if (epi == EPI_STORE) TSN_LAUNCH((gemm_sk_hl_kernel<EPI_STORE>), grid, block, 0, st, b);
+            else if (epi == EPI_RESID) TSN_LAUNCH((gemm_sk_hl_kernel<EPI_RESID>), grid, block, 0, st, b);
+            else if (epi == EPI_QKV) TSN_LAUNCH((gemm_sk_hl_kernel<EPI_QKV>), grid, block, 0, st, b);
+            else if (epi == EPI_SWIGLU) TSN_LAUNCH((gemm_sk_hl_kernel<EPI_SWIGLU>), grid, block, 0, st, b);
+            else { set_error("gemm: unknown epilogue"); return TSN_ERR_ARG; }
+        } else if (b.sk) {
             if (epi == EPI_STORE) TSN_LAUNCH((gemm_sk_kernel<EPI_STORE>), grid, block, 0, st, b);
             else if (epi == EPI_RESID) TSN_LAUNCH((gemm_sk_kernel<EPI_RESID>), grid, block, 0, st, b);
             else if (epi == EPI_QKV) TSN_LAUNCH((gemm_sk_kernel<EPI_QKV>), grid, block, 0, st, b);
             else if (epi == EPI_SWIGLU) TSN_LAUNCH((gemm_sk_kernel<EPI_SWIGLU>), grid, block, 0, st, b);
-            else if (epi == EPI_SNAKE) TSN_LAUNCH((gemm_sk_kernel<EPI_SNAKE>), grid, block, 0, st, b);
-            else if (epi == EPI_RSNAKE) TSN_LAUNCH((gemm_sk_kernel<EPI_RSNAKE>), grid, block, 0, st, b);
             else { set_error("gemm: unknown epilogue"); return TSN_ERR_ARG; }
         } else if (b.hl && b.ns2) {
             if (epi == EPI_STORE) TSN_LAUNCH((gemm_pipe2_hl_kernel<EPI_STORE>), grid, block, 0, st, b);
