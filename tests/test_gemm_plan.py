@@ -22,7 +22,7 @@ def test_stream_k_kernels(plan):
     """Stream-K: plain batches run the kernel with the plain K loop alone, a batch with one half-width-W problem
     the one with both; the snake convs never stream."""
     for epi in (QKV, SWIGLU):   # 297 tiles: a second round of 41
-        p = plan(epi, [(384, 99 * 128, 1024, 1)], half=0)
+        p = plan(epi, [(384, 99 * 128, 4096, 1)], half=0)
         assert p.sk == 1 and p.kernel == "gemm_sk_kernel<%d>" % epi, p
     mixed = [(344, 5632, 2048 * 3, 3, 1, 1), (308, 5632, 1024, 1, 0, 0)]
     p = plan(SWIGLU, mixed)
