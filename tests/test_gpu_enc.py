@@ -149,8 +149,9 @@ def test_encoders_gguf_load(tsn, rt, tmp_path):
 def test_encoder_gemm_edges(tsn, rt, orc, ctx, scale):
     """Row-block edges of the GEMMs (16-row MFMA blocks, the 32-, 80- and 128-row tiles), a K that ends half
     way through a 64-column step (d_ff = 96, 352) and, with scale, T5 FFN activations of about scale^2
-    (past the f16 range) and rows of one weight 2^-20 of the others. f32 against f32: three layers
-    amplify a rounding-level difference (6e-8) by less than 50."""
+    (past the f16 range) and rows of one weight 2^-20 of the others (k rows of a head, whose q rows are 2^20
+    larger, so that its scores keep their size). f32 against f32: three layers amplify a rounding-level
+    difference (6e-8) by less than 50."""
     ts = tsn.t5_spec_default().copy(d=192, d_ff=352 if ctx % 2 else 96, NL=3, NH=3, ctx=ctx, vocab=200)
     cs = tsn.clip_spec_default().copy(H=192, NL=3, NH=3, ctx=ctx, vocab=300)
     tw, cw = tsn.t5_synth_weights(ts, 31).copy(), tsn.clip_synth_weights(cs, 32).copy()
@@ -161,6 +162,8 @@ def test_encoder_gemm_edges(tsn, rt, orc, ctx, scale):
             tw[off:off + n] /= scale * scale
         elif name.endswith(".k") and scale != 1.0:
             tw[off:off + 64 * ts.d] *= 2.0 ** -20
+        elif name.endswith(".q") and scale != 1.0:
+            tw[off:off + 64 * ts.d] *= 2.0 ** 20
     r = rng(ctx)
     tids, cids = r.integers(2, 200, ctx).astype(np.int32), r.integers(0, 300, ctx).astype(np.int32)
     tids[ctx // 2 + 1:] = 0

@@ -11,6 +11,7 @@ rel-L2 <= 1e-5.
 import numpy as np
 import pytest
 
+import gemm_plan
 from conftest import f16r, rel_l2, rng
 
 pytestmark = pytest.mark.gpu
@@ -508,12 +509,13 @@ def test_copy_and_mean_edges(tsn, rt, n):
         assert np.array_equal(out.numpy().view(np.uint32), (acc / np.float32(rows)).view(np.uint32)), (rows, H)
 
 
-@pytest.mark.parametrize("M", [1, 31, 33, 64, 65, 96, 97, 128, 129])
-@pytest.mark.parametrize("N,K", [(8, 64), (128, 128), (136, 1088), (1024, 4096)])
+@pytest.mark.parametrize("M,N,K", [(m, 4096, k) for m, _ in gemm_plan.STORE_ROWS for k in gemm_plan.STORE_KS] +
+                         [c[:3] for c in gemm_plan.STORE_OTHER])
 def test_gemm_hilo_one_round_edges(tsn, rt, M, N, K):
-    """One-round hi|lo grids around the 32- to 128-row tiles, one K step, an odd number of steps, a ragged
-    column tile and (N = 1024) K splits. Against 64 bits: the parts carry 22 bits (2.4e-7 of a value),
-    and 32-bit sums of K / 32 terms add less than 3e-7 here."""
+    """One-round hi|lo grids around the edges of the 32-, 64-, 96- and 128-row tiles, one K step, odd numbers of
+    steps, a ragged column tile and K splits (the plan of every size is asserted in test_gemm_plan.py).
+    Against 64 bits: the parts carry 22 bits (2.4e-7 of a value), and 32-bit sums of K / 32 terms add less
+    than 3e-7 here."""
     r = rng(M * 7 + K)
     X = r.standard_normal((M, K)).astype(np.float32)
     W = (r.standard_normal((N, K)) * 0.03).astype(np.float16)

@@ -18,6 +18,7 @@ import numpy as np
 import pytest
 
 from conftest import rel_l2
+from gemm_plan import REF_ROWS
 
 pytestmark = pytest.mark.gpu
 
@@ -220,3 +221,26 @@ def test_ref_replay_refused_after_sampler_reallocation(tsn, rt, ref):
     m.replay()
     rt.sync()
     assert np.array_equal(xc.numpy().view(np.uint32), eager3.view(np.uint32))
+
+
+@pytest.mark.parametrize("T,n_joint", [(t, 0) for t in REF_ROWS] + [(451, 1)])
+def test_ref_block_rows(tsn, rt, orc, T, n_joint):
+    """A fused block (and a joint one) at latent lengths whose GEMMs take 32-, 64-, 96- and 128-row tiles of the
+    one-round kernel with ragged last tiles, and past one round the multi-round paired kernels and stream-K
+    (plans asserted in test_gemm_plan.py)."""
+    spec = tsn.ref_spec_for_duration(8, 1).copy(T=T, C=30, TS=77, n_joint=n_joint, n_fused=1)
+    w16 = tsn.ref_synth_weights(spec, 4242, 1.0)
+    m = tsn.RefDitModel(rt, spec)
+    try:
+        m.upload_weights(w16)
+        inp, dev = _io(tsn, rt, spec, seed=T)
+        S = spec.T + spec.C + spec.TS
+        taps = rt.empty((n_joint + 1, 1, S, spec.H))
+        v = _fwd(m, rt, spec, dev, taps).numpy()
+        vr, tr = orc.ref_dit_forward(spec.as_dict(), tsn.bf16_to_f32(w16), taps=True, **inp)
+        tg = taps.numpy()
+        err, blk = rel_l2(v, vr), max(rel_l2(a[:, :T], b[:, :T]) for a, b in zip(tg, tr))
+        print("T %d: velocity rel-L2 %.3g, worst block %.3g" % (T, err, blk))
+        assert err <= 1e-3 and blk <= 2e-3
+    finally:
+        m.close()
