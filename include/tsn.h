@@ -59,8 +59,8 @@ int tsn_runtime_alloc_stats(tsn_runtime *rt, size_t *count, size_t *bytes);
 /* ---------------- launcher runtime: tn::Runtime (src/net.h:18-51) ---------------- */
 /* Y[M,N] = X[M,K]·W[N,K]^T (+bias[N], f32). Runtime::gemm src/net.h:24-26, src/net.mm:14-23.
  * wdtype TSN_F16 with f32 X keeps the reference's f32-activation contract (gemm_mpp_h,
- * shaders/gemm_mpp.metal:19-25): X is split into an f16 hi|lo pair on the device and multiplied
- * against [W | W] on MFMA with f32 accumulation, so the product is f32-accurate (relative error
+ * shaders/gemm_mpp.metal:19-25): X is split into f16 hi|lo pairs on the device and both parts
+ * multiplied by W on MFMA with f32 accumulation, so the product is f32-accurate (relative error
  * about 2^-22 of the operand, against 2^-11 for an f16-rounded X). Y f32, or f16 on request. Shapes
  * the MFMA tiling does not take (K % 64, N % 8, unaligned W/bias/Y) run exact f32 products on the
  * SIMT path (f32 Y only). wdtype TSN_F16 with f16 X is the plain f16 product (opt-in, f16 operands

@@ -105,7 +105,7 @@ private:
 
     std::vector<StreamW> ja_, jt_, fu_;
     const uint16_t *Wmod_ = nullptr, *Wt0_ = nullptr, *Wt2_ = nullptr;
-    const half_t *Win2_ = nullptr, *Wfin2_ = nullptr;   // [W|W] f16 for the hi|lo projections
+    const half_t *Win2_ = nullptr, *Wfin2_ = nullptr;   // f16, each column twice, for the hi|lo projections
     const float *bmod_ = nullptr, *bt0_ = nullptr, *bt2_ = nullptr, *bin_ = nullptr, *bfin_ = nullptr;
     int fin_mod_off_ = 0;
     // the final adaLN + projection as one kernel (launch_final_out) where the shapes allow it

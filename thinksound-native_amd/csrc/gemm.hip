@@ -1698,7 +1698,8 @@ __global__ __launch_bounds__(512, 1) void gemm_hl2_kernel(const GemmBatch bt) {
     // has a read phase and a multiply phase, closed by one workgroup barrier each; group 1 runs one
     // barrier behind. When a wave refills the stage of step kt - 1 (in its read phase of step kt), both
     // groups' reads of that stage have ended a barrier earlier or more; its own DMAs of step kt + 1 are
-    // waited for before the read phase's barrier, two barriers before any wave reads that step.
+    // waited for before the read phase's barrier. Group 0's are two barriers ahead of their first reader, group
+    // 1's one: group 0 reads step kt + 1 right after the barrier that ends group 1's read phase of step kt.
     auto wait_left = [&](int n) { wait_tiles<LPT, NST - 2>(n); };   // until only n later steps' DMAs are in flight
     auto phase_end = [&]() {
         __builtin_amdgcn_sched_barrier(0);

@@ -64,7 +64,7 @@ struct GemmProblem {
     // Y[ymap(m)*ldy + 64j + c] = silu(w1 row 64j+c · a) * (w3 row 64j+c · a), f16, no bias
     void *Y; int ldy; RowMap ymap; int y_f16; int silu;
     // f16 Y (EPI_STORE, EPI_SWIGLU): nonzero writes paired rows (hi = f16(y), lo = f16(y - hi)), the A
-    // operand of a following w_half GEMM; K is then never split
+    // operand of a following w_half GEMM (K split, where it is: the reduce writes the pairs)
     int y_pair;
     // EPI_SNAKE, EPI_RSNAKE: A and W rows are paired: every 32 channels as 32 hi halves, then their 32
     // lo halves (Kc = 2*IC), and the product sums hi*W_hi + lo*W_hi + hi*W_lo (the dropped lo*W_lo term

@@ -4,7 +4,7 @@
 // reference launchers (ln_plain, geglu, gelu_quick, qkv_split3).
 //
 // Operand formats for f32-accurate products on f16 MFMA (x f32 in every case):
-//   f16 weights: x as an f16 hi|lo pair, hi = f16(x), lo = f16(x - hi), against [W | W];
+//   f16 weights: x as paired rows (hi = f16(x), lo = f16(x - hi)), both parts against one W;
 //   f32 weights: x as three parts [hi | lo | hi] against [W_hi | W_hi | W_lo]
 //   (hi·W_hi + lo·W_hi + hi·W_lo; the dropped lo·W_lo term is below 2^-22 relative).
 #include "kernels.h"

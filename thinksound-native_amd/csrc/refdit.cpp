@@ -138,7 +138,7 @@ int RefDitModel::create(Runtime *r, const RefDitSpec &sp) {
     TSN_TRY(af(&gc_, B * H));
     TSN_TRY(af(&gs_, B * H));
     TSN_TRY(af(&t_dev, B));
-    TSN_TRY(ah(&XN_, B * S * 2 * H));   // [hi | lo] rows; lo written for latent FFN inputs only
+    TSN_TRY(ah(&XN_, B * S * 2 * H));   // paired or plain rows (refdit.h)
     TSN_TRY(ah(&XE_, B * T * 2 * H));
     TSN_TRY(ah(&Z2_, B * T * 2 * (size_t)s.latent));
     TSN_TRY(ah(&XF2_, B * T * 2 * H));
@@ -617,7 +617,7 @@ int RefDitModel::enqueue_eval(const float *x, const float *t, const float *clip_
         modg_ = MODG_;
     }
     // extended_c = sync_gather + global_c per row, SiLU, as f16 hi|lo; then every per-row modulation
-    // (latent and fused blocks, final layer) in one GEMM with M = B*T against [W | W], f32-accurate
+    // (latent and fused blocks, final layer) in one GEMM with M = B*T (w_half), f32-accurate
     // in the operand (src/dit_fwd.cpp:133-136,186-189,271-274,288-291)
     TSN_TRY(run("bcast_add_silu_kernel", 0, 12.0 * B * T * (double)H,
                 [&] { return launch_bcast_add_silu_f16(sync_gather, gc, XE_, T, B * T, H, st); }));
@@ -634,7 +634,7 @@ int RefDitModel::enqueue_eval(const float *x, const float *t, const float *clip_
         mb.ws_bytes = ws_bytes_;
         TSN_TRY(gemm_run(mb, EPI_STORE));
     }
-    // input projection (src/dit_fwd.cpp:142-149): conv k3 over x as f16 hi|lo against [W|W]
+    // input projection (src/dit_fwd.cpp:142-149): conv k3 over paired x (w_half)
     // (f32-accurate) + b, SiLU -> SwiGLU conv k3 (w1|w3 in one GEMM) -> conv k3 w2 into the
     // latent rows of X, every operand f16 hi|lo
     const RowMap D{T, T, 0};   // dense rows, sample boundaries every T rows (conv zero padding)
@@ -687,7 +687,7 @@ int RefDitModel::enqueue_eval(const float *x, const float *t, const float *clip_
         if (taps) TSN_TRY(rt->dev.copy_d2d(taps + tap_n * tap++, X_, tap_n * 4));
     }
     // final layer (src/dit_fwd.cpp:287-303): per-row adaLN (2 chunks) as f16 hi|lo, conv k7 pad 3
-    // + b against [W|W] (f32-accurate), split over K
+    // + b (w_half, f32-accurate), split over K
     if (nblk == 0) {
         LnArgs ln;
         memset(&ln, 0, sizeof ln);

@@ -11,18 +11,18 @@
 //
 // HBM layout (B samples, S rows per sample: latent, then clip, then text):
 //   X    f32 [B][S][H]       residual streams, updated in place by GEMM epilogues
-//   XN   f16 [B][S][2H]      adaLN output (GEMM A operand), hi at [0, H), lo at [H, 2H): LN1 of
-//                            every stream (QKV operand), LN2 of the latent rows (FFN operand); rows
-//                            [0, B*T) double as the input projection's hidden (hi|lo)
-//   XE   f16 [B*T][2H]       silu(extended_c) as hi|lo, A operand of the per-row modulation GEMM
+//   XN   f16 [B][S][2H]      adaLN output (GEMM A operand): paired rows (kernels.h) for LN1 of every
+//                            stream (QKV operand) and LN2 of the latent rows (FFN operand), plain f16 for
+//                            LN2 of clip and text; rows [0, B*T) double as the input projection's hidden
+//   XE   f16 [B*T][2H]       silu(extended_c), paired, A operand of the per-row modulation GEMM
 //   MODL f32 [B*T][NMODL]    per-row modulation: every latent and fused block (6 chunks), final (2)
 //   MODG f32 [B][NMODG]      per-sample modulation of the clip and text streams (6, or 2 when pre-only)
 //   Q,K  f16 [B][NH][S][64], Vt f16 [B][NH][64][Sp] (joint); VtF [B][NH][64][SpF] (fused, S = T)
-//   AO   f16 [B][S][2H]      attention output as hi|lo
-//   HF   f16 [B][S][2F]      SwiGLU hidden, hi|lo for latent rows
-// Every QKV GEMM and the latent stream's out-proj and FFN GEMMs read hi|lo operands, each half
-// against the same weight columns (f32-accurate operands); the clip and text out-proj and FFN read
-// the hi halves only.
+//   AO   f16 [B][S][2H]      attention output, paired for latent rows, plain for the others
+//   HF   f16 [B][S][2F]      SwiGLU hidden, paired for latent rows, plain for the others
+// Every QKV GEMM and the latent stream's out-proj and FFN GEMMs read paired operands, both
+// parts against the same weight columns (f32-accurate operands); the clip and text out-proj and FFN read
+// plain f16 rows.
 #pragma once
 #include <map>
 #include <string>
@@ -54,8 +54,8 @@ public:
     int create(Runtime *rt, const RefDitSpec &s);
     // WeightSet::load (src/net.mm:126-173) for a flat BF16 buffer in manifest order, with the
     // upload-time transforms: qkv rows de-interleaved to q|k|v blocks, conv weights tap-major
-    // [OC][K][IC], w1/w3 interleaved in 64-row blocks for the SwiGLU epilogue, input and final conv
-    // weights duplicated as [w | w] for f32-accurate hi|lo operands, all GEMM weights f16.
+    // [OC][K][IC], w1/w3 interleaved in 64-row blocks for the SwiGLU epilogue, all GEMM
+    // weights f16.
     int upload_weights(const uint16_t *host_bf16, size_t numel);
     // the same from an f32 buffer (dequantized checkpoint tensors)
     int upload_weights_f32(const float *host_f32, size_t numel);

@@ -279,7 +279,7 @@ int Runtime::conv_prepare(const void *W, int wdt, void *Wp, uint32_t OC, uint32_
     return launch_conv_prepare(W, wdt, (half_t *)Wp, (int)OC, (int)IC, (int)K, dev.stream());
 }
 
-// Three routes, all f32-accurate (f16 weights: x as hi|lo against [W | W]; f32 weights: three-part
+// Three routes, all f32-accurate (f16 weights: x as paired rows, both parts against one W; f32 weights: three-part
 // products against [W_hi | W_hi | W_lo]):
 //   * stride 1, dilation 1, IC % 64 == 0: implicit GEMM over the split input, taps in K (no im2col);
 //   * other strides, dilations, transposed convs and channel counts: the gathered operand (the
@@ -309,7 +309,7 @@ int Runtime::conv(int wdt, const void *Wp, const float *bias, const float *x, fl
     q.W = (const half_t *)Wp; q.ldw = Kp; q.bias = bias; q.w_half = parts == 1;
     q.N = (int)OC; q.ldy = (int)OC; q.y_f16 = 0;
     b.nprob = 1;
-    const int ich = (int)IC * (parts == 1 ? 2 : 3);   // split input row: [hi | lo] or [hi | lo | hi]
+    const int ich = (int)IC * (parts == 1 ? 2 : 3);   // split input row: pairs, or [hi | lo | hi]
     if (stride == 1 && dil == 1 && !convt && IC % 64 == 0 && aligned16(x) &&
         2ULL * (OL + T) * ich * 2 < (1ULL << 31)) {
         void *buf = nullptr;

@@ -25,7 +25,7 @@ struct GemmParams {  // src/net.h:13-16; a zero ld means the packed default
 };
 
 // Y = X·Wᵀ (+bias) with f32 X and f16 W as an f32-accurate MFMA product: X is split into an f16
-// hi|lo pair in hl (M x 2K halves) and multiplied against [W | W]. gemm_hilo_ok tells whether the
+// hi|lo pairs in hl (M x 2K halves), both parts multiplied by one staged W. gemm_hilo_ok tells whether the
 // pipelined kernel takes the shape; hl needs gemm_hilo_bytes(M, K) bytes, 16-byte aligned. ws (f32,
 // ws_bytes; null for none) holds the partial sums of a classic K split, taken when the 128x128 grid
 // would leave most CUs idle over a long K; the partials are summed in split order, so the result
@@ -88,7 +88,7 @@ public:
     int init(int device);
 
     // Y[M,N] = X[M,K]·W[N,K]ᵀ (+bias)                              (src/net.h:24-26)
-    // wdt F16, X f32: f32-accurate MFMA product (X as an f16 hi|lo pair against [W | W]), Y f32 or f16;
+    // wdt F16, X f32: f32-accurate MFMA product (X as f16 hi|lo pairs, both parts against W), Y f32 or f16;
     //   shapes the pipelined kernel does not take run the f32 SIMT path (Y f32 only).
     // wdt F16, X f16: plain f16 MFMA product. wdt BF16, X bf16: bf16 MFMA product (f32 Y; MFMA
     // tiling only). wdt F32 / BF16 with X f32: f32 SIMT path (X, Y f32).

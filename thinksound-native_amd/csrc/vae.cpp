@@ -81,8 +81,8 @@ int vae_spec_check(const VaeSpec &s) {
                     "vae spec: transposed-conv kernel must be a multiple of its stride, at least twice it");
         T *= st;
         TSN_REQUIRE(T < (1LL << 30), "vae spec: audio too long");
-        // every GEMM operand row [hi | lo | hi] is addressed with 32-bit byte offsets (up to twice the
-        // rows of a stage, conv halo included)
+        // GEMM operand rows are addressed with 32-bit byte offsets (up to twice the rows of a stage, conv halo
+        // included). Paired rows take 4 bytes a value; the accepted length is that of 6 bytes
         TSN_REQUIRE(2 * T * 3 * s.width[n + 1] * 2 < (1LL << 31),
                     "vae spec: audio too long for one decode (split the latent into shorter segments)");
     }
