@@ -96,21 +96,26 @@ def read_counter_csv(path, counter):
     return out
 
 
+def calibration(per_kernel):
+    """the entry of the calibration copies, whatever their template arguments"""
+    return next(v for k, v in per_kernel.items() if k.split("<")[0] == "copy_kernel")
+
+
 def pmc_summary(fetch_csv, write_csv, cmd):
     """Text summary of FETCH_SIZE / WRITE_SIZE (KiB per dispatch) per kernel, scaled by the ratio of
     the calibration copy's known bytes to what the same counter reads for it."""
     fetch = read_counter_csv(fetch_csv, "FETCH_SIZE")
     write = read_counter_csv(write_csv, "WRITE_SIZE")
     cal_kib = CAL_COPY_FLOATS * 4 / 1024.0
-    cf = cal_kib / statistics.mean(fetch["copy_kernel"])
-    cw = cal_kib / statistics.mean(write["copy_kernel"])
+    cf = cal_kib / statistics.mean(calibration(fetch))
+    cw = cal_kib / statistics.mean(calibration(write))
     lines = ["# HBM traffic per dispatch, one 21-block DiT evaluation (B=2, La=256, Lt=141, S=397)",
              "# commands (rocprofv3 counter passes, one counter each):",
              "#   " + cmd.replace("{C}", "FETCH_SIZE"),
              "#   " + cmd.replace("{C}", "WRITE_SIZE"),
              "# calibration: copy_kernel of %d MiB read + %d MiB written reads FETCH %.1f KiB, WRITE %.1f KiB"
-             % (cal_kib / 1024, cal_kib / 1024, statistics.mean(fetch["copy_kernel"]),
-                statistics.mean(write["copy_kernel"])),
+             % (cal_kib / 1024, cal_kib / 1024, statistics.mean(calibration(fetch)),
+                statistics.mean(calibration(write))),
              "# scale factors: fetch %.4f, write %.4f (traffic = FETCH*1024*fetch_scale + WRITE*1024*write_scale)"
              % (cf, cw),
              "%-28s %10s %14s %14s %16s" % ("kernel", "dispatches", "FETCH KiB/d", "WRITE KiB/d", "traffic B/d")]
@@ -255,8 +260,8 @@ def pmc_util_summary(sq_csv, dram_csv, title, cmd):
     sq, dr = read_counter_rows(sq_csv), read_counter_rows(dram_csv)
     mean = statistics.mean
     cal_bytes = CAL_COPY_FLOATS * 4.0
-    rd_b = cal_bytes / mean(dr["copy_kernel"]["TCC_EA0_RDREQ_DRAM_sum"])
-    wr_b = cal_bytes / mean(dr["copy_kernel"]["TCC_EA0_WRREQ_DRAM_sum"])
+    rd_b = cal_bytes / mean(calibration(dr)["TCC_EA0_RDREQ_DRAM_sum"])
+    wr_b = cal_bytes / mean(calibration(dr)["TCC_EA0_WRREQ_DRAM_sum"])
     lines = ["# rocprofv3 counters per dispatch, " + title,
              "# commands (two counter passes):",
              "#   " + cmd.replace("{P}", "SQ_VALU_MFMA_BUSY_CYCLES SQ_BUSY_CU_CYCLES SQ_INSTS_VALU SQ_INSTS_MFMA "
