@@ -463,7 +463,7 @@ def test_launcher_surface_rest(tsn, rt, orc):
     assert np.array_equal(dd.numpy(), orc.qkv_split3(src, dst0, off))
 
 
-@pytest.mark.parametrize("S", [1, 63, 64, 65, 130])
+@pytest.mark.parametrize("S", [1, 15, 16, 17, 63, 64, 65, 130])
 def test_attention_pack_alignment(tsn, rt, S):
     """The operand packing with 16-byte loads and with single ones (odd strides and offsets): the same
     values in both layouts give bit-identical outputs."""

@@ -770,50 +770,40 @@ __global__ __launch_bounds__(256, 3) void flash_attn4q2_kernel(const AttnArgs a)
     }
 }
 
-// f32 [S, ld] q/k/v slices -> Q/K [nh][S][64], Vt [nh][64][Sp] (f16). One workgroup per 64 rows of a head: thread
-// t has columns 4 (t % 16) .. + 3 of rows t / 16 + 16 p, all twelve loads issued first, and V turns in LDS so
-// that Vt rows are written 16 bytes at a time (one thread per element wrote Vt two bytes at a time, Sp
-// apart: 331 rows x 16 heads 5.6 us, now 4.2). VEC: rows, strides and offsets allow 16-byte loads.
+// f32 [S, ld] q/k/v slices -> Q/K [nh][S][64], Vt [nh][64][Sp] (f16). One workgroup per PACK_ROWS rows of a head:
+// thread t has columns 4 (t % 16) .. + 3 of row t / 16, and V turns in LDS so that a Vt row is written 32 bytes
+// at a time (one thread per element wrote Vt two bytes at a time, Sp apart). A launch is as long as one
+// workgroup's loads and stores: 16 rows and one load of each of q, k and v a thread beat 32 and 64 rows at every
+// length (attention of 64 rows x 16 heads 7.4 us with one thread per element, 8.1, 7.5 and 7.0 with 64, 32 and 16
+// rows; 331 rows 11.4, 10.2, 9.6, 9.3; 1101 rows 28.1, 24.3, 23.8, 23.5). VEC: rows, strides and offsets allow
+// 16-byte loads.
+constexpr int PACK_ROWS = 16;
 template <bool VEC>
 __global__ __launch_bounds__(256) void attn_pack_kernel(const float *qkv, float q_scale, int S, int nh, int ld, int q_off,
                                                         int k_off, int v_off, half_t *Q, half_t *K, half_t *Vt, int Sp) {
-    constexpr int VP = 72;   // halves: 16-byte aligned rows
-    __shared__ __attribute__((aligned(16))) half_t vt[64 * VP];
-    const int tid = threadIdx.x, h = blockIdx.y, s0 = blockIdx.x * 64, r = tid >> 4, c = (tid & 15) * 4;
+    constexpr int VP = PACK_ROWS + 8;   // halves: 8-byte aligned rows
+    __shared__ __attribute__((aligned(8))) half_t vt[64 * VP];
+    const int tid = threadIdx.x, h = blockIdx.y, r = tid >> 4, s = blockIdx.x * PACK_ROWS + r, c = (tid & 15) * 4;
     auto load4 = [&](const float *p) {
         if constexpr (VEC) return *(const float4 *)p;
         else return make_float4(p[0], p[1], p[2], p[3]);
     };
-    float4 q[4], k[4], v[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const int s = s0 + r + 16 * p;
-        q[p] = k[p] = v[p] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (s < S) {
-            const float *row = qkv + (long long)s * ld + h * 64 + c;
-            q[p] = load4(row + q_off);
-            k[p] = load4(row + k_off);
-            v[p] = load4(row + v_off);
-        }
-    }
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        const int sl = r + 16 * p, s = s0 + sl;
-        vt[c * VP + sl] = (half_t)v[p].x;
-        vt[(c + 1) * VP + sl] = (half_t)v[p].y;
-        vt[(c + 2) * VP + sl] = (half_t)v[p].z;
-        vt[(c + 3) * VP + sl] = (half_t)v[p].w;
-        if (s >= S) continue;
+    // rows past the context: its last one, not stored, and V zero
+    const float *row = qkv + (long long)min(s, S - 1) * ld + h * 64 + c;
+    const float4 q = load4(row + q_off), k = load4(row + k_off), v = load4(row + v_off);
+    const bool in = s < S;
+    vt[c * VP + r] = (half_t)(in ? v.x : 0.f);
+    vt[(c + 1) * VP + r] = (half_t)(in ? v.y : 0.f);
+    vt[(c + 2) * VP + r] = (half_t)(in ? v.z : 0.f);
+    vt[(c + 3) * VP + r] = (half_t)(in ? v.w : 0.f);
+    if (in) {
         const long long o = ((long long)h * S + s) * 64 + c;
-        *(half4 *)(Q + o) = half4{(half_t)(q[p].x * q_scale), (half_t)(q[p].y * q_scale), (half_t)(q[p].z * q_scale),
-                                  (half_t)(q[p].w * q_scale)};
-        *(half4 *)(K + o) = half4{(half_t)k[p].x, (half_t)k[p].y, (half_t)k[p].z, (half_t)k[p].w};
+        *(half4 *)(Q + o) = half4{(half_t)(q.x * q_scale), (half_t)(q.y * q_scale), (half_t)(q.z * q_scale), (half_t)(q.w * q_scale)};
+        *(half4 *)(K + o) = half4{(half_t)k.x, (half_t)k.y, (half_t)k.z, (half_t)k.w};
     }
     __syncthreads();
-    const int d = tid >> 2, sc = (tid & 3) * 16;
-    half_t *o = Vt + ((long long)h * 64 + d) * Sp + s0 + sc;
-    *(half8 *)o = *(const half8 *)&vt[d * VP + sc];
-    *(half8 *)(o + 8) = *(const half8 *)&vt[d * VP + sc + 8];
+    const int d = tid >> 2, sc = (tid & 3) * 4;
+    *(half4 *)(Vt + ((long long)h * 64 + d) * Sp + blockIdx.x * PACK_ROWS + sc) = *(const half4 *)&vt[d * VP + sc];
 }
 
 } // namespace
@@ -855,7 +845,7 @@ int launch_attn_pack(const float *qkv, float q_scale, int S, int nh, int ld, int
     const bool vec = (((uintptr_t)qkv) & 15) == 0 && ((ld | q_off | k_off | v_off) & 3) == 0;
     for (int h0 = 0; h0 < nh; h0 += 65535) {   // grid.y limit
         const int n = nh - h0 < 65535 ? nh - h0 : 65535;
-        const dim3 grid((unsigned)(Sp / 64), (unsigned)n), block(256);
+        const dim3 grid((unsigned)(Sp / PACK_ROWS), (unsigned)n), block(256);
         const float *x = qkv + (long long)h0 * 64;
         half_t *q = Q + (long long)h0 * S * 64, *k = K + (long long)h0 * S * 64, *vt = Vt + (long long)h0 * 64 * Sp;
         if (vec) TSN_LAUNCH(attn_pack_kernel<true>, grid, block, 0, st, x, q_scale, S, n, ld, q_off, k_off, v_off, q, k, vt, Sp);
