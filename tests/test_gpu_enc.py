@@ -144,10 +144,10 @@ def test_encoders_gguf_load(tsn, rt, tmp_path):
             m.close()
 
 
-@pytest.mark.parametrize("ctx", [1, 16, 17, 32, 33, 80, 81, 128])
+@pytest.mark.parametrize("ctx", [1, 16, 17, 32, 33, 64, 65, 80, 81, 128])
 @pytest.mark.parametrize("scale", [1.0, 3e4])
 def test_encoder_gemm_edges(tsn, rt, orc, ctx, scale):
-    """Row-block edges of the GEMMs (16-row MFMA blocks, the 32-, 80- and 128-row tiles), a K that ends half
+    """Row-block edges of the GEMMs (16-row MFMA blocks, the 32-, 64-, 80- and 128-row tiles), a K that ends half
     way through a 64-column step (d_ff = 96, 352) and, with scale, T5 FFN activations of about scale^2
     (past the f16 range) and rows of one weight 2^-20 of the others (k rows of a head, whose q rows are 2^20
     larger, so that its scores keep their size). f32 against f32: three layers amplify a rounding-level
@@ -209,7 +209,7 @@ def _views(manifest, w):
     return {n: w[o:o + k] for n, k, o in manifest}
 
 
-@pytest.mark.parametrize("ctx", [9, 77, 100])
+@pytest.mark.parametrize("ctx", [9, 50, 77, 100])
 @pytest.mark.parametrize("k", [-20, 14, 20, 40])
 def test_encoders_keep_f32_operands(tsn, rt, ctx, k):
     """Powers of two moved between the two operands of a product (a channel of a norm weight or of a hidden row

@@ -121,13 +121,15 @@ __global__ __launch_bounds__(256) void enc_weight_pack_kernel(const float *__res
 // A step is 64 columns of K. 4 waves: wave w owns columns 32 (w & 1) .. + 31 of a 64-column tile and
 // K half w >> 1 of every step, and the two halves' sums are added through LDS at the end, so each
 // fragment of A read from LDS feeds two of W. A steps (6 KB per 16 rows) are shared by the waves through
-// two LDS buffers, loaded one step ahead. Fetches past the split's end take its last step again, so
+// two LDS buffers, loaded two steps ahead (one with five row blocks, for registers: a step of fewer blocks is
+// shorter than a load from L2; 2 T5 layers of 512, 8 rows: 83 us one step ahead, 71 two). Fetches past the split's end take its last step again, so
 // every wait in the loop has a fixed count of younger loads to leave in flight.
 //
 // MTP: the operand's row blocks; with MTP > MT, blockIdx.z picks the MT of them that the workgroup takes.
 template <int MT, int MTP>
 __global__ __launch_bounds__(256, 2) void enc_gemm_kernel(const EncGemmArgs g) {
     constexpr int CH = 2 * 3 * MT * 64, NA = (CH + 255) / 256;   // 16-byte chunks of an A step, per thread
+    constexpr int DA = MT < 5 ? 2 : 1;                           // steps that A is loaded ahead
     __shared__ __attribute__((aligned(16))) uintx4_t As[2][CH];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r16 = lane & 15, kq = lane >> 4, wn = wave & 1, kh = wave >> 1;
@@ -136,25 +138,25 @@ __global__ __launch_bounds__(256, 2) void enc_gemm_kernel(const EncGemmArgs g) {
     const int kt0 = z * g.kps, kt1 = min(nkt, kt0 + g.kps);
     const float *wb = g.W + ((long long)blockIdx.x * nkt * 4 + wave) * 1024;   // wave-uniform
     floatx4_t w[3][4];
-    uintx4_t a[NA];
+    uintx4_t a[DA][NA];
     auto fetch_w = [&](int kt, floatx4_t (&d)[4]) {
         const floatx4_t *p = (const floatx4_t *)(wb + (long long)min(kt, kt1 - 1) * 4096);
 #pragma unroll
         for (int q = 0; q < 4; ++q) d[q] = p[(unsigned)(q * 64 + lane)];
     };
     auto full = [&](int i) { return CH % 256 == 0 || i < NA - 1 || wave < CH % 256 / 64; };   // wave-uniform
-    auto fetch_a = [&](int kt) {
+    auto fetch_a = [&](int kt, uintx4_t (&d)[NA]) {
         const uintx4_t *p = (const uintx4_t *)g.Ap + ((long long)min(kt, kt1 - 1) * 6 * MTP + mb) * 64;
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int c = tid + 256 * i;
-            if (full(i)) a[i] = p[(unsigned)(MTP > MT ? c / (64 * MT) * (64 * MTP) + c % (64 * MT) : c)];
+            if (full(i)) d[i] = p[(unsigned)(MTP > MT ? c / (64 * MT) * (64 * MTP) + c % (64 * MT) : c)];
         }
     };
-    auto stash_a = [&](int b) {
+    auto stash_a = [&](int b, const uintx4_t (&d)[NA]) {
 #pragma unroll
         for (int i = 0; i < NA; ++i)
-            if (full(i)) As[b][tid + 256 * i] = a[i];
+            if (full(i)) As[b][tid + 256 * i] = d[i];
     };
     floatx4_t acc[2][MT], low[2][MT];
 #pragma unroll
@@ -190,34 +192,46 @@ __global__ __launch_bounds__(256, 2) void enc_gemm_kernel(const EncGemmArgs g) {
                     }
         }
     };
-    // Step kt issues A(kt + 1), then W(kt + 3) into the registers that W(kt) leaves: A(kt + 1) has to be in LDS
-    // at the step's end, with W(kt + 3) still in flight. LDS buffer (kt - kt0) & 1 holds A(kt); the other
-    // one was last read in step kt - 1, before the barrier that ended it.
-    fetch_a(kt0);
+    // Step kt issues A(kt + DA), then W(kt + 3) into the registers that W(kt) leaves: A(kt + 1) has to be in LDS
+    // at the step's end, with the younger loads still in flight. LDS buffer (kt - kt0) & 1 holds A(kt); the
+    // other one was last read in step kt - 1, before the barrier that ended it.
+    fetch_a(kt0, a[0]);
     fetch_w(kt0, w[0]);
     fetch_w(kt0 + 1, w[1]);
-    stash_a(0);
+    if constexpr (DA == 2) fetch_a(kt0 + 1, a[1]);
+    else stash_a(0, a[0]);
     fetch_w(kt0 + 2, w[2]);
+    if constexpr (DA == 2) stash_a(0, a[0]);
     __syncthreads();
-    int kt = kt0, b = 0;
-    auto step = [&](floatx4_t (&d)[4]) {
+    int kt = kt0;
+    auto step = [&](int b, floatx4_t (&d)[4], uintx4_t (&in)[NA], const uintx4_t (&out)[NA]) {
         bf16x8_t o[2][3];
-        fetch_a(kt + 1);
+        fetch_a(kt + DA, in);
         split_w(d, o);
         fetch_w(kt + 3, d);
         multiply(b, o);
-        stash_a(b ^ 1);
+        stash_a(b ^ 1, out);
         __syncthreads();
-        b ^= 1;
         ++kt;
     };
-    while (kt + 3 <= kt1) {
-        step(w[0]);
-        step(w[1]);
-        step(w[2]);
+    if constexpr (DA == 2) {
+        while (kt + 6 <= kt1) {
+#pragma unroll
+            for (int u = 0; u < 6; ++u) step(u & 1, w[u % 3], a[u & 1], a[(u & 1) ^ 1]);
+        }
+#pragma unroll
+        for (int u = 0; u < 5; ++u)   // the last zero to five steps
+            if (kt < kt1) step(u & 1, w[u % 3], a[u & 1], a[(u & 1) ^ 1]);
+    } else {
+        int b = 0;
+        while (kt + 3 <= kt1) {
+#pragma unroll
+            for (int u = 0; u < 3; ++u, b ^= 1) step(b, w[u], a[0], a[0]);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u, b ^= 1)
+            if (kt < kt1) step(b, w[u], a[0], a[0]);
     }
-    if (kt < kt1) step(w[0]);
-    if (kt < kt1) step(w[1]);
     // the weights are the first operand: a lane holds columns n0 + 16 j + 4 kq .. + 3 of row 16 i + r16;
     // 4 MT KB of the buffers' 12 MT
     floatx4_t *sum = (floatx4_t *)&As[0][0] + wn * 2 * MT * 64 + lane;
@@ -488,7 +502,8 @@ bool aligned16(const void *p) { return (((uintptr_t)p) & 15) == 0; }
 
 } // namespace
 
-int enc_row_blocks(int M) { return M <= 32 ? 2 : M <= 80 ? 5 : 8; }
+// 2 T5 layers 2048 wide: 64 rows 202 us with five row blocks, 197 with four (512 wide 94 and 91)
+int enc_row_blocks(int M) { return M <= 32 ? 2 : M <= 64 ? 4 : M <= 80 ? 5 : 8; }
 size_t enc_operand_bytes(int M, int K) {   // whole 64-column steps
     return (size_t)3 * enc_row_blocks(M) * 16 * ((K + 63) / 64 * 64) * sizeof(uint16_t);
 }
@@ -524,6 +539,7 @@ int launch_enc_gemm(EncGemmArgs &g, hipStream_t st) {
     g.splits = (steps + g.kps - 1) / g.kps;
     const dim3 grid(tiles, g.splits, mt == 8 ? 2 : 1), block(256);   // more than 80 rows: two halves
     if (mt == 2) TSN_LAUNCH((enc_gemm_kernel<2, 2>), grid, block, 0, st, g);
+    else if (mt == 4) TSN_LAUNCH((enc_gemm_kernel<4, 4>), grid, block, 0, st, g);
     else if (mt == 5) TSN_LAUNCH((enc_gemm_kernel<5, 5>), grid, block, 0, st, g);
     else TSN_LAUNCH((enc_gemm_kernel<4, 8>), grid, block, 0, st, g);
     TSN_HIP_CHECK(hipGetLastError());
@@ -565,6 +581,7 @@ int launch_enc_attention(const EncAttnArgs &a, hipStream_t st) {
     const dim3 grid((a.nh + 7) / 8 * 8 * ((a.S + EA_Q - 1) / EA_Q));
     const int mt = enc_row_blocks(a.S);
     if (mt == 2) TSN_LAUNCH(enc_attn_kernel<2>, grid, dim3(256), 0, st, a);
+    else if (mt == 4) TSN_LAUNCH(enc_attn_kernel<4>, grid, dim3(256), 0, st, a);
     else if (mt == 5) TSN_LAUNCH(enc_attn_kernel<5>, grid, dim3(320), 0, st, a);
     else TSN_LAUNCH(enc_attn_kernel<8>, grid, dim3(512), 0, st, a);
     TSN_HIP_CHECK(hipGetLastError());
