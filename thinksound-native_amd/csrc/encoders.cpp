@@ -152,7 +152,7 @@ std::vector<ManifestEntry> t5_manifest(const T5Spec &s) {
 }
 
 // K splits of a QKV GEMM: attention reads every split of k and v in each of a head's workgroups. 77 rows, 1024
-// wide: 4 splits 1.42 ms a prompt, 2 splits 1.48; 2048 wide: 2.49 ms with 4 and 2, 2.54 with 5.
+// wide: 2 splits 4% a prompt more than 4; 2048 wide: 4 and 2 the same, 5 2% more.
 constexpr int QKV_SPLITS = 4;
 
 int EncoderRunner::create_common(int ctx, int width, int ffn, int ffn_cols) {
